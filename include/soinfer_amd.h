@@ -630,6 +630,48 @@ int soi_grid_barrier_max_workgroups(int64_t* max_workgroups);
 int soi_grid_barrier_bench(int fenced, int64_t P, int64_t rounds, void* workspace, size_t workspace_bytes,
                            void* stream);
 
+/* --------------------------------------------------------------------------
+ * A whole prompt, one decoder layer at a time: the decode step's operators
+ * over T tokens (1 <= T <= 65535), each weight read once for a tile of
+ * tokens. Every value is bit for bit the one the decode step's operators give
+ * when the tokens are fed one at a time; the reference feeds them so
+ * (generate.py:429-463) and has no counterpart. [T, n] arrays are contiguous.
+ *   soi_embed_tokens: out[t] = table[tokens[t]] (device tokens; zeros for a
+ *     token outside the table).
+ *   soi_norm_tokens: h[t] = rmsnorm(x[t], weight); hidden % 8 == 0, 16-byte
+ *     aligned. one_pass (hidden 2048 only): the sum-of-squares partition of
+ *     the one-pass norm-fused GEMV, which soi_norm_gemv_one_pass tells for a
+ *     GEMV of [N, K] rows; else that of its general form.
+ *   soi_gemm_w4a16_tokens: y[t, n] = (W x[t])[n] as
+ *     soi_gemv_w4a16_group_lop3 gives it, or with `add` y[t, n] = y[t, n] +
+ *     that value as one binary16 addition. K and group_size multiples of 32,
+ *     Wq and x 16-byte aligned.
+ *   soi_silu_mul_tokens: h[t, i] = fp16(silu(gate) * up) of gate_up [T, 2 I],
+ *     gate then up rows, or interleaved by 8-row tiles (4 gate, 4 up).
+ *   soi_qk_norm_rope_tokens: token t at position pos[0] + t: q/k RMSNorm +
+ *     RoPE of qkv [T, (NQ + 2 NKV) * hd], q to q_out [T, NQ, hd], k and v to
+ *     the caches (nothing is appended outside [0, max_seq)).
+ *   soi_attention_tokens: out[t] [NQ, hd] = decode attention of q[t] over
+ *     pos[0] + t + 1 timesteps (clamped to [1, max_seq]) of caches that hold
+ *     them. SOI_ERR_UNSUPPORTED where soi_attention_tokens_supported is 0.
+ * ------------------------------------------------------------------------ */
+int soi_embed_tokens(const uint16_t* table, int64_t rows, int64_t hidden, const int32_t* tokens, int64_t T,
+                     uint16_t* out, void* stream);
+int soi_norm_gemv_one_pass(int64_t N, int64_t K, int64_t group_size, int swiglu);
+int soi_norm_tokens(const uint16_t* x, const uint16_t* weight, float eps, uint16_t* h, int64_t T, int64_t hidden,
+                    int one_pass, void* stream);
+int soi_gemm_w4a16_tokens(const uint8_t* Wq, const float* scale, const uint16_t* x, uint16_t* y, int64_t N, int64_t K,
+                          int64_t group_size, int64_t T, int add, void* stream);
+int soi_silu_mul_tokens(const uint16_t* gate_up, uint16_t* h, int64_t T, int64_t I, int interleaved, void* stream);
+int soi_qk_norm_rope_tokens(const uint16_t* qkv, const uint16_t* q_norm, const uint16_t* k_norm,
+                            const float* cos_table, const float* sin_table, const int32_t* pos, uint16_t* q_out,
+                            uint16_t* k_cache, uint16_t* v_cache, int64_t T, int64_t num_q_heads,
+                            int64_t num_kv_heads, int64_t max_seq, int64_t head_dim, float eps, void* stream);
+int soi_attention_tokens_supported(int64_t num_q_heads, int64_t num_kv_heads, int64_t head_dim, int64_t max_seq);
+int soi_attention_tokens(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v_cache, uint16_t* out,
+                         const int32_t* pos, int64_t T, int64_t num_q_heads, int64_t num_kv_heads, int64_t max_seq,
+                         int64_t head_dim, float scale, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1556,6 +1556,116 @@ void grid_barrier_bench(bool fenced, int64_t P, int64_t rounds, torch::Tensor wo
                  n);
 }
 
+// ---------------------------------------------------------------------------
+// a whole prompt, one layer at a time (T tokens; buffers hold at least T rows)
+// ---------------------------------------------------------------------------
+namespace {
+
+void need_int4(const torch::Tensor& Wq, const torch::Tensor& scale, const torch::Tensor& dev, int64_t K, int64_t gs,
+               const char* n, const char* arg) {
+    need(Wq, torch::kUInt8, dev, n, arg);
+    need(scale, torch::kFloat32, dev, n, arg);
+    TORCH_CHECK(gs >= 1 && Wq.dim() == 2 && Wq.size(1) == ((K + 7) / 8) * 4, n, "(", arg, "): Wq must be [N, ceil(K/8)*4]");
+    TORCH_CHECK(scale.dim() == 2 && scale.size(0) == Wq.size(0) && scale.size(1) == expected_num_groups(K, gs), n, "(",
+                arg, "): scale must be [N, ceil(K/group_size)]");
+}
+
+}  // namespace
+
+void embed_tokens_into(torch::Tensor table, torch::Tensor tokens, torch::Tensor out) {
+    const char* n = "embed_tokens_into";
+    need(table, torch::kFloat16, table, n, "table");
+    need(tokens, torch::kInt32, table, n, "tokens");
+    need(out, torch::kFloat16, table, n, "out");
+    TORCH_CHECK(table.dim() == 2, n, ": table must be [rows, hidden]");
+    need_numel(out, tokens.numel() * table.size(1), n, "out");
+    const at::DeviceGuard guard(table.device());
+    check_status(soi_embed_tokens(h16(table), table.size(0), table.size(1), tokens.data_ptr<int32_t>(), tokens.numel(),
+                                  h16m(out), cur_stream(table)),
+                 n);
+}
+
+// x[t] += o_proj(attention(rope(norm(qkv_proj(rmsnorm(x[t]))))) for T tokens at positions pos[0] + t; appends their
+// k and v. h, qkv, q, attn: scratch.
+void prompt_attention_(int64_t T, torch::Tensor x, torch::Tensor norm, torch::Tensor h, torch::Tensor qkv_Wq,
+                       torch::Tensor qkv_scale, torch::Tensor qkv, torch::Tensor q_norm, torch::Tensor k_norm,
+                       torch::Tensor cos_table, torch::Tensor sin_table, torch::Tensor pos, torch::Tensor q,
+                       torch::Tensor k_cache, torch::Tensor v_cache, torch::Tensor attn, torch::Tensor o_Wq,
+                       torch::Tensor o_scale, int64_t group_size, double eps) {
+    const char* n = "prompt_attention_";
+    TORCH_CHECK(T >= 1, n, ": T must be positive");
+    for (const torch::Tensor* t : {&x, &norm, &h, &qkv, &q_norm, &k_norm, &q, &k_cache, &v_cache, &attn})
+        need(*t, torch::kFloat16, x, n, "fp16 operand");
+    for (const torch::Tensor* t : {&cos_table, &sin_table}) need(*t, torch::kFloat32, x, n, "RoPE table");
+    need(pos, torch::kInt32, x, n, "pos");
+    need_numel(pos, 1, n, "pos");
+    const int64_t H = norm.numel();
+    need_int4(qkv_Wq, qkv_scale, x, H, group_size, n, "qkv");
+    TORCH_CHECK(k_cache.dim() == 3 && v_cache.sizes() == k_cache.sizes(), n, ": caches must be [NKV, max_seq, head_dim]");
+    const int64_t NKV = k_cache.size(0), S = k_cache.size(1), hd = k_cache.size(2);
+    const int64_t rows = qkv_Wq.size(0), NQ = rows / hd - 2 * NKV;
+    TORCH_CHECK(NQ >= 1 && rows == (NQ + 2 * NKV) * hd, n, ": qkv rows must be (NQ + 2 NKV) * head_dim");
+    need_int4(o_Wq, o_scale, x, NQ * hd, group_size, n, "o");
+    TORCH_CHECK(o_Wq.size(0) == H, n, ": o must have hidden rows");
+    TORCH_CHECK(q_norm.numel() == hd && k_norm.numel() == hd && cos_table.numel() == S * (hd / 2) &&
+                    sin_table.numel() == S * (hd / 2),
+                n, ": norm or RoPE table shape mismatch");
+    need_numel(x, T * H, n, "x");
+    need_numel(h, T * H, n, "h");
+    need_numel(qkv, T * rows, n, "qkv");
+    need_numel(q, T * NQ * hd, n, "q");
+    need_numel(attn, T * NQ * hd, n, "attn");
+    const at::DeviceGuard guard(x.device());
+    void* st = cur_stream(x);
+    check_status(soi_norm_tokens(h16(x), h16(norm), static_cast<float>(eps), h16m(h), T, H,
+                                 soi_norm_gemv_one_pass(rows, H, group_size, 0), st),
+                 n);
+    check_status(soi_gemm_w4a16_tokens(qkv_Wq.data_ptr<uint8_t>(), qkv_scale.data_ptr<float>(), h16(h), h16m(qkv), rows,
+                                       H, group_size, T, 0, st),
+                 n);
+    check_status(soi_qk_norm_rope_tokens(h16(qkv), h16(q_norm), h16(k_norm), cos_table.data_ptr<float>(),
+                                         sin_table.data_ptr<float>(), pos.data_ptr<int32_t>(), h16m(q), h16m(k_cache),
+                                         h16m(v_cache), T, NQ, NKV, S, hd, static_cast<float>(eps), st),
+                 n);
+    check_status(soi_attention_tokens(h16(q), h16(k_cache), h16(v_cache), h16m(attn), pos.data_ptr<int32_t>(), T, NQ,
+                                      NKV, S, hd, 1.0f / std::sqrt(static_cast<float>(hd)), st),
+                 n);
+    check_status(soi_gemm_w4a16_tokens(o_Wq.data_ptr<uint8_t>(), o_scale.data_ptr<float>(), h16(attn), h16m(x), H,
+                                       NQ * hd, group_size, T, 1, st),
+                 n);
+}
+
+// x[t] += down(fp16(silu(gate) * up)) of rmsnorm(x[t]) for T tokens; gu rows interleaved by 8-row tiles. h, gu, m: scratch.
+void prompt_mlp_dense_(int64_t T, torch::Tensor x, torch::Tensor norm, torch::Tensor h, torch::Tensor gu_Wq,
+                       torch::Tensor gu_scale, torch::Tensor gu, torch::Tensor m, torch::Tensor down_Wq,
+                       torch::Tensor down_scale, int64_t group_size, double eps) {
+    const char* n = "prompt_mlp_dense_";
+    TORCH_CHECK(T >= 1, n, ": T must be positive");
+    for (const torch::Tensor* t : {&x, &norm, &h, &gu, &m}) need(*t, torch::kFloat16, x, n, "fp16 operand");
+    const int64_t H = norm.numel();
+    need_int4(gu_Wq, gu_scale, x, H, group_size, n, "gu");
+    const int64_t I = gu_Wq.size(0) / 2;
+    TORCH_CHECK(gu_Wq.size(0) == 2 * I, n, ": gu must have 2 I rows");
+    need_int4(down_Wq, down_scale, x, I, group_size, n, "down");
+    TORCH_CHECK(down_Wq.size(0) == H, n, ": down must have hidden rows");
+    need_numel(x, T * H, n, "x");
+    need_numel(h, T * H, n, "h");
+    need_numel(gu, T * 2 * I, n, "gu");
+    need_numel(m, T * I, n, "m");
+    const at::DeviceGuard guard(x.device());
+    void* st = cur_stream(x);
+    check_status(soi_norm_tokens(h16(x), h16(norm), static_cast<float>(eps), h16m(h), T, H,
+                                 soi_norm_gemv_one_pass(2 * I, H, group_size, 1), st),
+                 n);
+    check_status(soi_gemm_w4a16_tokens(gu_Wq.data_ptr<uint8_t>(), gu_scale.data_ptr<float>(), h16(h), h16m(gu), 2 * I,
+                                       H, group_size, T, 0, st),
+                 n);
+    check_status(soi_silu_mul_tokens(h16(gu), h16m(m), T, I, 1, st), n);
+    check_status(soi_gemm_w4a16_tokens(down_Wq.data_ptr<uint8_t>(), down_scale.data_ptr<float>(), h16(m), h16m(x), H, I,
+                                       group_size, T, 1, st),
+                 n);
+}
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.doc() = "soinfer MI355X (gfx950) quantized decode hot path";
     m.def("gemv_w8a16", &gemv_w8a16, "INT8 GEMV");
@@ -1664,5 +1774,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("cache_scale"), py::arg("full_Wq"), py::arg("full_scale"), py::arg("slot_of"), py::arg("sel"),
           py::arg("h_sel"), py::arg("y"), py::arg("H"), py::arg("group_size"), py::arg("workspace"),
           py::arg("staging_Wq") = py::none());
+    m.def("embed_tokens_into", &embed_tokens_into, "embedding rows of device tokens");
+    m.def("attention_tokens_supported", &soi_attention_tokens_supported, "whether prompt_attention_ takes the heads");
+    m.def("prompt_attention_", &prompt_attention_, "one layer's attention block over T tokens, added to x");
+    m.def("prompt_mlp_dense_", &prompt_mlp_dense_, "one layer's dense MLP over T tokens, added to x");
     m.def("version", []() { return std::string(soi_version()); });
 }

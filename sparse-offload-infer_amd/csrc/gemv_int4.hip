@@ -655,7 +655,7 @@ extern "C" int soi_gemv_w4a16_rmsnorm_gate_up(const uint8_t* Wq, const float* sc
     const bool cs = (group_size % 32) == 0;
     const int Ki = static_cast<int>(K), gi = static_cast<int>(group_size);
     const bool full_k = (K / 32) % 64 == 0;
-    const bool one = cs && K == 2048;
+    const bool one = norm_gemv_one_pass(N, K, group_size, true);
     const dim3 grid(static_cast<unsigned>(N / 8));
     const SplitGUY ep{gate_out, up_out};
 #define SOI_N(CS, FL, OP)                                                                                          \
@@ -693,7 +693,8 @@ static int rmsnorm_impl(const uint8_t* Wq, const float* scale, const uint16_t* x
     const bool cs = (group_size % 32) == 0;
     const int Ki = static_cast<int>(K), gi = static_cast<int>(group_size);
     const bool full_k = (K / 32) % 64 == 0;
-    const bool one = cs && K == 2048;  // one 64-chunk pass: the lane's x chunk stays in registers
+    // one 64-chunk pass: the lane's x chunk stays in registers
+    const bool one = norm_gemv_one_pass(N, K, group_size, swiglu != 0);
     if (swiglu) {
         const dim3 grid(static_cast<unsigned>(N / 8));
         const SwigluY ep{y, gate_out};
@@ -708,9 +709,7 @@ static int rmsnorm_impl(const uint8_t* Wq, const float* scale, const uint16_t* x
 #undef SOI_N
         return launch_status(what);
     }
-    // each wave normalises the whole vector before its rows, so larger tiles than the plain GEMV's pay here
-    // (swept at K = 2048: N = 4096 / 6144 / 2048 best at 8 / 8 / 4 rows per wave)
-    const int R = N >= 4 * 1024 ? 8 : N >= 2 * 1024 ? 4 : N >= 1024 ? 2 : 1;
+    const int R = norm_gemv_rows(N);
     const bool full = cs && full_k && N % R == 0;
     const dim3 grid(static_cast<unsigned>(ceil_div64(N, R)));
     const StoreY ep{y};
@@ -718,8 +717,8 @@ static int rmsnorm_impl(const uint8_t* Wq, const float* scale, const uint16_t* x
     hipLaunchKernelGGL((gemv_int4_norm_kernel<RR, CS, FL, OP, StoreY>), grid, dim3(64), 0, s, rows, N, x, delta,   \
                        norm_weight, eps, x_out, h_out, ep, Ki, gi)
 #define SOI_NR(RR)                                      \
-    if (full && one && delta) SOI_N(RR, true, true, 1); \
-    else if (full && one) SOI_N(RR, true, true, 2);     \
+    if (one && delta) SOI_N(RR, true, true, 1);         \
+    else if (one) SOI_N(RR, true, true, 2);             \
     else if (full) SOI_N(RR, true, true, 0);            \
     else if (cs) SOI_N(RR, true, false, 0);             \
     else SOI_N(RR, false, false, 0)
@@ -732,6 +731,10 @@ static int rmsnorm_impl(const uint8_t* Wq, const float* scale, const uint16_t* x
 #undef SOI_NR
 #undef SOI_N
     return launch_status(what);
+}
+
+extern "C" int soi_norm_gemv_one_pass(int64_t N, int64_t K, int64_t group_size, int swiglu) {
+    return norm_gemv_one_pass(N, K, group_size, swiglu != 0) ? 1 : 0;
 }
 
 extern "C" int soi_gemv_w4a16_rmsnorm(const uint8_t* Wq, const float* scale, const uint16_t* x, const uint16_t* delta,

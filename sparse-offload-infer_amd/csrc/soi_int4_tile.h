@@ -284,6 +284,14 @@ struct SplitGUY {
     }
 };
 
+// Rows per wave of the RMSNorm-fused GEMV, and whether it takes the one-pass form of the norm (RegNormX). Larger
+// tiles than the plain GEMV's pay there, as each wave normalises the whole vector before its rows (swept at K =
+// 2048: N = 4096 / 6144 / 2048 best at 8 / 8 / 4 rows per wave). The SwiGLU forms always run 8-row tiles.
+inline int norm_gemv_rows(int64_t N) { return N >= 4 * 1024 ? 8 : N >= 2 * 1024 ? 4 : N >= 1024 ? 2 : 1; }
+inline bool norm_gemv_one_pass(int64_t N, int64_t K, int64_t gs, bool swiglu) {
+    return gs % 32 == 0 && K == 2048 && (swiglu || N % norm_gemv_rows(N) == 0);
+}
+
 // Streaming GEMV kernels ask the compiler for at least 6 resident waves per
 // SIMD (<= 80 VGPRs, no spills at these tile sizes): with the default
 // allocation the 8-row tile takes ~120 VGPRs (4 waves), and the extra waves'

@@ -49,6 +49,9 @@ from ..quant import formats, pack
 
 # Generation steps per replay of the chunk graph (decode replays it for each full chunk of the requested steps)
 GRAPH_CHUNK = 4
+# Prompt tokens that go through the layers together (bounds the activations' scratch: about 50 KB per token of the
+# Qwen3-1.7B shape)
+PROMPT_CHUNK = 1024
 
 
 @dataclass(frozen=True)
@@ -352,6 +355,7 @@ class DecodeEngine:
         if offload:
             self._setup_offload()
         self._x_final = self.x
+        self._prompt_buf = None  # scratch of _prompt_layers, made by the first prompt
         self._graph_layers = None
         self._graph_gen = None
         self._graph_gen_chunk = None  # GRAPH_CHUNK generation steps in one graph
@@ -786,10 +790,57 @@ class DecodeEngine:
         self.log_len.zero_()
         self._step_open = False
 
+    # ---- prompts ----
+    def _prompt_together(self, n: int) -> bool:
+        """Whether n prompt tokens go through the layers together (_prompt_layers) instead of one at a time: fused
+        layers within the token kernels' limits, and nothing that watches single steps."""
+        c = self.c
+        return n > 1 and self.fused and self.layer_hook is None and self.counts is None and self.mode == "dense" and \
+            c.hidden % 32 == 0 and c.intermediate % 32 == 0 and c.q_heads * c.head_dim % 32 == 0 and \
+            c.group_size % 32 == 0 and \
+            bool(_C.attention_tokens_supported(c.q_heads, c.kv_heads, c.head_dim, c.max_seq))
+
+    def _prompt_scratch(self, T: int) -> dict:
+        """Activations of T tokens, kept for the next prompt (T <= PROMPT_CHUNK; grown in powers of two)."""
+        if self._prompt_buf is None or self._prompt_buf["T"] < T:
+            c, cap = self.c, 1 << (T - 1).bit_length()
+
+            def buf(n):
+                return torch.empty(cap * n, dtype=torch.float16, device=self.device)
+
+            self._prompt_buf = dict(T=cap, x=buf(c.hidden), h=buf(c.hidden), qkv=buf(c.qkv_rows),
+                                    q=buf(c.q_heads * c.head_dim), attn=buf(c.q_heads * c.head_dim),
+                                    gu=buf(2 * c.intermediate), m=buf(c.intermediate))
+        return self._prompt_buf
+
+    def _prompt_layers(self, tokens: torch.Tensor):
+        """Every layer over the given tokens at positions pos, pos + 1, ... (device int32), then the final norm of
+        the last one; pos += their count. The hidden states and caches of _layers() token by token, bit for bit."""
+        c, T, eps, gs = self.c, tokens.numel(), self.c.rms_eps, self.c.group_size
+        b = self._prompt_scratch(T)
+        x = b["x"]
+        _C.embed_tokens_into(self.w.embed, tokens, x)
+        for l, L in enumerate(self.w.layers):
+            L, gu_il = self._layer(l, L)
+            _C.prompt_attention_(T, x, L.in_norm, b["h"], L.qkv_Wq, L.qkv_scale, b["qkv"], L.q_norm, L.k_norm,
+                                 self.cos_t, self.sin_t, self.pos, b["q"], self.k_cache[l], self.v_cache[l],
+                                 b["attn"], L.o_Wq, L.o_scale, gs, eps)
+            _C.prompt_mlp_dense_(T, x, L.post_norm, b["h"], *gu_il, b["gu"], b["m"], L.down_Wq, L.down_scale, gs, eps)
+            self._layer_done(l)
+        last = x[(T - 1) * c.hidden:T * c.hidden]
+        self._x_final.copy_(last)
+        _C.rmsnorm_into(last, self.w.final_norm, self.hn, eps)
+        _C.advance_position(self.pos, T)
+
     def prefill(self, prompt_ids, use_graph: bool = True):
         prompt = torch.as_tensor(list(prompt_ids), dtype=torch.int32, device=self.device)
         if prompt.numel() + 1 > self.c.max_seq:
             raise ValueError("prompt longer than the KV cache")
+        if self._prompt_together(prompt.numel()):
+            for part in prompt.split(PROMPT_CHUNK):
+                self._prompt_layers(part)
+            self.token.copy_(prompt[-1:])
+            return
         for i in range(prompt.numel()):
             self.token.copy_(prompt[i:i + 1])
             if use_graph:
