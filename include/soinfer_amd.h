@@ -659,9 +659,19 @@ int soi_embed_tokens(const uint16_t* table, int64_t rows, int64_t hidden, const 
                      uint16_t* out, void* stream);
 int soi_norm_gemv_one_pass(int64_t N, int64_t K, int64_t group_size, int swiglu);
 int soi_norm_tokens(const uint16_t* x, const uint16_t* weight, float eps, uint16_t* h, int64_t T, int64_t hidden,
-                    int one_pass, void* stream);
+                    int one_pass, int frag, void* stream);
 int soi_gemm_w4a16_tokens(const uint8_t* Wq, const float* scale, const uint16_t* x, uint16_t* y, int64_t N, int64_t K,
                           int64_t group_size, int64_t T, int add, void* stream);
+/* The same products on the matrix cores: binary32 sums over exact operands in another order than
+ * soi_gemm_w4a16_tokens (N a multiple of 4, K and group_size multiples of 128: soi_gemm_w4a16_mfma_supported; Wq and
+ * x 16-byte, y 8-byte aligned). x is in fragment layout: room for T rounded up to 16 tokens, element (t, k) at
+ *   ((((t/16) * (K/128) + k/128) * 4 + (k/8)%4) * 64 + ((k/32)%4) * 16 + t%16) * 8 + k%8,
+ * which soi_norm_tokens and soi_attention_tokens write with `frag` set. epilogue 0: y[t, n] = fp16(sum); 1: y[t, n]
+ * += fp16(sum), one binary16 addition; 2 (N % 256 == 0, rows interleaved by 8-row tiles, 4 gate then 4 up): y[t, i] =
+ * fp16(silu(fp16 gate) * fp16 up), [T, N/2] in fragment layout. */
+int soi_gemm_w4a16_mfma_supported(int64_t N, int64_t K, int64_t group_size);
+int soi_gemm_w4a16_mfma(const uint8_t* Wq, const float* scale, const uint16_t* x, uint16_t* y, int64_t N, int64_t K,
+                        int64_t group_size, int64_t T, int epilogue, void* stream);
 int soi_silu_mul_tokens(const uint16_t* gate_up, uint16_t* h, int64_t T, int64_t I, int interleaved, void* stream);
 int soi_qk_norm_rope_tokens(const uint16_t* qkv, const uint16_t* q_norm, const uint16_t* k_norm,
                             const float* cos_table, const float* sin_table, const int32_t* pos, uint16_t* q_out,
@@ -670,7 +680,7 @@ int soi_qk_norm_rope_tokens(const uint16_t* qkv, const uint16_t* q_norm, const u
 int soi_attention_tokens_supported(int64_t num_q_heads, int64_t num_kv_heads, int64_t head_dim, int64_t max_seq);
 int soi_attention_tokens(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v_cache, uint16_t* out,
                          const int32_t* pos, int64_t T, int64_t num_q_heads, int64_t num_kv_heads, int64_t max_seq,
-                         int64_t head_dim, float scale, void* stream);
+                         int64_t head_dim, float scale, int frag, void* stream);
 
 #ifdef __cplusplus
 }

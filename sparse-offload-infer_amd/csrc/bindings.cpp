@@ -1570,6 +1570,15 @@ void need_int4(const torch::Tensor& Wq, const torch::Tensor& scale, const torch:
                 arg, "): scale must be [N, ceil(K/group_size)]");
 }
 
+// One linear over T tokens: y = or += W x, on the matrix cores (x in fragment layout) or in the decode step's order.
+int prompt_linear(const torch::Tensor& Wq, const torch::Tensor& scale, const uint16_t* x, uint16_t* y, int64_t K,
+                  int64_t gs, int64_t T, bool add, bool mfma, void* st) {
+    const int64_t N = Wq.size(0);
+    if (mfma)
+        return soi_gemm_w4a16_mfma(Wq.data_ptr<uint8_t>(), scale.data_ptr<float>(), x, y, N, K, gs, T, add ? 1 : 0, st);
+    return soi_gemm_w4a16_tokens(Wq.data_ptr<uint8_t>(), scale.data_ptr<float>(), x, y, N, K, gs, T, add ? 1 : 0, st);
+}
+
 }  // namespace
 
 void embed_tokens_into(torch::Tensor table, torch::Tensor tokens, torch::Tensor out) {
@@ -1591,7 +1600,7 @@ void prompt_attention_(int64_t T, torch::Tensor x, torch::Tensor norm, torch::Te
                        torch::Tensor qkv_scale, torch::Tensor qkv, torch::Tensor q_norm, torch::Tensor k_norm,
                        torch::Tensor cos_table, torch::Tensor sin_table, torch::Tensor pos, torch::Tensor q,
                        torch::Tensor k_cache, torch::Tensor v_cache, torch::Tensor attn, torch::Tensor o_Wq,
-                       torch::Tensor o_scale, int64_t group_size, double eps) {
+                       torch::Tensor o_scale, int64_t group_size, double eps, bool mfma) {
     const char* n = "prompt_attention_";
     TORCH_CHECK(T >= 1, n, ": T must be positive");
     for (const torch::Tensor* t : {&x, &norm, &h, &qkv, &q_norm, &k_norm, &q, &k_cache, &v_cache, &attn})
@@ -1610,35 +1619,34 @@ void prompt_attention_(int64_t T, torch::Tensor x, torch::Tensor norm, torch::Te
     TORCH_CHECK(q_norm.numel() == hd && k_norm.numel() == hd && cos_table.numel() == S * (hd / 2) &&
                     sin_table.numel() == S * (hd / 2),
                 n, ": norm or RoPE table shape mismatch");
+    const int64_t T16 = (T + 15) / 16 * 16;  // whole 16-token tiles in fragment layout
     need_numel(x, T * H, n, "x");
-    need_numel(h, T * H, n, "h");
+    need_numel(h, T16 * H, n, "h");
     need_numel(qkv, T * rows, n, "qkv");
     need_numel(q, T * NQ * hd, n, "q");
-    need_numel(attn, T * NQ * hd, n, "attn");
+    need_numel(attn, T16 * NQ * hd, n, "attn");
+    const bool mfma_qkv = mfma && soi_gemm_w4a16_mfma_supported(rows, H, group_size);
+    const bool mfma_o = mfma && soi_gemm_w4a16_mfma_supported(H, NQ * hd, group_size);
     const at::DeviceGuard guard(x.device());
     void* st = cur_stream(x);
     check_status(soi_norm_tokens(h16(x), h16(norm), static_cast<float>(eps), h16m(h), T, H,
-                                 soi_norm_gemv_one_pass(rows, H, group_size, 0), st),
+                                 soi_norm_gemv_one_pass(rows, H, group_size, 0), mfma_qkv, st),
                  n);
-    check_status(soi_gemm_w4a16_tokens(qkv_Wq.data_ptr<uint8_t>(), qkv_scale.data_ptr<float>(), h16(h), h16m(qkv), rows,
-                                       H, group_size, T, 0, st),
-                 n);
+    check_status(prompt_linear(qkv_Wq, qkv_scale, h16(h), h16m(qkv), H, group_size, T, false, mfma_qkv, st), n);
     check_status(soi_qk_norm_rope_tokens(h16(qkv), h16(q_norm), h16(k_norm), cos_table.data_ptr<float>(),
                                          sin_table.data_ptr<float>(), pos.data_ptr<int32_t>(), h16m(q), h16m(k_cache),
                                          h16m(v_cache), T, NQ, NKV, S, hd, static_cast<float>(eps), st),
                  n);
     check_status(soi_attention_tokens(h16(q), h16(k_cache), h16(v_cache), h16m(attn), pos.data_ptr<int32_t>(), T, NQ,
-                                      NKV, S, hd, 1.0f / std::sqrt(static_cast<float>(hd)), st),
+                                      NKV, S, hd, 1.0f / std::sqrt(static_cast<float>(hd)), mfma_o, st),
                  n);
-    check_status(soi_gemm_w4a16_tokens(o_Wq.data_ptr<uint8_t>(), o_scale.data_ptr<float>(), h16(attn), h16m(x), H,
-                                       NQ * hd, group_size, T, 1, st),
-                 n);
+    check_status(prompt_linear(o_Wq, o_scale, h16(attn), h16m(x), NQ * hd, group_size, T, true, mfma_o, st), n);
 }
 
 // x[t] += down(fp16(silu(gate) * up)) of rmsnorm(x[t]) for T tokens; gu rows interleaved by 8-row tiles. h, gu, m: scratch.
 void prompt_mlp_dense_(int64_t T, torch::Tensor x, torch::Tensor norm, torch::Tensor h, torch::Tensor gu_Wq,
                        torch::Tensor gu_scale, torch::Tensor gu, torch::Tensor m, torch::Tensor down_Wq,
-                       torch::Tensor down_scale, int64_t group_size, double eps) {
+                       torch::Tensor down_scale, int64_t group_size, double eps, bool mfma) {
     const char* n = "prompt_mlp_dense_";
     TORCH_CHECK(T >= 1, n, ": T must be positive");
     for (const torch::Tensor* t : {&x, &norm, &h, &gu, &m}) need(*t, torch::kFloat16, x, n, "fp16 operand");
@@ -1649,21 +1657,25 @@ void prompt_mlp_dense_(int64_t T, torch::Tensor x, torch::Tensor norm, torch::Te
     need_int4(down_Wq, down_scale, x, I, group_size, n, "down");
     TORCH_CHECK(down_Wq.size(0) == H, n, ": down must have hidden rows");
     need_numel(x, T * H, n, "x");
-    need_numel(h, T * H, n, "h");
+    const int64_t T16 = (T + 15) / 16 * 16;
+    need_numel(h, T16 * H, n, "h");
     need_numel(gu, T * 2 * I, n, "gu");
-    need_numel(m, T * I, n, "m");
+    need_numel(m, T16 * I, n, "m");
+    mfma = mfma && soi_gemm_w4a16_mfma_supported(2 * I, H, group_size) && soi_gemm_w4a16_mfma_supported(H, I, group_size);
     const at::DeviceGuard guard(x.device());
     void* st = cur_stream(x);
     check_status(soi_norm_tokens(h16(x), h16(norm), static_cast<float>(eps), h16m(h), T, H,
-                                 soi_norm_gemv_one_pass(2 * I, H, group_size, 1), st),
+                                 soi_norm_gemv_one_pass(2 * I, H, group_size, 1), mfma, st),
                  n);
-    check_status(soi_gemm_w4a16_tokens(gu_Wq.data_ptr<uint8_t>(), gu_scale.data_ptr<float>(), h16(h), h16m(gu), 2 * I,
-                                       H, group_size, T, 0, st),
-                 n);
-    check_status(soi_silu_mul_tokens(h16(gu), h16m(m), T, I, 1, st), n);
-    check_status(soi_gemm_w4a16_tokens(down_Wq.data_ptr<uint8_t>(), down_scale.data_ptr<float>(), h16(m), h16m(x), H, I,
-                                       group_size, T, 1, st),
-                 n);
+    if (mfma) {
+        check_status(soi_gemm_w4a16_mfma(gu_Wq.data_ptr<uint8_t>(), gu_scale.data_ptr<float>(), h16(h), h16m(m), 2 * I,
+                                         H, group_size, T, 2, st),
+                     n);
+    } else {
+        check_status(prompt_linear(gu_Wq, gu_scale, h16(h), h16m(gu), H, group_size, T, false, false, st), n);
+        check_status(soi_silu_mul_tokens(h16(gu), h16m(m), T, I, 1, st), n);
+    }
+    check_status(prompt_linear(down_Wq, down_scale, h16(m), h16m(x), I, group_size, T, true, mfma, st), n);
 }
 
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {

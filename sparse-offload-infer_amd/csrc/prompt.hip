@@ -17,6 +17,7 @@
 #include "soi_host.h"
 #include "soi_attn.h"
 #include "soi_int4_tile.h"
+#include "soi_prompt.h"
 
 namespace soi {
 
@@ -38,13 +39,14 @@ __global__ __launch_bounds__(256) void embed_tokens_kernel(const uint16_t* __res
 // RMSNorm rows
 // ---------------------------------------------------------------------------
 // h[t] = rmsnorm(x[t], w), one wave per token, with the partition of the norm-fused GEMVs: REG, the one-pass form
-// (hidden 2048: lane l sums its 32 elements), else NormX's (lane l sums 16-byte chunks l, l + 64, ...).
+// (hidden 2048: lane l sums its 32 elements), else NormX's (lane l sums 16-byte chunks l, l + 64, ...). frag: h in
+// fragment layout.
 constexpr int kNormTokens = 4;  // waves (tokens) per workgroup
 
 template <bool REG>
 __global__ __launch_bounds__(kNormTokens * kWave) void norm_tokens_kernel(const uint16_t* __restrict__ x,
                                                                           const uint16_t* __restrict__ w, float eps,
-                                                                          uint16_t* __restrict__ h, int T, int K) {
+                                                                          uint16_t* __restrict__ h, int T, int K, int frag) {
     const int lane = threadIdx.x & 63;
     const int t = static_cast<int>(blockIdx.x) * kNormTokens + static_cast<int>(threadIdx.x >> 6);
     if (t >= T) return;  // wave-uniform
@@ -73,7 +75,7 @@ __global__ __launch_bounds__(kNormTokens * kWave) void norm_tokens_kernel(const 
         r.y = norm_f16x2(s.y, g.y, inv);
         r.z = norm_f16x2(s.z, g.z, inv);
         r.w = norm_f16x2(s.w, g.w, inv);
-        stg(h4 + c, r);
+        stg(frag ? reinterpret_cast<u32x4*>(h + frag_offset(t, 8 * c, K)) : h4 + c, r);
     }
 }
 
@@ -330,7 +332,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_tokens_kernel(const uint16_
                                                                    const uint16_t* __restrict__ vc,
                                                                    uint16_t* __restrict__ out,
                                                                    const int32_t* __restrict__ pos_ptr, int NQ, int NKV,
-                                                                   int S, float scale_log2) {
+                                                                   int S, float scale_log2, int frag) {
     constexpr int HD = LPR * 8;
     constexpr int RPI = kWave / LPR;
     constexpr int STEP = RPI * kAttnWaves;
@@ -347,6 +349,8 @@ __global__ __launch_bounds__(kAttnThreads) void attn_tokens_kernel(const uint16_
     const uint16_t* kbase = kc + static_cast<int64_t>(kvh) * S * HD;
     const uint16_t* vbase = vc + static_cast<int64_t>(kvh) * S * HD;
     const int64_t qo = (static_cast<int64_t>(t_q) * NQ + h) * HD;
+    // element d of the head's output: fragment layout (the o projection's x on the matrix cores) or [T, NQ * HD]
+    auto out_at = [&](int d) { return out + (frag ? frag_offset(t_q, h * HD + d, static_cast<int64_t>(NQ) * HD) : qo + d); };
     f16x2 qv[1][4];
     {
         const u32x4 r = ldg(reinterpret_cast<const u32x4*>(q + qo) + u);
@@ -371,7 +375,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_tokens_kernel(const uint16_
                 s_split[split * (HD + 2) + e] = v;
             } else if (e >= 2) {
                 const float lsum = wave_sum<1, HD>(s_state, 0, 1, w);
-                stg(out + qo + e - 2, f32_to_f16_bits(v / lsum));
+                stg(out_at(e - 2), f32_to_f16_bits(v / lsum));
             }
         }
         __syncthreads();  // the split's state is read before the next split's waves overwrite s_state
@@ -386,7 +390,7 @@ __global__ __launch_bounds__(kAttnThreads) void attn_tokens_kernel(const uint16_
             lsum = fmaf(s_split[s * (HD + 2) + 1], w, lsum);
             acc = fmaf(s_split[s * (HD + 2) + 2 + d], w, acc);
         }
-        stg(out + qo + d, f32_to_f16_bits(acc / lsum));
+        stg(out_at(d), f32_to_f16_bits(acc / lsum));
     }
 }
 
@@ -456,22 +460,23 @@ extern "C" int soi_embed_tokens(const uint16_t* table, int64_t rows, int64_t hid
 }
 
 extern "C" int soi_norm_tokens(const uint16_t* x, const uint16_t* weight, float eps, uint16_t* h, int64_t T,
-                               int64_t hidden, int one_pass, void* stream) {
+                               int64_t hidden, int one_pass, int frag, void* stream) {
     const char* what = "soi_norm_tokens";
     int s = check_tokens(T, what);
     if (s) return s;
     SOI_REQUIRE(hidden >= 8 && hidden % 8 == 0 && hidden <= (int64_t(1) << 24),
                 "%s: hidden must be a multiple of 8 in [8, 2^24]", what);
+    SOI_REQUIRE(!frag || hidden % 128 == 0, "%s: the fragment layout needs hidden %% 128 == 0", what);
     SOI_REQUIRE(!one_pass || hidden == 2048, "%s: the one-pass partition is for hidden = 2048", what);
     SOI_REQUIRE(x && weight && h && h != x, "%s: null pointer or h = x", what);
     SOI_REQUIRE(aligned16(x) && aligned16(weight) && aligned16(h), "%s: vectors must be 16-byte aligned", what);
     const dim3 grid(static_cast<unsigned>(ceil_div64(T, kNormTokens)));
     if (one_pass)
         hipLaunchKernelGGL(norm_tokens_kernel<true>, grid, dim3(kNormTokens * kWave), 0, as_stream(stream), x, weight,
-                           eps, h, static_cast<int>(T), static_cast<int>(hidden));
+                           eps, h, static_cast<int>(T), static_cast<int>(hidden), frag);
     else
         hipLaunchKernelGGL(norm_tokens_kernel<false>, grid, dim3(kNormTokens * kWave), 0, as_stream(stream), x, weight,
-                           eps, h, static_cast<int>(T), static_cast<int>(hidden));
+                           eps, h, static_cast<int>(T), static_cast<int>(hidden), frag);
     return launch_status(what);
 }
 
@@ -538,12 +543,13 @@ extern "C" int soi_attention_tokens_supported(int64_t NQ, int64_t NKV, int64_t h
 
 extern "C" int soi_attention_tokens(const uint16_t* q, const uint16_t* k_cache, const uint16_t* v_cache, uint16_t* out,
                                     const int32_t* pos, int64_t T, int64_t NQ, int64_t NKV, int64_t max_seq,
-                                    int64_t head_dim, float scale, void* stream) {
+                                    int64_t head_dim, float scale, int frag, void* stream) {
     const char* what = "soi_attention_tokens";
     int s = check_tokens(T, what);
     if (s) return s;
     SOI_REQUIRE(NQ >= 1 && NKV >= 1 && NQ % NKV == 0 && max_seq >= 1, "%s: bad head counts or max_seq_len", what);
     SOI_REQUIRE(q && k_cache && v_cache && out && pos, "%s: null pointer", what);
+    SOI_REQUIRE(!frag || NQ * head_dim % 128 == 0, "%s: the fragment layout needs NQ * head_dim %% 128 == 0", what);
     const size_t lds = attn_tokens_lds(NQ, NKV, head_dim, max_seq);
     if (!lds) {
         set_last_error("%s: head_dim must be a power of two in [8, 256], at most 8 query heads per KV head and a "
@@ -557,7 +563,7 @@ extern "C" int soi_attention_tokens(const uint16_t* q, const uint16_t* k_cache, 
     hipStream_t st = as_stream(stream);
 #define SOI_A(LL)                                                                                                     \
     hipLaunchKernelGGL(attn_tokens_kernel<LL>, grid, dim3(kAttnThreads), lds, st, q, k_cache, v_cache, out, pos,      \
-                       static_cast<int>(NQ), static_cast<int>(NKV), static_cast<int>(max_seq), scale_log2)
+                       static_cast<int>(NQ), static_cast<int>(NKV), static_cast<int>(max_seq), scale_log2, frag)
     switch (head_dim / 8) {
         case 1: SOI_A(1); break;
         case 2: SOI_A(2); break;

@@ -2,7 +2,11 @@
 hidden state, its norm and the first generated token bit for bit, at the edges of the token tiles (4 and 8 tokens),
 contexts past one attention workgroup's rows (split plan), ragged widths (hidden and attention widths that are no
 multiple of 2048 elements; the one-pass norm at hidden 2048), group sizes 32 to 128, a second prompt appended to the
-first, and streamed weights."""
+first, and streamed weights. The matrix-core products (dense prompts of PROMPT_MFMA tokens up) sum in another order:
+each is held to the binary64 product of the same operands, and the engine's state to the one-at-a-time state."""
+import ctypes
+from pathlib import Path
+
 import pytest
 import torch
 
@@ -30,6 +34,12 @@ def weights(request, dec):
     return dec.random_decoder(cfg, seed=7, linear_std=0.05, norm_jitter=0.1)
 
 
+@pytest.fixture
+def in_order(dec, monkeypatch):
+    """Prompts of every length in the decode step's order of operations."""
+    monkeypatch.setattr(dec, "PROMPT_MFMA", 1 << 30)
+
+
 def tokens(n, vocab, seed):
     return torch.randint(0, vocab, (n,), generator=torch.Generator().manual_seed(seed)).tolist()
 
@@ -49,8 +59,8 @@ def same_state(a, b, n, what):
     assert torch.equal(a.pos, b.pos) and torch.equal(a.token, b.token), f"{what}: position or token"
 
 
-@pytest.mark.parametrize("n", [2, 4, 5, 8, 9, 33, 301])
-def test_prompt_equals_single_steps(dec, weights, n):
+@pytest.mark.parametrize("n", [3, 4, 5, 8, 9, 33, 301])
+def test_prompt_equals_single_steps(dec, weights, in_order, n):
     a = dec.DecodeEngine(weights, "dense", max_new_tokens=2)
     b = dec.DecodeEngine(weights, "dense", max_new_tokens=2)
     prompt = tokens(n, weights.config.vocab, n)
@@ -78,3 +88,78 @@ def test_streamed_prompt_equals_resident(dec, weights):
         for _ in range(2):
             assert e.generate(prompt, 4) == want
             same_state(a, e, 24, f"overlap {overlap}")
+
+
+@pytest.mark.parametrize("n", [9, 16, 17, 65, 301])
+def test_matrix_core_prompt_near_single_steps(dec, weights, n):
+    """Each linear's binary16 result can move to a neighbour (2^-11), which the following layers carry: after two
+    layers the states stay within 1% of their largest element (the decode engine's own bound against the oracle on
+    such models is half of that on logits, which average the state)."""
+    a = dec.DecodeEngine(weights, "dense", max_new_tokens=2)
+    b = dec.DecodeEngine(weights, "dense", max_new_tokens=2)
+    prompt = tokens(n, weights.config.vocab, n)
+    for e in (a, b):
+        e.reset()
+    a.prefill(prompt)
+    one_at_a_time(b, prompt)
+    pairs = [(a.x_final, b.x_final), (a.hn, b.hn)]
+    for l in range(2):
+        pairs += [(a.k_cache[l][:, :n], b.k_cache[l][:, :n]), (a.v_cache[l][:, :n], b.v_cache[l][:, :n])]
+    for x, y in pairs:
+        x, y = x.float(), y.float()
+        assert (x - y).abs().max() <= 1e-2 * y.abs().max()
+    assert torch.equal(a.pos, b.pos)
+
+
+def fragments(x):
+    """x [T, K] in the layout soi_gemm_w4a16_mfma reads (tokens rounded up to 16; the rest NaN: never read into a
+    result)."""
+    T, K = x.shape
+    z = torch.full((-(-T // 16) * 16, K), float("nan"), dtype=x.dtype, device=x.device)
+    z[:T] = x
+    return z.view(-1, 16, K // 128, 4, 4, 8).permute(0, 2, 4, 3, 1, 5).contiguous()
+
+
+@pytest.mark.parametrize("N,K,gs", [(4, 128, 128), (20, 256, 256), (136, 1152, 128), (256, 1024, 128), (4096, 384, 384),
+                                    (2048, 6144, 128)])
+@pytest.mark.parametrize("T", [1, 16, 17, 33, 64, 65, 200])
+def test_matrix_core_linear(cuda, N, K, gs, T):
+    """Tiles of 16, 32 and 64 rows (N below, at and past each), one to four token tiles and their remainders, 4 and 8
+    waves over 1 to 48 steps, scale groups of 1 to 3 steps: against binary64. The sum of K products in binary32 is
+    within K 2^-24 of the sum of their absolute values; the result is then rounded to binary16."""
+    from soinfer.quant import formats, pack
+
+    lib = ctypes.CDLL(str(Path(pack.__file__).resolve().parent.parent / "libsoinfer_hip.so"))
+    g = torch.Generator(device=cuda).manual_seed(N + K + T)
+    qt = formats.quantize(torch.randn(N, K, generator=g, device=cuda) * 0.02, formats.QuantConfig(4, "group", gs))
+    W = pack.pack_int4(qt.qweight)[0].contiguous()
+    x = torch.randn(T, K, generator=g, device=cuda).half()
+    w64 = (qt.qweight.double().view(N, K // gs, gs) * qt.scale.double()[..., None]).view(N, K)
+    ref, mag = x.double() @ w64.T, x.double().abs() @ w64.abs().T
+    bound = K * 2.0 ** -24 * mag + 2.0 ** -11 * ref.abs() + 2.0 ** -24
+
+    def run(y, epilogue):
+        st = lib.soi_gemm_w4a16_mfma(*(ctypes.c_void_p(t.data_ptr()) for t in (W, qt.scale, fragments(x), y)),
+                                     *(ctypes.c_int64(v) for v in (N, K, gs, T)), ctypes.c_int(epilogue),
+                                     ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+        torch.cuda.synchronize()
+        return st
+
+    y = torch.full((T + 1, N), 7.0, dtype=torch.float16, device=cuda)
+    assert run(y, 0) == 0
+    assert bool(((y[:T].double() - ref).abs() <= bound).all())
+    assert bool((y[T] == 7.0).all()), "rows past the last token are untouched"
+    r = torch.randn(T, N, generator=g, device=cuda).half()
+    added = r.clone()
+    assert run(added, 1) == 0
+    assert torch.equal(added, r + y[:T]), "the residual form adds the same product once, in binary16"
+    h = torch.full((-(-T // 16) * 16 * (N // 2),), 7.0, dtype=torch.float16, device=cuda)
+    if N % 256:
+        assert run(h, 2) != 0, "the fragment layout of the gated output needs N / 2 a multiple of 128"
+        return
+    assert run(h, 2) == 0
+    t = y[:T].view(T, N // 8, 2, 4).float()
+    gate, up = t[:, :, 0], t[:, :, 1]
+    want = (gate / (1 + torch.exp(-gate)) * up).view(T, N // 2)
+    got = h.view(-1, N // 256, 4, 4, 16, 8).permute(0, 4, 1, 3, 2, 5).reshape(-1, N // 2)[:T].float()
+    assert bool(((got - want).abs() <= 2.0 ** -10 * want.abs() + 2.0 ** -24).all())
