@@ -1678,6 +1678,89 @@ void prompt_mlp_dense_(int64_t T, torch::Tensor x, torch::Tensor norm, torch::Te
     check_status(prompt_linear(down_Wq, down_scale, h16(m), h16m(x), I, group_size, T, true, mfma, st), n);
 }
 
+// x[t] += the DIP MLP of rmsnorm(x[t]) for T tokens: gate rows, the selection of k channels, up, the gating, the sparse
+// down over down_proj^T. Resident weights: gate_Wq holds gate then up rows [2 I, .] (up given as none). Cached: gate_Wq
+// holds the gate rows; the up and down^T rows that any token selects are fetched from the hot cache (cache_up,
+// cache_down, slot_of) or the host arena (device addresses) into the images, which then serve as the matrices.
+// norm_pair: the norm's partition of the gate|up launch (two rows per channel) instead of the gate launch's.
+// h, gu [T, 2 I], idx [T, k], hs [T, k]: scratch; mark [I]: stamps of earlier calls, none equal to `stamp`.
+void prompt_mlp_dip_(int64_t T, int64_t k, torch::Tensor x, torch::Tensor norm, torch::Tensor h, torch::Tensor gate_Wq,
+                     torch::Tensor gate_scale, torch::Tensor gu, torch::Tensor idx, torch::Tensor hs,
+                     c10::optional<torch::Tensor> down_Wq, torch::Tensor down_scale, int64_t group_size, double eps,
+                     bool norm_pair, c10::optional<torch::Tensor> up_scale, c10::optional<torch::Tensor> cache_up,
+                     c10::optional<torch::Tensor> cache_down, c10::optional<torch::Tensor> slot_of, int64_t host_up,
+                     int64_t host_down, c10::optional<torch::Tensor> image_up, c10::optional<torch::Tensor> image_down,
+                     c10::optional<torch::Tensor> mark, int64_t stamp) {
+    const char* n = "prompt_mlp_dip_";
+    TORCH_CHECK(T >= 1, n, ": T must be positive");
+    const bool cached = up_scale.has_value();
+    for (const torch::Tensor* t : {&x, &norm, &h, &gu, &hs}) need(*t, torch::kFloat16, x, n, "fp16 operand");
+    need(idx, torch::kInt32, x, n, "idx");
+    const int64_t H = norm.numel();
+    need_int4(gate_Wq, gate_scale, x, H, group_size, n, "gate");
+    const int64_t I = cached ? gate_Wq.size(0) : gate_Wq.size(0) / 2;
+    TORCH_CHECK(cached || gate_Wq.size(0) == 2 * I, n, ": resident weights need gate and up rows [2 I, .]");
+    TORCH_CHECK(k >= 1 && k <= I, n, ": k must be in [1, I]");
+    need_numel(x, T * H, n, "x");
+    need_numel(h, T * H, n, "h");
+    need_numel(gu, T * 2 * I, n, "gu");
+    need_numel(idx, T * k, n, "idx");
+    need_numel(hs, T * k, n, "hs");
+    if (cached) {
+        TORCH_CHECK(cache_up && cache_down && slot_of && image_up && image_down && mark && host_up && host_down, n,
+                    ": the cached form needs every cache argument");
+        need_int4(*image_up, *up_scale, x, H, group_size, n, "image_up");
+        need_int4(*image_down, down_scale, x, H, group_size, n, "image_down");
+        for (const torch::Tensor* t : {&*cache_up, &*cache_down}) {
+            need(*t, torch::kUInt8, x, n, "cache");
+            TORCH_CHECK(t->dim() == 2 && t->size(0) == cache_up->size(0) && (t->numel() == 0 || t->size(1) == image_up->size(1)),
+                        n, ": cache rows must match the images'");
+        }
+        need(*slot_of, torch::kInt32, x, n, "slot_of");
+        need(*mark, torch::kInt32, x, n, "mark");
+        need_numel(*slot_of, I, n, "slot_of");
+        need_numel(*mark, I, n, "mark");
+        TORCH_CHECK(image_up->size(0) == I && image_down->size(0) == I, n, ": images must have I rows");
+    } else {
+        TORCH_CHECK(down_Wq.has_value(), n, ": resident weights need down_Wq");
+        need_int4(*down_Wq, down_scale, x, H, group_size, n, "down");
+        TORCH_CHECK(down_Wq->size(0) == I, n, ": down^T must have I rows");
+    }
+    const at::DeviceGuard guard(x.device());
+    void* st = cur_stream(x);
+    const int64_t ld = cached ? I : 2 * I;
+    uint16_t* gate = h16m(gu);
+    uint16_t* up = gate + (cached ? T * I : I);
+    int32_t* ip = idx.data_ptr<int32_t>();
+    check_status(soi_norm_tokens(h16(x), h16(norm), static_cast<float>(eps), h16m(h), T, H,
+                                 norm_pair ? soi_norm_gemv_one_pass(2 * I, H, group_size, 1)
+                                           : soi_norm_gemv_one_pass(I, H, group_size, 0),
+                                 0, st),
+                 n);
+    check_status(prompt_linear(gate_Wq, gate_scale, h16(h), gate, H, group_size, T, false, false, st), n);
+    check_status(soi_dip_select_tokens(gate, ld, I, k, T, ip, cached ? mark->data_ptr<int32_t>() : nullptr,
+                                       static_cast<int32_t>(stamp), st),
+                 n);
+    const uint8_t* down = nullptr;
+    if (cached) {
+        const int64_t rb = image_up->size(1);
+        check_status(soi_dip_fetch_rows(cache_up->data_ptr<uint8_t>(), reinterpret_cast<const uint8_t*>(host_up),
+                                        image_up->data_ptr<uint8_t>(), rb, cache_down->data_ptr<uint8_t>(),
+                                        reinterpret_cast<const uint8_t*>(host_down), image_down->data_ptr<uint8_t>(),
+                                        rb, I, cache_up->size(0), slot_of->data_ptr<int32_t>(),
+                                        mark->data_ptr<int32_t>(), static_cast<int32_t>(stamp), st),
+                     n);
+        check_status(prompt_linear(*image_up, *up_scale, h16(h), up, H, group_size, T, false, false, st), n);
+        down = image_down->data_ptr<uint8_t>();
+    } else {
+        down = down_Wq->data_ptr<uint8_t>();
+    }
+    check_status(soi_dip_gate_tokens(gate, up, ld, I, ip, h16m(hs), k, T, st), n);
+    check_status(soi_sparse_down_tokens(down, down_scale.data_ptr<float>(), I, ip, h16(hs), h16m(x), H, k, group_size,
+                                        T, st),
+                 n);
+}
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.doc() = "soinfer MI355X (gfx950) quantized decode hot path";
     m.def("gemv_w8a16", &gemv_w8a16, "INT8 GEMV");
@@ -1790,5 +1873,13 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("attention_tokens_supported", &soi_attention_tokens_supported, "whether prompt_attention_ takes the heads");
     m.def("prompt_attention_", &prompt_attention_, "one layer's attention block over T tokens, added to x");
     m.def("prompt_mlp_dense_", &prompt_mlp_dense_, "one layer's dense MLP over T tokens, added to x");
+    m.def("dip_tokens_max_channels", &soi_dip_tokens_max_channels, "most channels prompt_mlp_dip_ selects from");
+    m.def("prompt_mlp_dip_", &prompt_mlp_dip_, "one layer's DIP MLP over T tokens, added to x", py::arg("T"),
+          py::arg("k"), py::arg("x"), py::arg("norm"), py::arg("h"), py::arg("gate_Wq"), py::arg("gate_scale"),
+          py::arg("gu"), py::arg("idx"), py::arg("hs"), py::arg("down_Wq"), py::arg("down_scale"),
+          py::arg("group_size"), py::arg("eps"), py::arg("norm_pair"), py::arg("up_scale") = py::none(),
+          py::arg("cache_up") = py::none(), py::arg("cache_down") = py::none(), py::arg("slot_of") = py::none(),
+          py::arg("host_up") = 0, py::arg("host_down") = 0, py::arg("image_up") = py::none(),
+          py::arg("image_down") = py::none(), py::arg("mark") = py::none(), py::arg("stamp") = 0);
     m.def("version", []() { return std::string(soi_version()); });
 }

@@ -800,7 +800,11 @@ class DecodeEngine:
         layers within the token kernels' limits, and nothing that watches single steps. Two tokens are faster one at
         a time (1.14 against 1.29 ms, three 1.70 against 1.29)."""
         c = self.c
-        return n > 2 and self.fused and self.layer_hook is None and self.counts is None and self.mode == "dense" and \
+        if self.mode != "dense" and (self.dip_dense_up or c.intermediate > _C.dip_tokens_max_channels()):
+            return False  # the dense-up schedule's down sums in an order of its own
+        if self.counts is not None and self.mode == "cached_dip":
+            return False
+        return n > 2 and self.fused and self.layer_hook is None and \
             c.hidden % 32 == 0 and c.intermediate % 32 == 0 and c.q_heads * c.head_dim % 32 == 0 and \
             c.group_size % 32 == 0 and \
             bool(_C.attention_tokens_supported(c.q_heads, c.kv_heads, c.head_dim, c.max_seq))
@@ -815,25 +819,56 @@ class DecodeEngine:
 
             self._prompt_buf = dict(T=cap, x=buf(c.hidden), h=buf(c.hidden), qkv=buf(c.qkv_rows),
                                     q=buf(c.q_heads * c.head_dim), attn=buf(c.q_heads * c.head_dim),
-                                    gu=buf(2 * c.intermediate), m=buf(c.intermediate))
+                                    gu=buf(2 * c.intermediate))
+            if self.mode == "dense":
+                self._prompt_buf["m"] = buf(c.intermediate)
+            else:
+                self._prompt_buf["hs"] = buf(self.k)
+                self._prompt_buf["idx"] = torch.empty(cap * self.k, dtype=torch.int32, device=self.device)
+            if self.mode == "cached_dip":  # images of one layer's up and down^T rows, and which rows are current
+                self._prompt_buf["images"] = [torch.empty(c.intermediate, self.st_up.shape[1], dtype=torch.uint8,
+                                                          device=self.device) for _ in range(2)]
+                self._prompt_buf["mark"] = torch.zeros(c.intermediate, dtype=torch.int32, device=self.device)
+                self._prompt_stamp = 0
         return self._prompt_buf
+
+    def _prompt_mlp(self, l: int, L: LayerWeights, gu_il, b: dict, T: int, mfma: bool):
+        """Layer l's MLP over T prompt tokens, added to their hidden states."""
+        c, I, gs, eps = self.c, self.c.intermediate, self.c.group_size, self.c.rms_eps
+        if self.mode == "dense":
+            _C.prompt_mlp_dense_(T, b["x"], L.post_norm, b["h"], *gu_il, b["gu"], b["m"], L.down_Wq, L.down_scale, gs,
+                                 eps, mfma)
+            return
+        args = (T, self.k, b["x"], L.post_norm, b["h"])
+        if self.mode == "dip":
+            _C.prompt_mlp_dip_(*args, L.gu_Wq, L.gu_scale, b["gu"], b["idx"], b["hs"], L.down_T_Wq, L.down_T_scale, gs,
+                               eps, self.dip_gated)
+            if self.counts is not None:
+                sel = b["idx"][:T * self.k].long()
+                self.counts[l].index_add_(0, sel, torch.ones_like(sel, dtype=self.counts[l].dtype))
+            return
+        cache, (up, down) = self.caches[l], b["images"]
+        self._prompt_stamp += 1
+        _C.prompt_mlp_dip_(*args, *L.gate(I), b["gu"], b["idx"], b["hs"], None, L.down_T_scale, gs, eps, False,
+                           up_scale=L.up(I)[1], cache_up=cache.up_Wq, cache_down=cache.down_Wq, slot_of=cache.slot_of,
+                           host_up=self.host_up_ptr[l], host_down=self.host_down_ptr[l], image_up=up, image_down=down,
+                           mark=b["mark"], stamp=self._prompt_stamp)
 
     def _prompt_layers(self, tokens: torch.Tensor):
         """Every layer over the given tokens at positions pos, pos + 1, ... (device int32), then the final norm of
-        the last one; pos += their count. Below PROMPT_MFMA tokens the hidden states and caches of _layers() token by
-        token, bit for bit; from there on the linears' binary32 sums run in the matrix cores' order."""
+        the last one; pos += their count. The hidden states and caches of _layers() token by token, bit for bit, but
+        for dense prompts of PROMPT_MFMA tokens up, whose linears' binary32 sums run in the matrix cores' order."""
         c, T, eps, gs = self.c, tokens.numel(), self.c.rms_eps, self.c.group_size
         b = self._prompt_scratch(T)
         x = b["x"]
-        mfma = T >= PROMPT_MFMA
+        mfma = self.mode == "dense" and T >= PROMPT_MFMA
         _C.embed_tokens_into(self.w.embed, tokens, x)
         for l, L in enumerate(self.w.layers):
             L, gu_il = self._layer(l, L)
             _C.prompt_attention_(T, x, L.in_norm, b["h"], L.qkv_Wq, L.qkv_scale, b["qkv"], L.q_norm, L.k_norm,
                                  self.cos_t, self.sin_t, self.pos, b["q"], self.k_cache[l], self.v_cache[l],
                                  b["attn"], L.o_Wq, L.o_scale, gs, eps, mfma)
-            _C.prompt_mlp_dense_(T, x, L.post_norm, b["h"], *gu_il, b["gu"], b["m"], L.down_Wq, L.down_scale, gs, eps,
-                                 mfma)
+            self._prompt_mlp(l, L, gu_il, b, T, mfma)
             self._layer_done(l)
         last = x[(T - 1) * c.hidden:T * c.hidden]
         self._x_final.copy_(last)

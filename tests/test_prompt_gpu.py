@@ -90,6 +90,46 @@ def test_streamed_prompt_equals_resident(dec, weights):
             same_state(a, e, 24, f"overlap {overlap}")
 
 
+def dip_engines(dec, w, k):
+    hot = [list(range(0, w.config.intermediate, 3)) for _ in range(w.config.layers)]
+    none = [[] for _ in range(w.config.layers)]
+    return {"indexed": dict(mode="dip"), "gated": dict(mode="dip", dip_schedule="gated"),
+            "cached": dict(mode="cached_dip", hot_channels=hot),
+            "all missing": dict(mode="cached_dip", hot_channels=none, miss_path="staged"),
+            "streamed": dict(mode="cached_dip", hot_channels=hot, offload=True)}
+
+
+@pytest.mark.parametrize("n,frac", [(3, 0.5), (9, 0.02), (33, 0.9), (301, 0.5), (4, 1.0)])
+def test_dip_prompt_equals_single_steps(dec, weights, n, frac):
+    """DIP: one selected channel per 50 (a row chunk of a few rows) up to all of them (several row chunks and their
+    remainder), resident and cache-aware. The selections agree where the hidden states do."""
+    c = weights.config
+    k = max(1, int(c.intermediate * frac))
+    prompt, more = tokens(n, c.vocab, n), tokens(5, c.vocab, n + 1)
+    for what, kw in dip_engines(dec, weights, k).items():
+        a, b = (dec.DecodeEngine(weights, dip_k=k, max_new_tokens=2, **kw) for _ in range(2))
+        for e in (a, b):
+            e.reset()
+        assert a._prompt_together(n)
+        for part, total in ((prompt, n), (more, n + 5)):
+            a.prefill(part, use_graph=False)
+            one_at_a_time(b, part)
+            same_state(a, b, total, f"{what}, {total} tokens")
+
+
+def test_calibration_counts_of_a_prompt(dec, weights):
+    c = weights.config
+    prompt, k = tokens(21, c.vocab, 5), c.intermediate // 3
+    a, b = (dec.DecodeEngine(weights, "dip", dip_k=k, max_new_tokens=1) for _ in range(2))
+    for e in (a, b):
+        e.counts = [torch.zeros(c.intermediate, dtype=torch.int64, device="cuda") for _ in range(c.layers)]
+        e.reset()
+    a.prefill(prompt, use_graph=False)
+    one_at_a_time(b, prompt)
+    for l in range(c.layers):
+        assert torch.equal(a.counts[l], b.counts[l]) and int(a.counts[l].sum()) == 21 * k
+
+
 @pytest.mark.parametrize("n", [9, 16, 17, 65, 301])
 def test_matrix_core_prompt_near_single_steps(dec, weights, n):
     """Each linear's binary16 result can move to a neighbour (2^-11), which the following layers carry: after two
