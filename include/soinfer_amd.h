@@ -704,6 +704,21 @@ int soi_sparse_down_tokens(const uint8_t* Wq_T, const float* scale_T, int64_t nu
                            const uint16_t* h, uint16_t* x, int64_t H, int64_t k, int64_t group_size, int64_t T,
                            void* stream);
 
+/* --------------------------------------------------------------------------
+ * Quantization and packing on the device: the values of formats.quantize
+ * (granularity "group", min-max scales) and pack.pack_int4 (reference
+ * python/soinfer/quant/formats.py:24-123, pack.py:14-69).
+ *   soi_quantize_group: w fp32 [N, K] -> q int8 [N, ceil(K/gs) * gs] (zeros
+ *     past K, 4-byte aligned) and scale fp32 [N, ceil(K/gs)]; group_size 32,
+ *     64, 128 or 256 (soi_quantize_group_supported), qmax in [1, 127].
+ *   soi_pack_int4: q int8 [N, K] -> uint8 [N, ceil(K/8) * 4], AWQ nibble
+ *     order, zeros past K; out 4-byte aligned.
+ * ------------------------------------------------------------------------ */
+int soi_quantize_group_supported(int64_t group_size);
+int soi_quantize_group(const float* w, int8_t* q, float* scale, int64_t N, int64_t K, int64_t group_size, int64_t qmax,
+                       void* stream);
+int soi_pack_int4(const int8_t* q, uint8_t* out, int64_t N, int64_t K, void* stream);
+
 #ifdef __cplusplus
 }
 #endif

@@ -1761,6 +1761,30 @@ void prompt_mlp_dip_(int64_t T, int64_t k, torch::Tensor x, torch::Tensor norm, 
                  n);
 }
 
+std::tuple<torch::Tensor, torch::Tensor> quantize_group(torch::Tensor w, int64_t group_size, int64_t qmax) {
+    const char* n = "quantize_group";
+    need(w, torch::kFloat32, w, n, "w");
+    TORCH_CHECK(w.dim() == 2 && group_size >= 1, n, ": w must be [N, K]");
+    const int64_t N = w.size(0), K = w.size(1), G = expected_num_groups(K, group_size);
+    const at::DeviceGuard guard(w.device());
+    auto q = torch::empty({N, G * group_size}, w.options().dtype(torch::kInt8));
+    auto scale = torch::empty({N, G}, w.options());
+    check_status(soi_quantize_group(w.data_ptr<float>(), q.data_ptr<int8_t>(), scale.data_ptr<float>(), N, K, group_size,
+                                    qmax, cur_stream(w)),
+                 n);
+    return {q, scale};
+}
+
+torch::Tensor pack_int4(torch::Tensor q) {
+    const char* n = "pack_int4";
+    need(q, torch::kInt8, q, n, "q");
+    TORCH_CHECK(q.dim() == 2, n, ": q must be [N, K]");
+    const at::DeviceGuard guard(q.device());
+    auto out = torch::empty({q.size(0), (q.size(1) + 7) / 8 * 4}, q.options().dtype(torch::kUInt8));
+    check_status(soi_pack_int4(q.data_ptr<int8_t>(), out.data_ptr<uint8_t>(), q.size(0), q.size(1), cur_stream(q)), n);
+    return out;
+}
+
 PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.doc() = "soinfer MI355X (gfx950) quantized decode hot path";
     m.def("gemv_w8a16", &gemv_w8a16, "INT8 GEMV");
@@ -1881,5 +1905,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("cache_up") = py::none(), py::arg("cache_down") = py::none(), py::arg("slot_of") = py::none(),
           py::arg("host_up") = 0, py::arg("host_down") = 0, py::arg("image_up") = py::none(),
           py::arg("image_down") = py::none(), py::arg("mark") = py::none(), py::arg("stamp") = 0);
+    m.def("quantize_group", &quantize_group, "symmetric group quantization: (codes, scales)");
+    m.def("pack_int4", &pack_int4, "int8 codes to AWQ-order INT4 rows");
     m.def("version", []() { return std::string(soi_version()); });
 }

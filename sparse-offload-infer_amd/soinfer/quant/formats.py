@@ -22,7 +22,7 @@ from typing import Callable, Optional
 
 import torch
 
-from . import calibrate
+from . import _device, calibrate
 
 GRANULARITIES = ("per_tensor", "per_channel", "group", "block32", "mx_e8m0")
 BLOCK32 = 32
@@ -87,6 +87,12 @@ def quantize(w: torch.Tensor, config: QuantConfig, scale_fn: Optional[Callable] 
 
     gs = int(config.group_size)
     G = -(-K // gs)
+    if config.granularity != "mx_e8m0" and fn is calibrate.min_max and 2 <= config.bits <= 8 and gs in (32, 64, 128, 256) \
+            and _device.takes_kernel(w):
+        from .. import _C  # one pass over w: the same scales and codes (csrc/quantize.hip)
+
+        q, scale = _C.quantize_group(w.contiguous().view(-1, K), gs, qmax)
+        return QuantTensor(q.view(*w.shape[:-1], G * gs), scale.view(*w.shape[:-1], G), config, K)
     if G * gs != K:
         w = torch.nn.functional.pad(w, (0, G * gs - K))
     grouped = w.reshape(*w.shape[:-1], G, gs)

@@ -14,6 +14,8 @@ from __future__ import annotations
 
 import torch
 
+from . import _device
+
 GROUP = 8
 AWQ_ORDER = (0, 2, 4, 6, 1, 3, 5, 7)
 # logical position j of a word -> (byte, shift) holding it
@@ -39,6 +41,10 @@ def pack_int4(q: torch.Tensor) -> tuple[torch.Tensor, int]:
         raise ValueError(f"pack_int4 expects int8, got {q.dtype}")
     K = q.shape[-1]
     words = -(-K // GROUP)
+    if _device.takes_kernel(q):
+        from .. import _C  # the same bytes in one pass (csrc/quantize.hip)
+
+        return _C.pack_int4(q.contiguous().view(-1, K)).view(*q.shape[:-1], words * 4), K
     if words * GROUP != K:
         q = torch.nn.functional.pad(q, (0, words * GROUP - K))
     nib = (q.to(torch.int32) & 0xF).reshape(*q.shape[:-1], words, GROUP)
