@@ -719,6 +719,15 @@ int soi_quantize_group(const float* w, int8_t* q, float* scale, int64_t N, int64
                        void* stream);
 int soi_pack_int4(const int8_t* q, uint8_t* out, int64_t N, int64_t K, void* stream);
 
+/* y[N0 + N1] = W0 x, then W1 x (each row as soi_gemv_w4a16_group_lop3 gives it; both matrices [., K], N1 may be 0) in one
+ * launch. clear: this many words (at most N0 + N1) are set to zero, e.g. the arrival counters of a sparse down that
+ * follows on the stream. No reference counterpart. */
+int soi_gemv_w4a16_pair(const uint8_t* Wq0, const float* scale0, int64_t N0, const uint8_t* Wq1, const float* scale1,
+                        int64_t N1, const uint16_t* x, uint16_t* y, int64_t K, int64_t group_size, int64_t num_groups,
+                        uint32_t* clear, int64_t clear_words, void* stream);
+/* Arrival-counter words at the start of a soi_sparse_accumulate workspace (the part that must start at zero). */
+int64_t soi_sparse_accumulate_counter_words(int64_t H);
+
 #ifdef __cplusplus
 }
 #endif

@@ -511,6 +511,23 @@ extern "C" int soi_gemv_w4a16_group_lop3(const uint8_t* Wq, const float* scale, 
     return dense_int4<true>(Wq, scale, x, y, N, K, group_size, num_groups, stream, "soi_gemv_w4a16_group_lop3");
 }
 
+extern "C" int soi_gemv_w4a16_pair(const uint8_t* Wq0, const float* scale0, int64_t N0, const uint8_t* Wq1,
+                                   const float* scale1, int64_t N1, const uint16_t* x, uint16_t* y, int64_t K,
+                                   int64_t group_size, int64_t num_groups, uint32_t* clear, int64_t clear_words,
+                                   void* stream) {
+    const char* what = "soi_gemv_w4a16_pair";
+    int st = check_int4_common(K, group_size, num_groups, what);
+    if (st) return st;
+    SOI_REQUIRE(N0 >= 1 && N1 >= 0 && N0 + N1 <= (int64_t(1) << 31) - 1, "%s: N0 or N1 out of range", what);
+    SOI_REQUIRE(Wq0 && scale0 && x && y && (N1 == 0 || (Wq1 && scale1)), "%s: null pointer", what);
+    SOI_REQUIRE(clear_words >= 0 && clear_words <= N0 + N1 && (clear_words == 0 || clear),
+                "%s: at most one word per row can be cleared", what);
+    const bool vec = (K % 32 == 0) && aligned16(Wq0) && aligned16(x) && (N1 == 0 || aligned16(Wq1));
+    PairRows rows{Wq0, scale0, Wq1, scale1, N0, ceil_div64(K, 8) * 4, num_groups};
+    return launch_int4<true>(rows, N0 + N1, x, StoreYClear{y, clear, clear_words}, K, group_size, vec,
+                             as_stream(stream), what);
+}
+
 extern "C" int soi_gemv_w4a16_residual(const uint8_t* Wq, const float* scale, const uint16_t* x, uint16_t* y,
                                        const uint16_t* res, uint16_t* res_out, int64_t N, int64_t K,
                                        int64_t group_size, int64_t num_groups, void* stream) {

@@ -199,6 +199,21 @@ struct StoreY {
     }
 };
 
+// StoreYClear: StoreY, and word r of clear = 0 for every row r < words: arrival counters of a later launch on the
+// stream start at zero without a fill launch of their own.
+struct StoreYClear {
+    static constexpr bool kSwiglu = false;
+    static constexpr bool kPrefetch = false;
+    struct Pre {};
+    uint16_t* y;
+    uint32_t* clear;
+    int64_t words;
+    __device__ __forceinline__ void store(int64_t row, float total, bool valid) const {
+        stg(y + row, valid ? f32_to_f16_bits(total) : uint16_t(0x7e00u));
+        if (row < words) stg(clear + row, 0u);
+    }
+};
+
 // StoreYAdd: StoreY, and res_out[row] = res[row] + y[row] as one binary16 addition
 // (the residual update the next RMSNorm would otherwise do on load, with the same
 // rounding). res[row] is requested before the tile's weights.

@@ -32,6 +32,24 @@ struct DenseRows {
     __device__ __forceinline__ RowRef get(int64_t j) const { return resolve(key(j), j); }
 };
 
+// rows 0 .. N0-1 of one [N0, row_bytes] matrix, then the rows of a second of the same width
+struct PairRows {
+    const uint8_t* W0;
+    const float* S0;
+    const uint8_t* W1;
+    const float* S1;
+    int64_t N0;
+    int64_t row_bytes;
+    int64_t G;
+    __device__ __forceinline__ int64_t key(int64_t j) const { return j; }
+    __device__ __forceinline__ RowRef resolve(int64_t k, int64_t) const {
+        const bool first = k < N0;
+        const int64_t r = first ? k : k - N0;
+        return {(first ? W0 : W1) + r * row_bytes, (first ? S0 : S1) + r * G, true};
+    }
+    __device__ __forceinline__ RowRef get(int64_t j) const { return resolve(key(j), j); }
+};
+
 // row j resolved by descriptor: top bit set -> staging row, else cache row
 struct DescRows {
     const uint8_t* cW;

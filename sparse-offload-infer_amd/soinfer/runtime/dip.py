@@ -25,6 +25,7 @@ from typing import Optional
 import torch
 import torch.nn.functional as F
 
+from .. import _C
 from .. import ops
 from ..offload.hot_cache import HotCache
 
@@ -51,9 +52,7 @@ class DipMLPWeights:
 
 def select_channels(w: DipMLPWeights, x: torch.Tensor, dip_k: int) -> tuple[torch.Tensor, torch.Tensor]:
     """gate = W_gate x (dense) and the DIP selection idx (int32 [dip_k], ascending)."""
-    gate = ops.gemv_w4a16_group_lop3(w.gate_Wq, w.gate_scale, x, w.hidden_size, w.group_size)
-    abs_g = gate.float().abs().contiguous()
-    idx = ops.topk_threshold_select(abs_g, dip_k)
+    gate, idx, _ = _C.dip_gate_select(w.gate_Wq, w.gate_scale, x, dip_k, w.hidden_size, w.group_size)
     return gate, idx
 
 
@@ -64,14 +63,14 @@ def silu_gate(gate: torch.Tensor, idx: torch.Tensor, u: torch.Tensor) -> torch.T
 
 
 def dip_mlp(w: DipMLPWeights, x: torch.Tensor, dip_k: int, channel_counts: Optional[torch.Tensor] = None):
-    """Resident-weight DIP MLP. Returns (y [H] fp16, idx [dip_k] int32)."""
-    gate, idx = select_channels(w, x, dip_k)
+    """Resident-weight DIP MLP. Returns (y [H] fp16, idx [dip_k] int32). Two launches: gate and up of every channel,
+    then the selection inside the sparse down (up of an unselected channel is not used: reading it costs less than
+    the launch that would leave it out)."""
+    y, idx = _C.dip_mlp(w.gate_Wq, w.gate_scale, w.up_Wq, w.up_scale, w.down_T_Wq, w.down_T_scale, x, dip_k,
+                        w.hidden_size, w.group_size)
     if channel_counts is not None:
         channel_counts.scatter_add_(0, idx.long(), torch.ones(idx.shape[0], dtype=channel_counts.dtype,
                                                               device=idx.device))
-    u = ops.gemv_w4a16_indexed(w.up_Wq, w.up_scale, idx, x, w.hidden_size, w.group_size)
-    h = silu_gate(gate, idx, u)
-    y = ops.gemv_w4a16_indexed_accumulate(w.down_T_Wq, w.down_T_scale, idx, h, w.hidden_size, w.group_size)
     return y, idx
 
 
@@ -95,38 +94,78 @@ def dip_mlp_gathered(w: DipMLPWeights, x: torch.Tensor, dip_k: int):
 def cached_dip_mlp(w: DipMLPWeights, cache: HotCache, x: torch.Tensor, dip_k: int,
                    host_up: Optional[torch.Tensor] = None, host_down_T: Optional[torch.Tensor] = None,
                    staging: Optional[torch.Tensor] = None, miss_bytes: Optional[list] = None):
-    """Cache-aware DIP MLP: selected channels resident in `cache` are read from it, the misses from a
-    staging buffer; one fused kernel per direction. Misses are fetched from the device-resident weights
-    (default) or, when host_up / host_down_T (pinned [I, row_nbytes]) are given, from pinned host memory
-    through `staging` (pinned, >= dip_k * row_nbytes) with the staged H2D gather. Bit-identical to dip_mlp.
+    """Cache-aware DIP MLP: selected channels resident in `cache` are read from it, the misses from the
+    device-resident weights (default) or, when host_up / host_down_T (pinned [I, row_nbytes]) and `staging` (pinned,
+    >= dip_k * row_nbytes) are given, from pinned host memory. The kernels read pinned rows through their device
+    mapping; host tensors that have none go through `staging` with the staged H2D gather. Bit-identical to dip_mlp.
     Returns (y, idx, miss_count)."""
+    hosted = host_up is not None and host_down_T is not None
+    if hosted and not _mapped(w, host_up, host_down_T, staging, dip_k):
+        return _cached_mlp_staged(w, cache, x, dip_k, host_up, host_down_T, staging, miss_bytes)
+    count = torch.empty(1, dtype=torch.int32, pin_memory=True)
+    gate, idx, ws = _C.dip_gate_select(w.gate_Wq, w.gate_scale, x, dip_k, w.hidden_size, w.group_size, cache.slot_of,
+                                       count)
+    counted = torch.cuda.Event()
+    counted.record(torch.cuda.current_stream(x.device))
+    y = _cached_mlp(w, cache, x, gate, idx, ws, host_up if hosted else w.up_Wq, host_down_T if hosted else w.down_T_Wq)
+    counted.synchronize()  # the count is read while the GEMVs run
+    mc = int(count)
+    if miss_bytes is not None:
+        miss_bytes.append(mc * (w.up_Wq.shape[1] + w.down_T_Wq.shape[1]))
+    return y, idx, mc
+
+
+def _mapped(w: DipMLPWeights, host_up: torch.Tensor, host_down_T: torch.Tensor, staging, dip_k: int) -> bool:
+    """Whether the host rows are pinned matrices of the weights' shapes (readable by the kernels), with the staging
+    buffer that the gathers of the same call would need."""
+    def pinned(t):
+        return isinstance(t, torch.Tensor) and t.device.type == "cpu" and t.dtype == torch.uint8 and \
+            t.is_contiguous() and t.is_pinned()
+
+    return pinned(host_up) and pinned(host_down_T) and pinned(staging) and host_up.shape == w.up_Wq.shape and \
+        host_down_T.shape == w.down_T_Wq.shape and \
+        staging.numel() >= dip_k * max(host_up.shape[1], host_down_T.shape[1])
+
+
+def _cached_mlp_staged(w: DipMLPWeights, cache: HotCache, x: torch.Tensor, dip_k: int, host_up, host_down_T, staging,
+                       miss_bytes: Optional[list]):
+    """cached_dip_mlp with the misses gathered on the host, one matrix after the other through `staging`."""
     gate, idx = select_channels(w, x, dip_k)
     desc, miss_channels, miss_count = ops.build_dip_descriptors(idx, cache.slot_of)
     mc = int(miss_count.item())
-    miss = miss_channels[:mc]
-    miss_l = miss.long()
-    dev = x.device
-    up_st = torch.empty(mc, w.up_Wq.shape[1], dtype=torch.uint8, device=dev)
-    down_st = torch.empty(mc, w.down_T_Wq.shape[1], dtype=torch.uint8, device=dev)
+    miss_l = miss_channels[:mc].long()
+    up_st = torch.empty(mc, w.up_Wq.shape[1], dtype=torch.uint8, device=x.device)
+    down_st = torch.empty(mc, w.down_T_Wq.shape[1], dtype=torch.uint8, device=x.device)
     if mc:
-        if host_up is not None and host_down_T is not None:
-            miss_cpu = miss_l.cpu()
-            ops.gather_rows_staged(host_up, miss_cpu, staging, up_st)
-            torch.cuda.current_stream().synchronize()  # staging reused for the second gather
-            ops.gather_rows_staged(host_down_T, miss_cpu, staging, down_st)
-        else:
-            ops.gather_rows_device(w.up_Wq, miss, up_st)
-            ops.gather_rows_device(w.down_T_Wq, miss, down_st)
+        miss_cpu = miss_l.cpu()
+        ops.gather_rows_staged(host_up, miss_cpu, staging, up_st)
+        torch.cuda.current_stream().synchronize()  # staging reused for the second gather
+        ops.gather_rows_staged(host_down_T, miss_cpu, staging, down_st)
     if miss_bytes is not None:
         miss_bytes.append(mc * (w.up_Wq.shape[1] + w.down_T_Wq.shape[1]))
-    up_st_scale = w.up_scale.index_select(0, miss_l)
-    down_st_scale = w.down_T_scale.index_select(0, miss_l)
-    u = ops.gemv_dip_fused_up(cache.up_Wq, cache.up_scale, up_st, up_st_scale, desc, x, w.hidden_size,
-                              w.group_size)
+    u = ops.gemv_dip_fused_up(cache.up_Wq, cache.up_scale, up_st, w.up_scale.index_select(0, miss_l), desc, x,
+                              w.hidden_size, w.group_size)
     h = silu_gate(gate, idx, u)
-    y = ops.gemv_dip_fused_down(cache.down_Wq, cache.down_scale, down_st, down_st_scale, desc, h,
-                                w.hidden_size, w.group_size)
+    y = ops.gemv_dip_fused_down(cache.down_Wq, cache.down_scale, down_st, w.down_T_scale.index_select(0, miss_l), desc,
+                                h, w.hidden_size, w.group_size)
     return y, idx, mc
+
+
+def _cached_mlp(w: DipMLPWeights, cache: HotCache, x, gate, idx, ws, full_up, full_down_T) -> torch.Tensor:
+    """The up and down halves over the hot cache: hits from the cache, misses from full_up / full_down_T in place. For
+    misses in host memory the up GEMV also copies its channels' down^T rows to the device (whole rows cross PCIe faster
+    than the down's column slices)."""
+    H, gs, k = w.hidden_size, w.group_size, idx.shape[0]
+    h = torch.empty(k, dtype=torch.float16, device=x.device)
+    row = full_down_T.shape[1]
+    copy = not full_down_T.is_cuda and row % 16 == 0 and row <= 4096 and full_down_T.data_ptr() % 16 == 0
+    staged = torch.empty(k, row, dtype=torch.uint8, device=x.device) if copy else None
+    _C.gemv_dip_cached_up_silu_into(cache.up_Wq, cache.up_scale, full_up, w.up_scale, cache.slot_of, idx, x, gate, h, H,
+                                    gs, full_down_T if copy else None, staged)
+    y = torch.empty(H, dtype=torch.float16, device=x.device)
+    _C.gemv_dip_cached_down_into(cache.down_Wq, cache.down_scale, full_down_T, w.down_T_scale, cache.slot_of, idx, h, y,
+                                 H, gs, ws, staged)
+    return y
 
 
 def cached_dip_mlp_direct(w: DipMLPWeights, cache: HotCache, x: torch.Tensor, dip_k: int,
@@ -137,21 +176,16 @@ def cached_dip_mlp_direct(w: DipMLPWeights, cache: HotCache, x: torch.Tensor, di
     full_down_T (pinned host memory read through its device mapping, or device tensors; default: the
     resident weights). No descriptors, no gather, no staging buffer and no host sync; the SiLU gating is the
     up GEMV's epilogue. Bit-identical to dip_mlp and cached_dip_mlp. Returns (y, idx)."""
-    from .. import _C
-
-    gate, idx = select_channels(w, x, dip_k)
+    gate, idx, ws = _C.dip_gate_select(w.gate_Wq, w.gate_scale, x, dip_k, w.hidden_size, w.group_size)
     full_up = w.up_Wq if full_up is None else full_up
     full_down_T = w.down_T_Wq if full_down_T is None else full_down_T
     H, gs = w.hidden_size, w.group_size
     h = torch.empty(dip_k, dtype=torch.float16, device=x.device)
     _C.gemv_dip_cached_up_silu_into(cache.up_Wq, cache.up_scale, full_up, w.up_scale, cache.slot_of, idx, x, gate,
                                     h, H, gs)
-    if workspace is None:
-        workspace = torch.zeros(max(1, _C.sparse_accumulate_workspace_bytes(H, dip_k)), dtype=torch.uint8,
-                                device=x.device)
     y = torch.empty(H, dtype=torch.float16, device=x.device)
     _C.gemv_dip_cached_down_into(cache.down_Wq, cache.down_scale, full_down_T, w.down_T_scale, cache.slot_of, idx,
-                                 h, y, H, gs, workspace)
+                                 h, y, H, gs, ws if workspace is None else workspace)
     return y, idx
 
 
