@@ -258,14 +258,15 @@ int soi_gemv_w4a16_indexed_accumulate(const uint8_t* Wq_T, const float* scale_T,
  * kvh = h / (NQ/NKV), t < cur_len. q: fp16 [NQ, hd]; k_cache, v_cache:
  * fp16 [NKV, max_seq, hd]; out: fp16 [NQ, hd]; 1 <= cur_len <= max_seq,
  * NQ % NKV == 0. `scale` is the score multiplier (the binding passes
- * 1/sqrt(hd)). One launch: a short context is one workgroup per KV head; a
- * long one is split over the KV sequence and the last split of each KV head
- * combines the split states in a fixed order. The workspace
+ * 1/sqrt(hd)). A short context is one launch (a workgroup per query head); a
+ * long one is split over the KV sequence and a second launch combines the
+ * split states in a fixed order. The workspace
  * (soi_decode_attention_workspace_bytes, 16-byte aligned) holds the split
- * states and ends in arrival counters that must be zero before the first
- * call (e.g. zero-filled once); every call leaves them zero, so a workspace
- * is reused across calls and graph replays (calls that overlap on one
- * workspace race). Replaces launch_decode_attention
+ * states; this form reads nothing from it that it has not written. It ends in
+ * arrival counters for the device-position forms below, which need them zero
+ * before the first call (e.g. zero-filled once) and leave them zero, so a
+ * workspace is reused across calls and graph replays (calls that overlap on
+ * one workspace race). Replaces launch_decode_attention
  * (csrc/kernels/decode_attention.cu:57-63; binding csrc/bindings.cpp:468-488).
  * ------------------------------------------------------------------------ */
 size_t soi_decode_attention_workspace_bytes(int64_t NQ, int64_t NKV, int64_t head_dim, int64_t cur_len);

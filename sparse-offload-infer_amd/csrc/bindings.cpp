@@ -469,7 +469,9 @@ torch::Tensor decode_attention(torch::Tensor q, torch::Tensor k_cache, torch::Te
     auto out = torch::empty({NQ, hd}, q.options());
     const float scale = 1.0f / std::sqrt(static_cast<float>(hd));
     const size_t wsb = soi_decode_attention_workspace_bytes(NQ, NKV, hd, cur_len);
-    auto ws = zeroed_workspace(q, wsb);
+    // a host length combines its splits in a second launch, so no arrival counter is read: the workspace need not be
+    // cleared (the fill was a third of the call: 10.3 us at L = 1999, 16 / 8 heads of 128)
+    auto ws = torch::empty({static_cast<int64_t>(wsb > 0 ? wsb : 1)}, q.options().dtype(torch::kUInt8));
     check_status(soi_decode_attention(h16(q), h16(k_cache), h16(v_cache), h16m(out), NQ, NKV, S, hd, cur_len, scale,
                                       ws.data_ptr<uint8_t>(), wsb, cur_stream(q)),
                  "decode_attention");
