@@ -728,7 +728,7 @@ struct AttnLdsX {
     const uint16_t* s_x;
     const uint16_t* b;
     __device__ __forceinline__ const uint16_t* base() const { return b; }
-    template <bool VEC, bool FULL>
+    template <int VEC, bool FULL>
     __device__ __forceinline__ void load(int, int c, bool cv, f16x2 xv[16]) const {
         lds_x_chunk<FULL>(s_x, c, cv, xv);
     }
@@ -745,7 +745,7 @@ struct AttnOnePassX {
     int p;        // pos[0]
     u32x4 xc[4];  // x[32l .. 32l+31] of out
     __device__ __forceinline__ const uint16_t* base() const { return oa.attn_out; }
-    template <bool VEC, bool FULL>
+    template <int VEC, bool FULL>
     __device__ __forceinline__ void load(int K, int c, bool cv, f16x2 xv[16]) const {
         const int L = p < 0 ? 1 : (p >= oa.S ? oa.S : p + 1);  // cur_len_of
         const int ns = attn_splits(oa, L);

@@ -50,7 +50,7 @@ struct MissCopy {
     }
 };
 
-template <int R, int PU, bool VEC, bool CHUNK_SCALE, bool BITFIELD, bool FULL, class Rows, class EP, class CP>
+template <int R, int PU, int VEC, bool CHUNK_SCALE, bool BITFIELD, bool FULL, class Rows, class EP, class CP>
 __device__ __forceinline__ void gemv_int4_body(const Rows& rows, int64_t N, const uint16_t* __restrict__ x,
                                                const EP& ep, int K, int gs, const CP& cp) {
     const int64_t row0 = static_cast<int64_t>(blockIdx.x) * R;
@@ -101,7 +101,7 @@ __device__ __forceinline__ void gemv_int4_body(const Rows& rows, int64_t N, cons
 }
 
 // Single-pass tiles: the default register budget (occupancy-driven scheduling).
-template <int R, int PU, bool VEC, bool CHUNK_SCALE, bool BITFIELD, bool FULL, class Rows, class EP = StoreY,
+template <int R, int PU, int VEC, bool CHUNK_SCALE, bool BITFIELD, bool FULL, class Rows, class EP = StoreY,
           class CP = NoCopy>
 __global__ __launch_bounds__(64) void gemv_int4_kernel(Rows rows, int64_t N, const uint16_t* __restrict__ x, EP ep,
                                                        int K, int gs, CP cp = CP{}) {
@@ -112,7 +112,7 @@ __global__ __launch_bounds__(64) void gemv_int4_kernel(Rows rows, int64_t N, con
 // has about one wave per SIMD, so occupancy buys nothing, while every pass's loads must be in flight at once
 // (R*PU weight chunks + PU x chunks, ~90 VGPRs). With the default budget the scheduler kept 5 waves per SIMD by
 // reusing registers, which serialised the passes' loads into several round trips.
-template <int R, int PU, bool VEC, bool CHUNK_SCALE, bool BITFIELD, bool FULL, class Rows, class EP = StoreY,
+template <int R, int PU, int VEC, bool CHUNK_SCALE, bool BITFIELD, bool FULL, class Rows, class EP = StoreY,
           class CP = NoCopy>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(1, 4))) void gemv_int4_mp_kernel(
     Rows rows, int64_t N, const uint16_t* __restrict__ x, EP ep, int K, int gs, CP cp = CP{}) {
@@ -133,7 +133,7 @@ __device__ __forceinline__ void misaligned_rows_nan(uint16_t* y, int64_t N, int6
 // row tile b % tiles of problem b / tiles. Pointer tables live in device
 // memory; a problem with a null pointer writes nothing, a misaligned one NaN
 // rows (misaligned_rows_nan).
-template <int R, int PU, bool VEC, bool CHUNK_SCALE, bool FULL>
+template <int R, int PU, int VEC, bool CHUNK_SCALE, bool FULL>
 __device__ __forceinline__ void gemv_int4_batched_body(const uint8_t* const* __restrict__ Wp,
                                                        const float* const* __restrict__ Sp,
                                                        const uint16_t* const* __restrict__ Xp,
@@ -147,7 +147,7 @@ __device__ __forceinline__ void gemv_int4_batched_body(const uint8_t* const* __r
     uint16_t* y = ldg(Yp + p);
     if (!W || !S || !x || !y) return;
     const uintptr_t bad = reinterpret_cast<uintptr_t>(W) | reinterpret_cast<uintptr_t>(x);
-    if (VEC && (bad & 15u)) {
+    if (VEC == kAligned && (bad & 15u)) {
         misaligned_rows_nan<R>(y, N, static_cast<int64_t>(tile) * R);
         return;
     }
@@ -161,11 +161,11 @@ __device__ __forceinline__ void gemv_int4_batched_body(const uint8_t* const* __r
     const uint8_t* const* __restrict__ Wp, const float* const* __restrict__ Sp,                              \
         const uint16_t* const* __restrict__ Xp, uint16_t* const* __restrict__ Yp, int64_t N, int K, int gs, int G, \
         int tiles
-template <int R, int PU, bool VEC, bool CHUNK_SCALE, bool FULL>
+template <int R, int PU, int VEC, bool CHUNK_SCALE, bool FULL>
 __global__ __launch_bounds__(64) void gemv_int4_batched_kernel(SOI_BATCHED_PARAMS) {
     gemv_int4_batched_body<R, PU, VEC, CHUNK_SCALE, FULL>(Wp, Sp, Xp, Yp, N, K, gs, G, tiles);
 }
-template <int R, int PU, bool VEC, bool CHUNK_SCALE, bool FULL>
+template <int R, int PU, int VEC, bool CHUNK_SCALE, bool FULL>
 __global__ __launch_bounds__(64) SOI_GEMV_OCCUPANCY void gemv_int4_batched_occ_kernel(SOI_BATCHED_PARAMS) {
     gemv_int4_batched_body<R, PU, VEC, CHUNK_SCALE, FULL>(Wp, Sp, Xp, Yp, N, K, gs, G, tiles);
 }
@@ -266,7 +266,7 @@ struct GroupClasses {
     int G[kMaxClasses];
 };
 
-template <int R, bool VEC, bool CHUNK_SCALE, bool FULL>
+template <int R, int VEC, bool CHUNK_SCALE, bool FULL>
 __device__ __forceinline__ void gemv_int4_grouped_body(const uint8_t* const* __restrict__ Wp,
                                                        const float* const* __restrict__ Sp,
                                                        const uint16_t* const* __restrict__ Xp,
@@ -296,7 +296,7 @@ __device__ __forceinline__ void gemv_int4_grouped_body(const uint8_t* const* __r
     uint16_t* y = ldg(Yp + p);
     if (!W || !S || !x || !y) return;
     const uintptr_t bad = reinterpret_cast<uintptr_t>(W) | reinterpret_cast<uintptr_t>(x);
-    if (VEC && (bad & 15u)) {
+    if (VEC == kAligned && (bad & 15u)) {
         misaligned_rows_nan<R>(y, N, static_cast<int64_t>(tile) * R);
         return;
     }
@@ -309,11 +309,11 @@ __device__ __forceinline__ void gemv_int4_grouped_body(const uint8_t* const* __r
 #define SOI_GROUPED_PARAMS                                                                                   \
     const uint8_t* const* __restrict__ Wp, const float* const* __restrict__ Sp,                            \
         const uint16_t* const* __restrict__ Xp, uint16_t* const* __restrict__ Yp, GroupClasses cl, int gs
-template <int R, bool VEC, bool CHUNK_SCALE, bool FULL>
+template <int R, int VEC, bool CHUNK_SCALE, bool FULL>
 __global__ __launch_bounds__(64) void gemv_int4_grouped_kernel(SOI_GROUPED_PARAMS) {
     gemv_int4_grouped_body<R, VEC, CHUNK_SCALE, FULL>(Wp, Sp, Xp, Yp, cl, gs);
 }
-template <int R, bool VEC, bool CHUNK_SCALE, bool FULL>
+template <int R, int VEC, bool CHUNK_SCALE, bool FULL>
 __global__ __launch_bounds__(64) SOI_GEMV_OCCUPANCY void gemv_int4_grouped_occ_kernel(SOI_GROUPED_PARAMS) {
     gemv_int4_grouped_body<R, VEC, CHUNK_SCALE, FULL>(Wp, Sp, Xp, Yp, cl, gs);
 }
@@ -322,11 +322,11 @@ __global__ __launch_bounds__(64) SOI_GEMV_OCCUPANCY void gemv_int4_grouped_occ_k
 // The occupancy hint is applied where the tile fits its register budget
 // without spilling (checked on the compiler's output): vector loads, one
 // scale per chunk, and one pass per batch (or at most 4 row segments).
-constexpr bool occ_fits(int R, int PU, bool VEC, bool CS, bool FULL) {
-    return VEC && CS && (PU == 1 || (R * PU <= 4 && FULL));
+constexpr bool occ_fits(int R, int PU, int VEC, bool CS, bool FULL) {
+    return VEC == kAligned && CS && (PU == 1 || (R * PU <= 4 && FULL));
 }
 
-template <int R, int PU, bool V, bool CS, bool FL>
+template <int R, int PU, int V, bool CS, bool FL>
 static void launch_batched_kernel(dim3 grid, hipStream_t st, const uint8_t* const* Wp, const float* const* Sp,
                                   const uint16_t* const* Xp, uint16_t* const* Yp, int64_t N, int K, int gs, int G,
                                   int tiles) {
@@ -338,7 +338,7 @@ static void launch_batched_kernel(dim3 grid, hipStream_t st, const uint8_t* cons
                            gs, G, tiles);
 }
 
-template <int R, bool V, bool CS, bool FL>
+template <int R, int V, bool CS, bool FL>
 static void launch_grouped_kernel(dim3 grid, hipStream_t st, const uint8_t* const* Wp, const float* const* Sp,
                                   const uint16_t* const* Xp, uint16_t* const* Yp, const GroupClasses& cl, int gs) {
     if constexpr (occ_fits(R, 1, V, CS, FL))
@@ -356,23 +356,23 @@ struct Int4Plan {
     int R, PU;
 };
 
-// PU: passes per batch (all of them up to 4); R: rows per wave, 8 for a
+// PU: passes per batch (passes_per_batch; 2 where rows are read from any address, whose tiles are bound by their tail
+// handling, not by batches); R: rows per wave, 8 for a
 // one-pass tile over >= 4096 rows, else 2 from 2048 rows, else 1. Swept on
 // single cold launches of the Qwen3-1.7B shapes: 4-row tiles were slower than
 // both 8- and 2-row tiles at every shape (gate/up 6144x2048: 3.39 / 3.93 /
 // 3.53 us for 8 / 4 / 2 rows), and more than 8 row segments in flight per
 // wave did not pay.
-static Int4Plan plan_int4(int64_t N, int64_t K, bool vec) {
+static Int4Plan plan_int4(int64_t N, int64_t K, int vec) {
     const int64_t chunks = ceil_div64(ceil_div64(K, 8), 4);
     const int64_t passes = ceil_div64(chunks, kWave);
     Int4Plan p{1, 1};
-    p.PU = vec ? static_cast<int>(passes < 4 ? passes : 4) : 1;
-    if (p.PU == 3 && passes > 3) p.PU = 4;
+    p.PU = vec == kAligned ? passes_per_batch(passes) : vec == kAnyAlign && passes > 1 ? 2 : 1;
     p.R = (N >= 4 * 1024 && p.PU == 1) ? 8 : N >= 2 * 1024 ? 2 : 1;
     return p;
 }
 
-template <int RR, int PP, bool V, bool CS, bool BF, bool FL, class Rows, class EP, class CP>
+template <int RR, int PP, int V, bool CS, bool BF, bool FL, class Rows, class EP, class CP>
 static void launch_int4_kernel(dim3 grid, hipStream_t st, const Rows& rows, int64_t N, const uint16_t* x, const EP& ep,
                                int K, int gs, const CP& cp) {
     if constexpr (PP > 1)
@@ -384,44 +384,60 @@ static void launch_int4_kernel(dim3 grid, hipStream_t st, const Rows& rows, int6
 }
 
 template <bool BITFIELD, class Rows, class EP = StoreY, class CP = NoCopy>
-static int launch_int4(const Rows& rows, int64_t N, const uint16_t* x, const EP& ep, int64_t K, int64_t gs, bool vec,
+static int launch_int4(const Rows& rows, int64_t N, const uint16_t* x, const EP& ep, int64_t K, int64_t gs, bool aligned,
                        hipStream_t st, const char* what, const CP& cp = CP{}) {
     if (N == 0) return SOI_OK;
+    const int vec = aligned ? kAligned : K >= 32 ? kAnyAlign : kScalar;
     Int4Plan pl = plan_int4(N, K, vec);
-    // a multi-pass tile over more than 2048 rows: 4 rows per wave (2560 x 9728 7.7 against 8.1 us, 4096 x 12288
-    // 9.9 against 10.6 us back to back on cold copies; 2048 x 6144 stays at 2 rows, 3.8 against 4.0 us)
-    if (pl.PU > 1 && N > 2 * 1024) pl.R = 4;
+    // rows of more than 3 passes, over more than 2048 rows: 4 rows per wave (2560 x 9728 6.34 against 6.35 us with 2,
+    // 4096 x 12288 8.0 against 8.3, 5120 x 17408 14.5 against 14.9, 8192 x 8192 9.6 against 10.7, cold copies); rows of
+    // 2 or 3 passes stay at 2 (4096 x 4096 3.9 against 4.2 us with 4, 5120 x 5120 5.7 against 6.3, 2048 x 6144 3.8
+    // against 4.0)
+    const int64_t passes = ceil_div64(ceil_div64(ceil_div64(K, 8), 4), kWave);
+    if (pl.PU > 1 && N > 2 * 1024 && (passes > 3 || vec != kAligned)) pl.R = 4;
     const bool cs = (gs % 32) == 0;
-    const bool full = vec && cs && (N % pl.R == 0) && ((K / 32) % (64 * pl.PU) == 0);
+    const bool full = aligned && cs && (N % pl.R == 0) && ((K / 32) % (64 * pl.PU) == 0);
     const dim3 grid(static_cast<unsigned>(ceil_div64(N, pl.R)));
     const int Ki = static_cast<int>(K), gi = static_cast<int>(gs);
 #define SOI_L(RR, PP, V, CS, FL) \
     launch_int4_kernel<RR, PP, V, CS, BITFIELD, FL>(grid, st, rows, N, x, ep, Ki, gi, cp)
 #define SOI_CS(RR, PP, V)                    \
-    if (V && full) SOI_L(RR, PP, V, true, true); \
-    else if (cs) SOI_L(RR, PP, V, true, false);  \
+    if constexpr (V == kAligned) {                \
+        if (full) SOI_L(RR, PP, V, true, true);   \
+        else if (cs) SOI_L(RR, PP, V, true, false); \
+        else SOI_L(RR, PP, V, false, false);      \
+    } else if (cs) SOI_L(RR, PP, V, true, false); \
     else SOI_L(RR, PP, V, false, false)
     const int key = pl.R * 10 + pl.PU;
-    if (vec) {
+    if (vec == kAligned) {
         switch (key) {
-            case 81: SOI_CS(8, 1, true); break;
-            case 21: SOI_CS(2, 1, true); break;
-            case 11: SOI_CS(1, 1, true); break;
-            case 22: SOI_CS(2, 2, true); break;
-            case 12: SOI_CS(1, 2, true); break;
-            case 23: SOI_CS(2, 3, true); break;
-            case 13: SOI_CS(1, 3, true); break;
-            case 24: SOI_CS(2, 4, true); break;
-            case 42: SOI_CS(4, 2, true); break;
-            case 43: SOI_CS(4, 3, true); break;
-            case 44: SOI_CS(4, 4, true); break;
-            default: SOI_CS(1, 4, true); break;
+            case 81: SOI_CS(8, 1, kAligned); break;
+            case 21: SOI_CS(2, 1, kAligned); break;
+            case 11: SOI_CS(1, 1, kAligned); break;
+            case 22: SOI_CS(2, 2, kAligned); break;
+            case 12: SOI_CS(1, 2, kAligned); break;
+            case 23: SOI_CS(2, 3, kAligned); break;
+            case 13: SOI_CS(1, 3, kAligned); break;
+            case 24: SOI_CS(2, 4, kAligned); break;
+            case 42: SOI_CS(4, 2, kAligned); break;
+            case 43: SOI_CS(4, 3, kAligned); break;
+            case 44: SOI_CS(4, 4, kAligned); break;
+            default: SOI_CS(1, 4, kAligned); break;
+        }
+    } else if (vec == kAnyAlign) {
+        switch (key) {
+            case 81: SOI_CS(8, 1, kAnyAlign); break;
+            case 21: SOI_CS(2, 1, kAnyAlign); break;
+            case 11: SOI_CS(1, 1, kAnyAlign); break;
+            case 42: SOI_CS(4, 2, kAnyAlign); break;
+            case 22: SOI_CS(2, 2, kAnyAlign); break;
+            default: SOI_CS(1, 2, kAnyAlign); break;
         }
     } else {
         switch (pl.R) {
-            case 8: SOI_CS(8, 1, false); break;
-            case 2: SOI_CS(2, 1, false); break;
-            default: SOI_CS(1, 1, false); break;
+            case 8: SOI_CS(8, 1, kScalar); break;
+            case 2: SOI_CS(2, 1, kScalar); break;
+            default: SOI_CS(1, 1, kScalar); break;
         }
     }
 #undef SOI_CS
@@ -432,7 +448,8 @@ static int launch_int4(const Rows& rows, int64_t N, const uint16_t* x, const EP&
 static int launch_int4_batched(const uint8_t* const* Wp, const float* const* Sp, const uint16_t* const* Xp,
                                uint16_t* const* Yp, int64_t P, int64_t N, int64_t K, int64_t gs, int64_t G,
                                hipStream_t st, const char* what) {
-    const bool vec = (K % 32) == 0;
+    const bool aligned = (K % 32) == 0;
+    const int vec = aligned ? kAligned : K >= 32 ? kAnyAlign : kScalar;
     Int4Plan pl = plan_int4(N * P, K, vec);  // rows per wave chosen on the total row count
     if (P > 1) {  // throughput regime: one pass per batch, 8 rows per wave (measured best when streaming)
         pl.PU = 1;
@@ -441,32 +458,43 @@ static int launch_int4_batched(const uint8_t* const* Wp, const float* const* Sp,
     const int64_t tiles = ceil_div64(N, pl.R);
     SOI_REQUIRE(tiles * P <= (int64_t(1) << 31) - 1, "%s: too many row tiles", what);
     const bool cs = (gs % 32) == 0;
-    const bool full = vec && cs && (N % pl.R == 0) && ((K / 32) % (64 * pl.PU) == 0);
+    const bool full = aligned && cs && (N % pl.R == 0) && ((K / 32) % (64 * pl.PU) == 0);
     const dim3 grid(static_cast<unsigned>(tiles * P));
     const int Ki = static_cast<int>(K), gi = static_cast<int>(gs), Gi = static_cast<int>(G), ti = static_cast<int>(tiles);
 #define SOI_B(RR, PP, V, CS, FL) launch_batched_kernel<RR, PP, V, CS, FL>(grid, st, Wp, Sp, Xp, Yp, N, Ki, gi, Gi, ti)
 #define SOI_BCS(RR, PP, V)                        \
-    if (V && full) SOI_B(RR, PP, V, true, true);  \
-    else if (cs) SOI_B(RR, PP, V, true, false);   \
+    if constexpr (V == kAligned) {                \
+        if (full) SOI_B(RR, PP, V, true, true);   \
+        else if (cs) SOI_B(RR, PP, V, true, false); \
+        else SOI_B(RR, PP, V, false, false);      \
+    } else if (cs) SOI_B(RR, PP, V, true, false); \
     else SOI_B(RR, PP, V, false, false)
     const int key = pl.R * 10 + pl.PU;
-    if (vec) {
+    if (vec == kAligned) {
         switch (key) {
-            case 81: SOI_BCS(8, 1, true); break;
-            case 21: SOI_BCS(2, 1, true); break;
-            case 11: SOI_BCS(1, 1, true); break;
-            case 22: SOI_BCS(2, 2, true); break;
-            case 12: SOI_BCS(1, 2, true); break;
-            case 23: SOI_BCS(2, 3, true); break;
-            case 13: SOI_BCS(1, 3, true); break;
-            case 24: SOI_BCS(2, 4, true); break;
-            default: SOI_BCS(1, 4, true); break;
+            case 81: SOI_BCS(8, 1, kAligned); break;
+            case 21: SOI_BCS(2, 1, kAligned); break;
+            case 11: SOI_BCS(1, 1, kAligned); break;
+            case 22: SOI_BCS(2, 2, kAligned); break;
+            case 12: SOI_BCS(1, 2, kAligned); break;
+            case 23: SOI_BCS(2, 3, kAligned); break;
+            case 13: SOI_BCS(1, 3, kAligned); break;
+            case 24: SOI_BCS(2, 4, kAligned); break;
+            default: SOI_BCS(1, 4, kAligned); break;
+        }
+    } else if (vec == kAnyAlign) {
+        switch (key) {
+            case 81: SOI_BCS(8, 1, kAnyAlign); break;
+            case 21: SOI_BCS(2, 1, kAnyAlign); break;
+            case 11: SOI_BCS(1, 1, kAnyAlign); break;
+            case 22: SOI_BCS(2, 2, kAnyAlign); break;
+            default: SOI_BCS(1, 2, kAnyAlign); break;
         }
     } else {
         switch (pl.R) {
-            case 8: SOI_BCS(8, 1, false); break;
-            case 2: SOI_BCS(2, 1, false); break;
-            default: SOI_BCS(1, 1, false); break;
+            case 8: SOI_BCS(8, 1, kScalar); break;
+            case 2: SOI_BCS(2, 1, kScalar); break;
+            default: SOI_BCS(1, 1, kScalar); break;
         }
     }
 #undef SOI_BCS
@@ -590,7 +618,7 @@ extern "C" int soi_gemv_w4a16_grouped(const uint8_t* const* Wq_ptrs, const float
     constexpr int R = 8;
     GroupClasses cl{};
     int64_t wg = 0, problems = 0;
-    bool vec = true, full = (group_size % 32) == 0;
+    bool vec = true, whole = true, full = (group_size % 32) == 0;  // whole: every row has a whole 32-element chunk
     int n = 0;
     for (int64_t c = 0; c < num_classes; ++c) {
         const int64_t P = class_count[c], N = class_N[c], K = class_K[c];
@@ -609,6 +637,7 @@ extern "C" int soi_gemv_w4a16_grouped(const uint8_t* const* Wq_ptrs, const float
         cl.K[n] = static_cast<int>(K);
         cl.G[n] = static_cast<int>(ceil_div64(K, group_size));
         vec = vec && (K % 32) == 0;
+        whole = whole && K >= 32;
         full = full && (N % R) == 0 && ((K / 32) % 64) == 0;
         wg += tiles * P;
         problems += P;
@@ -625,11 +654,13 @@ extern "C" int soi_gemv_w4a16_grouped(const uint8_t* const* Wq_ptrs, const float
     const bool cs = (group_size % 32) == 0;
     hipStream_t st = as_stream(stream);
 #define SOI_G(V, CS, FL) launch_grouped_kernel<R, V, CS, FL>(grid, st, Wq_ptrs, scale_ptrs, x_ptrs, y_ptrs, cl, gi)
-    if (full) SOI_G(true, true, true);
-    else if (vec && cs) SOI_G(true, true, false);
-    else if (vec) SOI_G(true, false, false);
-    else if (cs) SOI_G(false, true, false);
-    else SOI_G(false, false, false);
+    if (full) SOI_G(kAligned, true, true);
+    else if (vec && cs) SOI_G(kAligned, true, false);
+    else if (vec) SOI_G(kAligned, false, false);
+    else if (whole && cs) SOI_G(kAnyAlign, true, false);
+    else if (whole) SOI_G(kAnyAlign, false, false);
+    else if (cs) SOI_G(kScalar, true, false);
+    else SOI_G(kScalar, false, false);
 #undef SOI_G
     return launch_status(what);
 }

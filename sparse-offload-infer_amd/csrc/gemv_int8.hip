@@ -7,9 +7,13 @@
 // One wave per workgroup, R rows per wave, PU 64-chunk passes per batch.
 // Lane l owns 16-byte chunk l of each pass (16 consecutive k), so a wave-wide
 // dwordx4 load reads 1 KB of a row; R*PU such loads are issued before any
-// arithmetic. Loads are unconditional: a lane past the last chunk (or any
-// byte past K) reads the zero word instead (address select, no branch), and
-// row addresses are wave-uniform (scalar registers). Bytes become exact
+// arithmetic. Loads are unconditional: a lane past the last chunk reads the
+// zero word instead (address select, no branch), and row addresses are
+// wave-uniform (scalar registers). Rows of any length and alignment are read
+// the same way (kAnyAlign, soi_int4_tile.h): the load of a row's last, shorter
+// chunk is moved back to end with the row and its bytes are moved down in
+// registers (byte by byte, 4096 x 4100 took 32.8 us and 512 x 16163 24.5 us);
+// only rows under 16 bytes are read by bytes. Bytes become exact
 // binary16 integers (soi_device.h), pairs are accumulated with an ordered
 // v_dot2 chain, the scale is applied once per chunk (per word when 16 does
 // not divide group_size), and the R row totals come out of one transposed
@@ -20,12 +24,13 @@
 // then, which reads past a [N,1] scale when the caller passes gs < K.
 #include "soi_device.h"
 #include "soi_host.h"
+#include "soi_int4_tile.h"
 
 namespace soi {
 
 // Rows row0 .. row0 + R - 1 of one problem, by the calling wave (the single and batched kernels share it, so a
 // batched problem's y is bit-identical to the single launch's).
-template <int R, int PU, bool VEC, bool CHUNK_SCALE, bool FULL>
+template <int R, int PU, int VEC, bool CHUNK_SCALE, bool FULL>
 __device__ __forceinline__ void gemv_int8_rows(const int8_t* __restrict__ W, const float* __restrict__ S,
                                                int64_t srow_stride, int64_t N, const uint16_t* __restrict__ x,
                                                uint16_t* __restrict__ y, int K, int gs, int G, int64_t row0) {
@@ -48,6 +53,12 @@ __device__ __forceinline__ void gemv_int8_rows(const int8_t* __restrict__ W, con
     float acc[R];
 #pragma unroll
     for (int r = 0; r < R; ++r) acc[r] = 0.0f;
+    uint32_t x_tail = 0;  // x's last chunk when it is not whole: lane e < 8 holds its pair e, zeros past K
+    if constexpr (VEC == kAnyAlign) {
+        const uint16_t* zh = reinterpret_cast<const uint16_t*>(zw);
+        const int ka = 16 * (chunks - 1) + 2 * lane;
+        x_tail = ldg(ka < K ? x + ka : zh) | (static_cast<uint32_t>(ldg(ka + 1 < K ? x + ka + 1 : zh)) << 16);
+    }
 
     for (int c0 = 0; c0 < chunks; c0 += kWave * PU) {
         uint32_t wv[PU][R][4];
@@ -60,15 +71,22 @@ __device__ __forceinline__ void gemv_int8_rows(const int8_t* __restrict__ W, con
             const int k0 = 16 * c;
 #pragma unroll
             for (int r = 0; r < R; ++r) {
-                if (VEC) {
+                if (VEC == kAligned) {
                     const u32x4* q = reinterpret_cast<const u32x4*>(wr[r]) + c;
                     const u32x4 t = ldg_stream(cv ? q : reinterpret_cast<const u32x4*>(zw));
                     wv[p][r][0] = t.x;
                     wv[p][r][1] = t.y;
                     wv[p][r][2] = t.z;
                     wv[p][r][3] = t.w;
+                } else if (VEC == kAnyAlign) {
+                    const u32x4 t = ldg_any(cv ? wr[r] + (k0 + 16 > K ? K - 16 : k0)
+                                               : reinterpret_cast<const uint8_t*>(zw));
+                    wv[p][r][0] = t.x;
+                    wv[p][r][1] = t.y;
+                    wv[p][r][2] = t.z;
+                    wv[p][r][3] = t.w;
                 } else {
-                    // ragged K: bytes past K read as 0x00 -> value 0 (x there is 0 too)
+                    // bytes past K read as 0x00 -> value 0 (x there is 0 too)
                     const uint8_t* zb = reinterpret_cast<const uint8_t*>(zw);
 #pragma unroll
                     for (int i = 0; i < 4; ++i) {
@@ -91,10 +109,13 @@ __device__ __forceinline__ void gemv_int8_rows(const int8_t* __restrict__ W, con
                     }
                 }
             }
-            if (VEC) {  // K % 16 == 0: a valid chunk is fully inside x
+            if (VEC != kScalar) {  // a valid chunk is fully inside x, or (kAnyAlign) the tail, filled in below
                 const u32x4* xp = reinterpret_cast<const u32x4*>(x + k0);
                 const u32x4* z4 = reinterpret_cast<const u32x4*>(zw);
-                const u32x4 a = ldg(cv ? xp : z4), b = ldg(cv ? xp + 1 : z4);
+                const bool xw = VEC == kAligned ? cv : cv && k0 + 16 <= K;
+                const u32x4* pa = xw ? xp : z4;
+                const u32x4* pb = xw ? xp + 1 : z4;
+                const u32x4 a = VEC == kAligned ? ldg(pa) : ldg_any(pa), b = VEC == kAligned ? ldg(pb) : ldg_any(pb);
                 xv[p][0] = as_f16x2(a.x);
                 xv[p][1] = as_f16x2(a.y);
                 xv[p][2] = as_f16x2(a.z);
@@ -111,6 +132,31 @@ __device__ __forceinline__ void gemv_int8_rows(const int8_t* __restrict__ W, con
                     const uint32_t lo = ldg((cv && ka < K) ? x + ka : zh);
                     const uint32_t hi = ldg((cv && kb < K) ? x + kb : zh);
                     xv[p][e] = as_f16x2(lo | (hi << 16));
+                }
+            }
+        }
+        if constexpr (VEC == kAnyAlign) {
+            // (after every load is issued: branches between them would wait for each)
+            __builtin_amdgcn_sched_barrier(0);
+            if ((K & 15) && c0 + kWave * PU >= chunks) {  // wave-uniform: this batch holds the last chunk
+                // its bytes are the load's last K % 16: down by the rest, words first
+                const int by = 16 - (K & 15);
+#pragma unroll
+                for (int p = 0; p < PU; ++p) {
+                    const bool tail = c0 + p * kWave + lane == chunks - 1;
+                    spread_x_tail<8>(x_tail, tail, xv[p]);
+#pragma unroll
+                    for (int r = 0; r < R; ++r) {
+                        if (by >> 2) shift_w_tail(wv[p][r], tail, 4 - (by >> 2));
+                        if (by & 3) {
+                            uint32_t* w = wv[p][r];
+#pragma unroll
+                            for (int i = 0; i < 4; ++i) {
+                                const uint32_t up = i < 3 ? w[i + 1] : 0u;
+                                w[i] = tail ? __builtin_amdgcn_alignbyte(up, w[i], by & 3) : w[i];
+                            }
+                        }
+                    }
                 }
             }
         }
@@ -147,7 +193,7 @@ __device__ __forceinline__ void gemv_int8_rows(const int8_t* __restrict__ W, con
     if ((lane & (64 / R - 1)) == 0 && (FULL || row0 + r < N)) stg(y + row0 + r, f32_to_f16_bits(total));
 }
 
-template <int R, int PU, bool VEC, bool CHUNK_SCALE, bool FULL>
+template <int R, int PU, int VEC, bool CHUNK_SCALE, bool FULL>
 __global__ __launch_bounds__(64) void gemv_int8_kernel(const int8_t* __restrict__ W, const float* __restrict__ S,
                                                        int64_t srow_stride, int64_t N, const uint16_t* __restrict__ x,
                                                        uint16_t* __restrict__ y, int K, int gs, int G) {
@@ -158,7 +204,7 @@ __global__ __launch_bounds__(64) void gemv_int8_kernel(const int8_t* __restrict_
 // Batched form: P problems of one shape; workgroup b takes row tile b % tiles of problem b / tiles. The pointer
 // tables live in device memory; a problem with a null pointer writes nothing, and (VEC) one whose W or x is not
 // 16-byte aligned gets NaN rows instead of being read with dwordx4 loads.
-template <int R, int PU, bool VEC, bool CHUNK_SCALE, bool FULL>
+template <int R, int PU, int VEC, bool CHUNK_SCALE, bool FULL>
 __global__ __launch_bounds__(64) void gemv_int8_batched_kernel(const int8_t* const* __restrict__ Wp,
                                                                const float* const* __restrict__ Sp,
                                                                const uint16_t* const* __restrict__ Xp,
@@ -172,7 +218,7 @@ __global__ __launch_bounds__(64) void gemv_int8_batched_kernel(const int8_t* con
     const uint16_t* x = ldg(Xp + p);
     uint16_t* y = ldg(Yp + p);
     if (!W || !S || !x || !y) return;
-    if (VEC && ((reinterpret_cast<uintptr_t>(W) | reinterpret_cast<uintptr_t>(x)) & 15u)) {
+    if (VEC == kAligned && ((reinterpret_cast<uintptr_t>(W) | reinterpret_cast<uintptr_t>(x)) & 15u)) {
         const int64_t r = row0 + static_cast<int64_t>(threadIdx.x);
         if (threadIdx.x < R && r < N) stg(y + r, static_cast<uint16_t>(0x7e00u));
         return;
@@ -184,19 +230,22 @@ struct Int8Plan {
     int R, PU;
 };
 
-// PU: passes per batch, the largest of 4, 3, 2 that divides the pass count
-// (all of them when there are fewer than 4); R: the most rows per wave with
+// PU: passes per batch: over 2048 rows up, the most that leave the fewest empty
+// passes (17408 x 5120, 5 passes, 24.6 us in batches of 4 and 20.5 in batches of
+// 3; 4096 x 10240, 10 passes, 11.5 of 4 and 10.5 of 2), below that the fewest
+// batches (256 x 10240 5.1 us in batches of 2, 4.4 of 4); R: the most rows per wave with
 // R*PU <= 8 1 KB row segments in flight that still leaves >= 2048 waves in the
 // grid (swept on the Qwen3-1.7B shapes: more waves beat more rows per wave).
-static Int8Plan plan_int8(int64_t N, int64_t K, bool vec) {
+static Int8Plan plan_int8(int64_t N, int64_t K, int vec) {
     const int64_t passes = ceil_div64(ceil_div64(K, 16), kWave);
     Int8Plan p{1, 1};
-    if (vec) {
-        if (passes <= 4) p.PU = static_cast<int>(passes);
-        else if (passes % 4 == 0) p.PU = 4;
-        else if (passes % 3 == 0) p.PU = 3;
-        else if (passes % 2 == 0) p.PU = 2;
-        else p.PU = 4;
+    if (vec != kScalar) {
+        p.PU = passes_per_batch(passes);
+        if (N >= 2048) {  // enough waves to hide a round trip: the fewest empty passes, then the longest batches
+            p.PU = static_cast<int>(passes < 4 ? passes : 4);
+            for (int u = p.PU - 1; u >= 2; --u)
+                if (ceil_div64(passes, u) * u < ceil_div64(passes, p.PU) * p.PU) p.PU = u;
+        }
     }
     int R = 8;
     while (R > 1 && (R * p.PU > 8 || N / R < 2048)) R >>= 1;
@@ -226,34 +275,42 @@ static int check_int8(int64_t N, int64_t K, int64_t group_size, int64_t num_grou
 // Picks the instantiation (R, PU, VEC, CHUNK_SCALE, FULL) of the plan and calls launch.go<...>() with it; the
 // launcher (SingleInt8Launch or BatchedInt8Launch) holds the arguments of its kernel form.
 template <class Launch>
-static void dispatch_int8(const Int8Plan& pl, bool vec, bool full, bool chunk_scale, Launch&& launch) {
+static void dispatch_int8(const Int8Plan& pl, int vec, bool full, bool chunk_scale, Launch&& launch) {
 #define SOI_L(RR, PP, V, CS, FL) launch.template go<RR, PP, V, CS, FL>()
 #define SOI_CS(RR, PP, V)                                     \
-    if (V && full && chunk_scale) SOI_L(RR, PP, V, true, true); \
-    else if (chunk_scale) SOI_L(RR, PP, V, true, false);        \
+    if constexpr (V == kAligned) {                               \
+        if (full && chunk_scale) SOI_L(RR, PP, V, true, true);   \
+        else if (chunk_scale) SOI_L(RR, PP, V, true, false);     \
+        else SOI_L(RR, PP, V, false, false);                     \
+    } else if (chunk_scale) SOI_L(RR, PP, V, true, false);       \
     else SOI_L(RR, PP, V, false, false)
-    if (vec) {
-        switch (pl.R * 10 + pl.PU) {
-            case 81: SOI_CS(8, 1, true); break;
-            case 41: SOI_CS(4, 1, true); break;
-            case 21: SOI_CS(2, 1, true); break;
-            case 11: SOI_CS(1, 1, true); break;
-            case 42: SOI_CS(4, 2, true); break;
-            case 22: SOI_CS(2, 2, true); break;
-            case 12: SOI_CS(1, 2, true); break;
-            case 23: SOI_CS(2, 3, true); break;
-            case 13: SOI_CS(1, 3, true); break;
-            case 24: SOI_CS(2, 4, true); break;
-            default: SOI_CS(1, 4, true); break;
-        }
+#define SOI_VEC(V)                                   \
+    switch (pl.R * 10 + pl.PU) {                     \
+        case 81: SOI_CS(8, 1, V); break;             \
+        case 41: SOI_CS(4, 1, V); break;             \
+        case 21: SOI_CS(2, 1, V); break;             \
+        case 11: SOI_CS(1, 1, V); break;             \
+        case 42: SOI_CS(4, 2, V); break;             \
+        case 22: SOI_CS(2, 2, V); break;             \
+        case 12: SOI_CS(1, 2, V); break;             \
+        case 23: SOI_CS(2, 3, V); break;             \
+        case 13: SOI_CS(1, 3, V); break;             \
+        case 24: SOI_CS(2, 4, V); break;             \
+        default: SOI_CS(1, 4, V); break;             \
+    }
+    if (vec == kAligned) {
+        SOI_VEC(kAligned)
+    } else if (vec == kAnyAlign) {
+        SOI_VEC(kAnyAlign)
     } else {
         switch (pl.R) {
-            case 8: SOI_CS(8, 1, false); break;
-            case 4: SOI_CS(4, 1, false); break;
-            case 2: SOI_CS(2, 1, false); break;
-            default: SOI_CS(1, 1, false); break;
+            case 8: SOI_CS(8, 1, kScalar); break;
+            case 4: SOI_CS(4, 1, kScalar); break;
+            case 2: SOI_CS(2, 1, kScalar); break;
+            default: SOI_CS(1, 1, kScalar); break;
         }
     }
+#undef SOI_VEC
 #undef SOI_CS
 #undef SOI_L
 }
@@ -267,7 +324,7 @@ struct SingleInt8Launch {
     const uint16_t* x;
     uint16_t* y;
     int K, gs, G;
-    template <int R, int PU, bool V, bool CS, bool FL>
+    template <int R, int PU, int V, bool CS, bool FL>
     void go() const {
         hipLaunchKernelGGL((gemv_int8_kernel<R, PU, V, CS, FL>), grid, dim3(64), 0, st, W, S, stride, N, x, y, K, gs,
                            G);
@@ -283,7 +340,7 @@ struct BatchedInt8Launch {
     uint16_t* const* Yp;
     int64_t stride, N;
     int K, gs, G;
-    template <int R, int PU, bool V, bool CS, bool FL>
+    template <int R, int PU, int V, bool CS, bool FL>
     void go() const {
         const int tiles = static_cast<int>(ceil_div64(N, R));
         const dim3 grid(static_cast<unsigned>(P * tiles));
@@ -300,10 +357,10 @@ extern "C" int soi_gemv_w8a16(const int8_t* Wq, const float* scale, const uint16
     if (s) return s;
     if (N == 0) return SOI_OK;
     SOI_REQUIRE(Wq && scale && x && y, "%s: null pointer", what);
-    const bool vec = (K % 16 == 0) && aligned16(Wq) && aligned16(x);
+    const int vec = (K % 16 == 0) && aligned16(Wq) && aligned16(x) ? kAligned : K >= 16 ? kAnyAlign : kScalar;
     const bool chunk_scale = (num_groups == 1) || (group_size % 16 == 0);
     const Int8Plan pl = plan_int8(N, K, vec);
-    const bool full = vec && (N % pl.R == 0) && ((K / 16) % (kWave * pl.PU) == 0);
+    const bool full = vec == kAligned && (N % pl.R == 0) && ((K / 16) % (kWave * pl.PU) == 0);
     SingleInt8Launch L{dim3(static_cast<unsigned>(ceil_div64(N, pl.R))), as_stream(stream), Wq, scale,
                        scale_row_stride, N, x, y, static_cast<int>(K), static_cast<int>(group_size),
                        static_cast<int>(num_groups)};
@@ -322,7 +379,7 @@ extern "C" int soi_gemv_w8a16_batched(const int8_t* const* Wq_ptrs, const float*
     if (N == 0 || P == 0) return SOI_OK;
     SOI_REQUIRE(Wq_ptrs && scale_ptrs && x_ptrs && y_ptrs, "%s: null pointer table", what);
     // the single form's passes per batch for this shape (with aligned operands)
-    const bool vec = K % 16 == 0;
+    const int vec = K % 16 == 0 ? kAligned : K >= 16 ? kAnyAlign : kScalar;
     const bool chunk_scale = (num_groups == 1) || (group_size % 16 == 0);
     Int8Plan pl = plan_int8(N, K, vec);
     // several problems fill the grid whatever the tile, so the tile takes the most rows its pass count allows
@@ -333,7 +390,7 @@ extern "C" int soi_gemv_w8a16_batched(const int8_t* const* Wq_ptrs, const float*
         const int rmax = pl.PU == 1 ? 8 : pl.PU == 2 ? 4 : 2;
         while (pl.R < rmax && N % (2 * pl.R) == 0) pl.R *= 2;
     }
-    const bool full = vec && (N % pl.R == 0) && ((K / 16) % (kWave * pl.PU) == 0);
+    const bool full = vec == kAligned && (N % pl.R == 0) && ((K / 16) % (kWave * pl.PU) == 0);
     SOI_REQUIRE(P * ceil_div64(N, pl.R) <= (int64_t(1) << 31) - 1, "%s: grid too large", what);
     BatchedInt8Launch L{P, as_stream(stream), Wq_ptrs, scale_ptrs, x_ptrs, y_ptrs, scale_row_stride, N,
                         static_cast<int>(K), static_cast<int>(group_size), static_cast<int>(num_groups)};

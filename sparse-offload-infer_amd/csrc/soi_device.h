@@ -53,6 +53,13 @@ __device__ __forceinline__ T ldg_stream(const T* p) {
     return __builtin_nontemporal_load((gT*)(p));
 }
 
+// 16 bytes from any address (global memory takes unaligned dwordx4 loads: one instruction, a second line at most).
+typedef uint32_t u32x4_any __attribute__((ext_vector_type(4), aligned(1)));
+__device__ __forceinline__ u32x4 ldg_any(const void* p) {
+    typedef const __attribute__((address_space(1))) u32x4_any gT;
+    return *(gT*)(p);
+}
+
 // A pointer known to be the same in every lane, moved to scalar registers.
 template <class T>
 __device__ __forceinline__ T* uniform_ptr(T* p) {

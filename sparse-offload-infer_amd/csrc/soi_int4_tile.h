@@ -29,14 +29,28 @@ constexpr float kTwo20 = 1048576.0f;
 // or row with nothing to read loads from g_zero16 instead (address select, no
 // branch), contributing exact zeros.
 
-template <bool VEC, bool FULL>
+// How a tile reads rows and x (VEC below): kScalar, word by word (rows of less than one 32-element chunk); kAligned,
+// 16-byte loads (K % 32 == 0 and 16-byte aligned rows and x); kAnyAlign, the same loads from any address, for every
+// other K and alignment. There the last chunk of a row holds `words % 4` words: its load is moved back to end with the
+// row (never past it, so nothing beyond the matrix is touched) and the words are moved down in registers; what is left
+// above them meets zeros of x. (Read word by word, 512 x 16163 took 19.1 us and 4096 x 4100 10.7 us.)
+constexpr int kScalar = 0, kAligned = 1, kAnyAlign = 2;
+
+template <int VEC, bool FULL>
 __device__ __forceinline__ void load_w_chunk(const uint8_t* __restrict__ row, bool ok, int words, int c,
                                              uint32_t wv[4]) {
     const uint32_t* z = g_zero16;
-    if (VEC) {
+    if (VEC == kAligned) {
         const u32x4* p = reinterpret_cast<const u32x4*>(row) + c;
         if (!FULL) p = ok ? p : reinterpret_cast<const u32x4*>(z);
         const u32x4 t = ldg_stream(p);  // weights are read once: non-temporal
+        wv[0] = t.x;
+        wv[1] = t.y;
+        wv[2] = t.z;
+        wv[3] = t.w;
+    } else if (VEC == kAnyAlign) {
+        const u32x4 t = ldg_any(ok ? row + 4 * static_cast<int64_t>(4 * c + 4 > words ? words - 4 : 4 * c)
+                                   : reinterpret_cast<const uint8_t*>(z));
         wv[0] = t.x;
         wv[1] = t.y;
         wv[2] = t.z;
@@ -51,15 +65,50 @@ __device__ __forceinline__ void load_w_chunk(const uint8_t* __restrict__ row, bo
     }
 }
 
-template <bool VEC, bool FULL>
+// x's last chunk when it is not whole (K % 32 != 0): lane e < 16 holds its pair e, zeros past K.
+__device__ __forceinline__ uint32_t load_x_tail(const uint16_t* __restrict__ x, int K, int chunks) {
+    const uint16_t* z = reinterpret_cast<const uint16_t*>(g_zero16);
+    const int ka = 32 * (chunks - 1) + 2 * static_cast<int>(threadIdx.x & 63);
+    const uint32_t lo = ldg(ka < K ? x + ka : z), hi = ldg(ka + 1 < K ? x + ka + 1 : z);
+    return lo | (hi << 16);
+}
+
+// A last chunk of `have` < 4 words, loaded with its row's end (moved back): its words down to the front in the lane that
+// holds it. After every row's load is issued: branches (wave-uniform) between the loads would wait for each.
+__device__ __forceinline__ void shift_w_tail(uint32_t wv[4], bool tail, int have) {
+    const int by = 4 - have;
+    if (by & 1) {
+        wv[0] = tail ? wv[1] : wv[0];
+        wv[1] = tail ? wv[2] : wv[1];
+        wv[2] = tail ? wv[3] : wv[2];
+    }
+    if (by & 2) {
+        wv[0] = tail ? wv[2] : wv[0];
+        wv[1] = tail ? wv[3] : wv[1];
+    }
+}
+
+// The tail's PAIRS pairs into every lane that wants them.
+template <int PAIRS>
+__device__ __forceinline__ void spread_x_tail(uint32_t tail, bool want, f16x2 (&xv)[PAIRS]) {
+#pragma unroll
+    for (int e = 0; e < PAIRS; ++e) {
+        const uint32_t t = static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(tail), e));
+        xv[e] = want ? as_f16x2(t) : xv[e];
+    }
+}
+
+template <int VEC, bool FULL>
 __device__ __forceinline__ void load_x_chunk(const uint16_t* __restrict__ x, int K, int c, bool cv, f16x2 xv[16]) {
     const int k0 = 32 * c;
-    if (VEC) {  // K % 32 == 0: a valid chunk is fully inside x
+    if (VEC != kScalar) {  // a valid chunk is fully inside x, or (kAnyAlign) the tail: zeros here, spread_x_tail later
         const u32x4* z = reinterpret_cast<const u32x4*>(g_zero16);
         const u32x4* xp = reinterpret_cast<const u32x4*>(x + k0);
+        if (VEC == kAnyAlign) cv = cv && k0 + 32 <= K;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-            const u32x4 t = ldg(FULL ? xp + i : (cv ? xp + i : z));
+            const u32x4* p = FULL ? xp + i : (cv ? xp + i : z);
+            const u32x4 t = VEC == kAligned ? ldg(p) : ldg_any(p);
             xv[4 * i + 0] = as_f16x2(t.x);
             xv[4 * i + 1] = as_f16x2(t.y);
             xv[4 * i + 2] = as_f16x2(t.z);
@@ -87,7 +136,7 @@ struct PlainX {
     static constexpr bool kSinglePass = false;
     const uint16_t* x;
     __device__ __forceinline__ const uint16_t* base() const { return x; }
-    template <bool VEC, bool FULL>
+    template <int VEC, bool FULL>
     __device__ __forceinline__ void load(int K, int c, bool cv, f16x2 xv[16]) const {
         load_x_chunk<VEC, FULL>(x, K, c, cv, xv);
     }
@@ -100,7 +149,7 @@ struct NormX {
     const uint16_t* w;
     float inv;
     __device__ __forceinline__ const uint16_t* base() const { return a; }
-    template <bool VEC, bool FULL>
+    template <int VEC, bool FULL>
     __device__ __forceinline__ void load(int, int c, bool cv, f16x2 xv[16]) const {
         const u32x4* z = reinterpret_cast<const u32x4*>(g_zero16);
         const u32x4* a4 = reinterpret_cast<const u32x4*>(a) + 4 * c;
@@ -147,7 +196,7 @@ struct RegNormX {
     uint16_t* h_out;
     const uint16_t* b;  // a K-element vector for unresolvable rows
     __device__ __forceinline__ const uint16_t* base() const { return b; }
-    template <bool VEC, bool FULL>
+    template <int VEC, bool FULL>
     __device__ __forceinline__ void load(int, int, bool, f16x2 xv[16]) const {
         const int lane = threadIdx.x & (kWave - 1);
         u32x4 s[4];
@@ -299,6 +348,14 @@ struct SplitGUY {
     }
 };
 
+// Passes per batch of a row of `passes` 64-chunk passes: at most 4, the fewest batches (each is a memory round trip), and
+// among those the fewest empty passes in the last one (an empty pass costs its loads: INT4 2560 x 9728, 5 passes, 7.5 us
+// in batches of 4 and 6.4 in batches of 3; 5120 x 17408, 9 passes, 17.8 and 14.6).
+inline int passes_per_batch(int64_t passes) {
+    const int64_t batches = (passes + 3) / 4;
+    return static_cast<int>((passes + batches - 1) / batches);
+}
+
 // Rows per wave of the RMSNorm-fused GEMV, and whether it takes the one-pass form of the norm (RegNormX). Larger
 // tiles than the plain GEMV's pay there, as each wave normalises the whole vector before its rows (swept at K =
 // 2048: N = 4096 / 6144 / 2048 best at 8 / 8 / 4 rows per wave). The SwiGLU forms always run 8-row tiles.
@@ -315,7 +372,7 @@ inline bool norm_gemv_one_pass(int64_t N, int64_t K, int64_t gs, bool swiglu) {
 
 // R rows per wave; PU passes (64 chunks each) loaded per batch, so a wave has
 // R*PU 1 KB row segments in flight before it does any arithmetic.
-template <int R, int PU, bool VEC, bool CHUNK_SCALE, bool BITFIELD, bool FULL, class Rows, class XS, class EP>
+template <int R, int PU, int VEC, bool CHUNK_SCALE, bool BITFIELD, bool FULL, class Rows, class XS, class EP>
 __device__ __forceinline__ void gemv_int4_tile(const Rows& rows, int64_t N, const XS& xsrc, const EP& ep, int K,
                                                int gs, int64_t row0) {
     constexpr int SC = CHUNK_SCALE ? 1 : 4;
@@ -362,6 +419,9 @@ __device__ __forceinline__ void gemv_int4_tile(const Rows& rows, int64_t N, cons
 #pragma unroll
     for (int r = 0; r < R; ++r) acc[r] = 0.0f;
 
+    uint32_t x_tail = 0;
+    if constexpr (VEC == kAnyAlign) x_tail = load_x_tail(xsrc.base(), K, chunks);
+
     const int c_end = XS::kSinglePass ? kWave * PU : chunks;  // single pass: no loop for the compiler to keep
     for (int c0 = 0; c0 < c_end; c0 += kWave * PU) {
         uint32_t wv[PU][R][4];
@@ -390,6 +450,20 @@ __device__ __forceinline__ void gemv_int4_tile(const Rows& rows, int64_t N, cons
             // a single-pass x source computes x from registers: keep that work after the weight loads
             if constexpr (XS::kSinglePass) __builtin_amdgcn_sched_barrier(0);
             xsrc.template load<VEC, FULL>(K, c, cv, xv[p]);
+        }
+        if constexpr (VEC == kAnyAlign) {
+            __builtin_amdgcn_sched_barrier(0);
+            if ((K & 31) && c0 + kWave * PU >= chunks) {  // wave-uniform: this batch holds the last chunk
+#pragma unroll
+                for (int p = 0; p < PU; ++p) {
+                    const bool tail = c0 + p * kWave + lane == chunks - 1;
+                    spread_x_tail<16>(x_tail, tail, xv[p]);
+                    if (words & 3) {
+#pragma unroll
+                        for (int r = 0; r < R; ++r) shift_w_tail(wv[p][r], tail, words & 3);
+                    }
+                }
+            }
         }
         // the x sums only after every pass's loads are issued (summing pass p's x first would make the wave wait
         // for it before requesting pass p + 1); with several passes the order is pinned for the scheduler too
