@@ -535,7 +535,8 @@ def bench_decode(D, w, hot, dev, n_prompt: int = 64, n_new: int = 128, hot_sweep
         eng = D.DecodeEngine(w, base, dip_k=None if base == "dense" else k,
                              hot_channels=mode_hot if base == "cached_dip" else None,
                              max_new_tokens=n_new,
-                             dip_schedule={"dip_dense_up": "dense_up", "dip_gated": "gated"}.get(kind),
+                             dip_schedule={"dip": "indexed", "dip_dense_up": "dense_up",
+                                           "dip_gated": "gated"}.get(kind),
                              miss_path="staged" if mode == "cached_dip_staged" else "direct",
                              offload=kind.endswith("_offload"), overlap_copy=not mode.endswith("_serial"),
                              int4_head=int4_head)

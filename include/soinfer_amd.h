@@ -719,6 +719,8 @@ int soi_quantize_group_supported(int64_t group_size);
 int soi_quantize_group(const float* w, int8_t* q, float* scale, int64_t N, int64_t K, int64_t group_size, int64_t qmax,
                        void* stream);
 int soi_pack_int4(const int8_t* q, uint8_t* out, int64_t N, int64_t K, void* stream);
+/* Packed codes [n, ceil(H/8)*4] -> the transpose, packed [H, n/2] (n % 8 == 0; both 4-byte aligned). */
+int soi_transpose_int4(const uint8_t* Wq, uint8_t* out, int64_t n, int64_t H, void* stream);
 
 /* y[N0 + N1] = W0 x, then W1 x (each row as soi_gemv_w4a16_group_lop3 gives it; both matrices [., K], N1 may be 0) in one
  * launch. clear: this many words (at most N0 + N1) are set to zero, e.g. the arrival counters of a sparse down that

@@ -1787,6 +1787,18 @@ torch::Tensor pack_int4(torch::Tensor q) {
     return out;
 }
 
+torch::Tensor transpose_int4(torch::Tensor Wq, int64_t H) {
+    const char* n = "transpose_int4";
+    need(Wq, torch::kUInt8, Wq, n, "Wq");
+    TORCH_CHECK(Wq.dim() == 2 && H >= 1 && Wq.size(1) == (H + 7) / 8 * 4 && Wq.size(0) % 8 == 0, n,
+                ": Wq must be [n, ceil(H/8)*4], n a multiple of 8");
+    const at::DeviceGuard guard(Wq.device());
+    auto out = torch::empty({H, Wq.size(0) / 2}, Wq.options());
+    if (Wq.size(0) == 0) return out;
+    check_status(soi_transpose_int4(Wq.data_ptr<uint8_t>(), out.data_ptr<uint8_t>(), Wq.size(0), H, cur_stream(Wq)), n);
+    return out;
+}
+
 // ---------------------------------------------------------------------------
 // one DIP MLP call (soinfer.runtime.dip): allocations and launches in one place
 // ---------------------------------------------------------------------------
@@ -2002,6 +2014,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("attention_tokens_supported", &soi_attention_tokens_supported, "whether prompt_attention_ takes the heads");
     m.def("prompt_attention_", &prompt_attention_, "one layer's attention block over T tokens, added to x");
     m.def("prompt_mlp_dense_", &prompt_mlp_dense_, "one layer's dense MLP over T tokens, added to x");
+    m.def("norm_gemv_one_pass",
+          [](int64_t N, int64_t K, int64_t gs, bool swiglu) { return soi_norm_gemv_one_pass(N, K, gs, swiglu ? 1 : 0) != 0; },
+          "whether the RMSNorm-fused GEMV of [N, K] rows takes the one-pass norm partition");
     m.def("dip_tokens_max_channels", &soi_dip_tokens_max_channels, "most channels prompt_mlp_dip_ selects from");
     m.def("prompt_mlp_dip_", &prompt_mlp_dip_, "one layer's DIP MLP over T tokens, added to x", py::arg("T"),
           py::arg("k"), py::arg("x"), py::arg("norm"), py::arg("h"), py::arg("gate_Wq"), py::arg("gate_scale"),
@@ -2012,6 +2027,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("image_down") = py::none(), py::arg("mark") = py::none(), py::arg("stamp") = 0);
     m.def("quantize_group", &quantize_group, "symmetric group quantization: (codes, scales)");
     m.def("pack_int4", &pack_int4, "int8 codes to AWQ-order INT4 rows");
+    m.def("transpose_int4", &transpose_int4, "the transpose of packed INT4 rows, packed");
     m.def("dip_mlp", &dip_mlp, "one DIP MLP over resident weights: (y, idx)");
     m.def("dip_gate_select", &dip_gate_select, "gate, selection and a cleared down workspace (and the miss count)",
           py::arg("gate_Wq"), py::arg("gate_scale"), py::arg("x"), py::arg("k"), py::arg("K"), py::arg("group_size"),

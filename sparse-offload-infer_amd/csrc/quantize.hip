@@ -103,9 +103,55 @@ __global__ __launch_bounds__(kQuantThreads) void pack_int4_kernel(const int8_t* 
     stg(out + id, pack8(v[0], v[1]));
 }
 
+// out [H, n/8] words = the transpose of the n x H codes of in [n, words] (both AWQ order, no rounding): a workgroup turns a
+// 64 x 64 tile in LDS, so both sides move 32-byte row segments. (As tensor
+// operations the 28 copies of a Qwen3-1.7B-shaped DIP engine took 7 ms of its construction.)
+constexpr int kTile = 64;
+
+__global__ __launch_bounds__(kQuantThreads) void transpose_int4_kernel(const uint32_t* __restrict__ in,
+                                                                       uint32_t* __restrict__ out, int n, int H,
+                                                                       int words) {
+    __shared__ uint8_t s[kTile][kTile + 4];  // [column][channel]
+    const int c0 = static_cast<int>(blockIdx.y) * kTile, w0 = static_cast<int>(blockIdx.x) * (kTile / 8);
+    const int tid = threadIdx.x;
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+        const int id = tid + it * kQuantThreads, ch = id >> 3, w = id & 7;  // 8 words of each of 64 channels
+        const uint32_t v = c0 + ch < n && w0 + w < words ? ldg(in + static_cast<int64_t>(c0 + ch) * words + w0 + w) : 0u;
+#pragma unroll
+        for (int j = 0; j < 8; ++j)  // element j of a word: nibble j / 2 (even j) or 4 + j / 2
+            s[8 * w + j][ch] = static_cast<uint8_t>((v >> (4 * ((j >> 1) + ((j & 1) << 2)))) & 15u);
+    }
+    __syncthreads();
+#pragma unroll
+    for (int it = 0; it < 2; ++it) {
+        const int id = tid + it * kQuantThreads, col = id >> 3, w = id & 7;
+        const int64_t row = static_cast<int64_t>(w0) * 8 + col;
+        if (row >= H || c0 + 8 * w >= n) continue;
+        const uint32_t* p = reinterpret_cast<const uint32_t*>(&s[col][8 * w]);
+        stg(out + row * (n >> 3) + (c0 >> 3) + w, pack8(p[0], p[1]));
+    }
+}
+
 }  // namespace soi
 
 using namespace soi;
+
+extern "C" int soi_transpose_int4(const uint8_t* Wq, uint8_t* out, int64_t n, int64_t H, void* stream) {
+    const char* what = "soi_transpose_int4";
+    SOI_REQUIRE(n >= 8 && n % 8 == 0 && n <= 65535 * int64_t(kTile) && H >= 1 && H <= (int64_t(1) << 30),
+                "%s: n must be a multiple of 8", what);
+    SOI_REQUIRE(Wq && out && ((reinterpret_cast<uintptr_t>(Wq) | reinterpret_cast<uintptr_t>(out)) & 3u) == 0,
+                "%s: null pointer or rows not 4-byte aligned", what);
+    const int64_t words = ceil_div64(H, 8);
+    hipLaunchKernelGGL(transpose_int4_kernel,
+                       dim3(static_cast<unsigned>(ceil_div64(words, kTile / 8)),
+                            static_cast<unsigned>(ceil_div64(n, kTile))),
+                       dim3(kQuantThreads), 0, as_stream(stream), reinterpret_cast<const uint32_t*>(Wq),
+                       reinterpret_cast<uint32_t*>(out), static_cast<int>(n), static_cast<int>(H),
+                       static_cast<int>(words));
+    return launch_status(what);
+}
 
 extern "C" int soi_quantize_group_supported(int64_t group_size) {
     return group_size == 32 || group_size == 64 || group_size == 128 || group_size == 256 ? 1 : 0;

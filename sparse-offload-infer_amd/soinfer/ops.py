@@ -278,6 +278,9 @@ def transposed_down_T(Wq_T: torch.Tensor, scale_T: torch.Tensor, H: int) -> tupl
     n = Wq_T.shape[0]
     if n % 8:
         raise ValueError("transposed_down_T: the channel count must be a multiple of 8")
+    if Wq_T.is_cuda and Wq_T.dtype == torch.uint8 and Wq_T.is_contiguous() and Wq_T.data_ptr() % 4 == 0 and n and \
+            Wq_T.dim() == 2 and Wq_T.shape[1] == -(-H // 8) * 4:
+        return _C.transpose_int4(Wq_T, H), scale_T.t().contiguous()
     q = pack.unpack_int4(Wq_T, H)  # int8 [n, H]
     Wt, _ = pack.pack_int4(q.t().contiguous())
     return Wt.contiguous(), scale_T.t().contiguous()

@@ -216,9 +216,9 @@ class DecodeEngine:
     """Greedy decoder over DecoderWeights. mode: "dense", "dip" (top dip_k channels per layer, weights
     resident) or "cached_dip" (hot channels resident, the rest in pinned host memory; miss_path "direct" reads
     the misses in place inside the up / down kernels, "staged" gathers them into device staging first).
-    dip_schedule (mode "dip"): "indexed" (default; 4 MLP launches, the schedule cached_dip equals bit for bit),
-    "gated" (2 MLP launches, the same tokens and hidden states as "indexed" bit for bit) or "dense_up" (2 MLP
-    launches, y summed in another order; dip_dense_up=True is the same).
+    dip_schedule (mode "dip"): "indexed" (4 MLP launches, the schedule cached_dip equals bit for bit), "gated" (2 MLP
+    launches, the same tokens and hidden states as "indexed" bit for bit) or "dense_up" (2 MLP launches, y summed in
+    another order; dip_dense_up=True is the same). Default: the indexed results, by the gated launches where they fit.
     offload=True keeps the dense weights of every layer (q|k|v, o, and gate|up + down for dense or gate for
     cached DIP) in a pinned host arena and copies each layer's block into one of two device slots: the
     reference's streamed configuration (WeightPipeline, generate.py:85-138). With overlap_copy=True (default)
@@ -247,6 +247,14 @@ class DecodeEngine:
                  defer_attention_combine: bool = True, int4_head: bool = False, dip_schedule: Optional[str] = None):
         if mode not in ("dense", "dip", "cached_dip"):
             raise ValueError(f"unknown mode {mode!r}")
+        # no schedule named: the indexed schedule's results from the gated schedule's two MLP launches, bit for bit the
+        # same where both norm the MLP input in one partition (a token of the 28-layer Qwen3-1.7B shape at k/I = 0.5
+        # takes 0.75 against 0.94 ms); single steps that a layer hook watches run the indexed launches
+        c0 = w.config
+        self._gated_auto = dip_schedule is None and not dip_dense_up and mode == "dip" and fused and \
+            c0.intermediate % 4 == 0 and \
+            _C.norm_gemv_one_pass(c0.intermediate, c0.hidden, c0.group_size, False) == \
+            _C.norm_gemv_one_pass(2 * c0.intermediate, c0.hidden, c0.group_size, True)
         if dip_schedule is None:
             dip_schedule = "dense_up" if dip_dense_up else "indexed"
         if dip_schedule not in ("indexed", "dense_up", "gated"):
@@ -266,7 +274,7 @@ class DecodeEngine:
         # accumulate reads them in place)
         self.down_copy = down_copy
         # DIP schedules for resident weights (mode 'dip'):
-        #  * "indexed" (default): RMSNorm-fused gate GEMV, top-k, up GEMV over the selected rows with the SiLU
+        #  * "indexed": RMSNorm-fused gate GEMV, top-k, up GEMV over the selected rows with the SiLU
         #    epilogue, sparse down over the selected down^T rows (4 MLP launches); the cache-aware modes equal it
         #    bit for bit;
         #  * "gated" (2 MLP launches, the same y as "indexed" bit for bit): where the shape fits
@@ -285,7 +293,7 @@ class DecodeEngine:
         self.dip_schedule = dip_schedule
         self.dip_dense_up = dip_dense_up
         self.dip_gated = dip_schedule == "gated"
-        self.dip_gated_tr = self.dip_gated and dip_k is not None and 1 <= dip_k <= w.config.intermediate and \
+        self.dip_gated_tr = (self.dip_gated or self._gated_auto) and dip_k is not None and 1 <= dip_k <= w.config.intermediate and \
             _C.dip_select_down_ordered_lds_bytes(w.config.hidden, w.config.intermediate, dip_k) > 0
         c = w.config
         self.w, self.c, self.mode, self.fused = w, c, mode, fused
@@ -343,7 +351,7 @@ class DecodeEngine:
         if dip_dense_up or self.dip_gated_tr:
             # down_proj^T's values transposed for the one-launch down (the same quantized values, no rounding)
             self.down_tt = [ops.transposed_down_T(L.down_T_Wq, L.down_T_scale, H) for L in w.layers]
-        if fused and (mode == "dense" or dip_schedule != "indexed"):
+        if fused and (mode == "dense" or dip_schedule != "indexed" or self._gated_auto):
             # gate|up rows interleaved by 8-row tiles (gate 4t..4t+3, up 4t..4t+3) for the SwiGLU epilogue
             t = torch.arange(I // 4, device=dev)
             perm = torch.stack([4 * t + i for i in range(4)] + [I + 4 * t + i for i in range(4)], 1).reshape(-1)
@@ -556,6 +564,11 @@ class DecodeEngine:
                                       res if res_out is not None else None, res_out)
         self._count_selection(l)
 
+    @property
+    def _gated_now(self) -> bool:
+        """Whether this step's MLPs run the gated schedule's launches."""
+        return self.dip_gated or (self._gated_auto and self.layer_hook is None)
+
     def _gated_down(self, l: int, L: LayerWeights, gate: torch.Tensor, hu: torch.Tensor,
                     res: Optional[torch.Tensor] = None, res_out: Optional[torch.Tensor] = None):
         """Selection + sparse down of the gated schedule. Over the transposed copy (hu = h of every channel) the
@@ -635,7 +648,7 @@ class DecodeEngine:
         cur, other = self.x, self.x2
         fold = self.residual_epilogue
         # the down launch writes the residual
-        down_res = fold and (self.mode == "dense" or self.dip_dense_up or self.dip_gated_tr)
+        down_res = fold and (self.mode == "dense" or self.dip_dense_up or (self._gated_now and self.dip_gated_tr))
         last = len(self.w.layers) - 1
         _C.embed_lookup_into(self.w.embed, self.token, cur)
         for l, L in enumerate(self.w.layers):
@@ -700,7 +713,7 @@ class DecodeEngine:
                                                    H, gs)
             self._dense_down(l, gate, self.gu[I:], x, res_out)
             return
-        if self.dip_gated:
+        if self._gated_now:
             gW, gS = gu_il
             if self.dip_gated_tr:  # gate and h of every channel, as the dense-up schedule's first launch
                 _C.gemv_w4a16_rmsnorm_swiglu_gate_into(gW, gS, x, delta, L.post_norm, eps, x_out, gate,

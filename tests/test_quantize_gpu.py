@@ -75,3 +75,16 @@ def test_observed_calls_take_the_expressions(cuda):
     plain = w.detach()
     rows = torch.vmap(lambda r: formats.quantize(r, cfg).scale)(plain)
     same(rows, formats.quantize(plain, cfg).scale)
+
+
+@pytest.mark.parametrize("n,H", [(8, 1), (8, 8), (64, 64), (72, 65), (136, 1000), (6144, 2048)])
+def test_transposed_rows(cuda, n, H):
+    from soinfer import ops
+    from soinfer.quant import pack
+
+    q = torch.randint(-8, 8, (n, H), generator=torch.Generator().manual_seed(n + H), dtype=torch.int8)
+    s = torch.rand(n, 3)
+    W = pack.pack_int4(q)[0]
+    got, gs = ops.transposed_down_T(W.to(cuda), s.to(cuda), H)
+    same(got, pack.pack_int4(q.t().contiguous())[0])
+    same(gs, s.t().contiguous())
