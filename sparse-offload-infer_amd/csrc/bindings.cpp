@@ -1864,7 +1864,7 @@ std::tuple<torch::Tensor, torch::Tensor> dip_mlp(torch::Tensor gate_Wq, torch::T
 
 // First half of the cache-aware DIP MLP: (gate [I], idx [k], workspace of the down, counters cleared). With slot_of,
 // also the number of selected channels outside the cache, written to miss_count (one int32 of device memory or of
-// pinned host memory). The second half reads missing rows from pinned memory in place: the call takes 115 us at 20% of
+// pinned host memory). The second half reads missing rows from pinned memory in place: the call takes 126 us at 20% of
 // the channels cached (5 MB of misses, 88 us at the link's rate) against 398 us with host gathers through staging.
 std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> dip_gate_select(torch::Tensor gate_Wq, torch::Tensor gate_scale,
                                                                         torch::Tensor x, int64_t k, int64_t K,

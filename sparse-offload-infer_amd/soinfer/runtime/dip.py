@@ -105,10 +105,14 @@ def cached_dip_mlp(w: DipMLPWeights, cache: HotCache, x: torch.Tensor, dip_k: in
     count = torch.empty(1, dtype=torch.int32, pin_memory=True)
     gate, idx, ws = _C.dip_gate_select(w.gate_Wq, w.gate_scale, x, dip_k, w.hidden_size, w.group_size, cache.slot_of,
                                        count)
-    counted = torch.cuda.Event()
-    counted.record(torch.cuda.current_stream(x.device))
-    y = _cached_mlp(w, cache, x, gate, idx, ws, host_up if hosted else w.up_Wq, host_down_T if hosted else w.down_T_Wq)
-    counted.synchronize()  # the count is read while the GEMVs run
+    stream, read = torch.cuda.current_stream(x.device), torch.cuda.Event()
+    if hosted:
+        y = _cached_mlp(w, cache, x, gate, idx, ws, host_up, host_down_T, lambda: read.record(stream))
+    else:
+        read.record(stream)
+        y = _cached_mlp(w, cache, x, gate, idx, ws, w.up_Wq, w.down_T_Wq)
+    # the count has arrived, and the host rows, which the caller may change or free once this returns, have been read
+    read.synchronize()
     mc = int(count)
     if miss_bytes is not None:
         miss_bytes.append(mc * (w.up_Wq.shape[1] + w.down_T_Wq.shape[1]))
@@ -151,10 +155,11 @@ def _cached_mlp_staged(w: DipMLPWeights, cache: HotCache, x: torch.Tensor, dip_k
     return y, idx, mc
 
 
-def _cached_mlp(w: DipMLPWeights, cache: HotCache, x, gate, idx, ws, full_up, full_down_T) -> torch.Tensor:
+def _cached_mlp(w: DipMLPWeights, cache: HotCache, x, gate, idx, ws, full_up, full_down_T,
+                rows_read=lambda: None) -> torch.Tensor:
     """The up and down halves over the hot cache: hits from the cache, misses from full_up / full_down_T in place. For
     misses in host memory the up GEMV also copies its channels' down^T rows to the device (whole rows cross PCIe faster
-    than the down's column slices)."""
+    than the down's column slices). rows_read() is called after the last launch that reads full_up or full_down_T."""
     H, gs, k = w.hidden_size, w.group_size, idx.shape[0]
     h = torch.empty(k, dtype=torch.float16, device=x.device)
     row = full_down_T.shape[1]
@@ -162,9 +167,13 @@ def _cached_mlp(w: DipMLPWeights, cache: HotCache, x, gate, idx, ws, full_up, fu
     staged = torch.empty(k, row, dtype=torch.uint8, device=x.device) if copy else None
     _C.gemv_dip_cached_up_silu_into(cache.up_Wq, cache.up_scale, full_up, w.up_scale, cache.slot_of, idx, x, gate, h, H,
                                     gs, full_down_T if copy else None, staged)
+    if copy:
+        rows_read()
     y = torch.empty(H, dtype=torch.float16, device=x.device)
     _C.gemv_dip_cached_down_into(cache.down_Wq, cache.down_scale, full_down_T, w.down_T_scale, cache.slot_of, idx, h, y,
                                  H, gs, ws, staged)
+    if not copy:
+        rows_read()
     return y
 
 

@@ -81,3 +81,18 @@ def test_refusals(cuda):
         dip.cached_dip_mlp(w, cache, x, 32, *pinned, tiny)
     with pytest.raises(RuntimeError):  # not pinned
         dip.cached_dip_mlp(w, cache, x, 32, *[p.clone() for p in pinned], tiny)
+
+
+def test_host_rows_belong_to_the_caller_after_the_call(cuda):
+    from soinfer.offload.hot_cache import HotCache
+    from soinfer.runtime import dip
+
+    w, x = make(cuda, 4096, 2048, 128, 9)
+    y, idx = by_operators(w, x, 4096)
+    cache = HotCache.build(w.up_Wq, w.up_scale, w.down_T_Wq, w.down_T_scale, [7])
+    pinned = [torch.empty(t.shape, dtype=torch.uint8, pin_memory=True).copy_(t) for t in (w.up_Wq, w.down_T_Wq)]
+    staging = torch.empty(pinned[0].numel(), dtype=torch.uint8, pin_memory=True)
+    got = dip.cached_dip_mlp(w, cache, x, 4096, *pinned, staging)
+    for p in pinned:  # 8 MB of misses take far longer over the link than this
+        p.zero_()
+    assert torch.equal(got[0], y) and torch.equal(got[1], idx)
