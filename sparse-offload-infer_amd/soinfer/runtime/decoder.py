@@ -857,8 +857,7 @@ class DecodeEngine:
             _C.prompt_mlp_dip_(*args, L.gu_Wq, L.gu_scale, b["gu"], b["idx"], b["hs"], L.down_T_Wq, L.down_T_scale, gs,
                                eps, self.dip_gated)
             if self.counts is not None:
-                sel = b["idx"][:T * self.k].long()
-                self.counts[l].index_add_(0, sel, torch.ones_like(sel, dtype=self.counts[l].dtype))
+                add_selection_counts(self.counts[l], b["idx"][:T * self.k])
             return
         cache, (up, down) = self.caches[l], b["images"]
         self._prompt_stamp += 1
@@ -930,6 +929,12 @@ class DecodeEngine:
         if eos_token_id is not None and eos_token_id in out:
             out = out[:out.index(eos_token_id) + 1]
         return list(prompt_ids) + out
+
+
+def add_selection_counts(counts: torch.Tensor, sel: torch.Tensor) -> None:
+    """counts[c] += the occurrences of channel c in sel (int32). Negative entries name no channel (a prompt token with
+    fewer than k gates that are numbers leaves the rest of its list at -1) and count nothing."""
+    counts.index_add_(0, sel.long().clamp_min_(0), (sel >= 0).to(counts.dtype))
 
 
 def calibrate_channel_counts(w: DecoderWeights, dip_k: int, calib_tokens) -> list:

@@ -203,3 +203,56 @@ def test_matrix_core_linear(cuda, N, K, gs, T):
     want = (gate / (1 + torch.exp(-gate)) * up).view(T, N // 2)
     got = h.view(-1, N // 256, 4, 4, 16, 8).permute(0, 4, 1, 3, 2, 5).reshape(-1, N // 2)[:T].float()
     assert bool(((got - want).abs() <= 2.0 ** -10 * want.abs() + 2.0 ** -24).all())
+
+
+def hip_lib():
+    from soinfer.quant import pack
+
+    return ctypes.CDLL(str(Path(pack.__file__).resolve().parent.parent / "libsoinfer_hip.so"))
+
+
+@pytest.mark.parametrize("n,k", [(512, 200), (6144, 3072), (16384, 16384)])
+def test_selection_of_gates_that_are_not_numbers(cuda, n, k):
+    """A token with m < k gates that are numbers selects those and leaves -1 in the rest of its list and no mark; the
+    other tokens' lists are those of the same gates without it."""
+    g = torch.Generator(device=cuda).manual_seed(n)
+    gate = torch.randn(4, n, generator=g, device=cuda).half()
+    gate[1] = float("nan")
+    m = max(1, k // 3)
+    numbers = torch.randperm(n, generator=g, device=cuda)[:m].sort().values
+    kept = gate[2, numbers].clone()
+    gate[2] = float("nan")
+    gate[2, numbers] = kept
+    idx = torch.full((4, k), 12345678, dtype=torch.int32, device=cuda)
+    mark = torch.zeros(n, dtype=torch.int32, device=cuda)
+    ptr = [ctypes.c_void_p(t.data_ptr()) for t in (gate, idx, mark)]
+    st = hip_lib().soi_dip_select_tokens(ptr[0], *(ctypes.c_int64(v) for v in (n, n, k, 4)), ptr[1], ptr[2],
+                                         ctypes.c_int32(9), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert st == 0
+    from soinfer import ops
+
+    for t in (0, 3):
+        assert torch.equal(idx[t], ops.topk_threshold_select(gate[t].float().abs(), k))
+    assert bool((idx[1] == -1).all())
+    assert torch.equal(idx[2, :m].long(), numbers) and bool((idx[2, m:] == -1).all())
+    named = torch.zeros(n, dtype=torch.bool, device=cuda)
+    for t in (0, 2, 3):
+        named[idx[t][idx[t] >= 0].long()] = True
+    assert torch.equal(mark == 9, named)
+
+
+def test_calibration_counts_of_a_token_without_numbers(dec, weights):
+    """A token whose hidden state is not a number selects nothing: the counts are the other tokens'. (Last in the prompt:
+    tokens after it attend to its K and V.)"""
+    import dataclasses
+
+    c = weights.config
+    embed = weights.embed.clone()
+    embed[5] = float("nan")
+    w = dataclasses.replace(weights, embed=embed)
+    k = c.intermediate // 3
+    prompt = [t if t != 5 else 6 for t in tokens(21, c.vocab, 5)]
+    want = dec.calibrate_channel_counts(w, k, prompt)
+    got = dec.calibrate_channel_counts(w, k, prompt + [5])
+    for a, b in zip(got, want):
+        assert torch.equal(a, b) and int(b.sum()) == 21 * k
