@@ -103,14 +103,20 @@ def cached_dip_mlp(w: DipMLPWeights, cache: HotCache, x: torch.Tensor, dip_k: in
     if hosted and not _mapped(w, host_up, host_down_T, staging, dip_k):
         return _cached_mlp_staged(w, cache, x, dip_k, host_up, host_down_T, staging, miss_bytes)
     count = torch.empty(1, dtype=torch.int32, pin_memory=True)
-    gate, idx, ws = _C.dip_gate_select(w.gate_Wq, w.gate_scale, x, dip_k, w.hidden_size, w.group_size, cache.slot_of,
-                                       count)
     stream, read = torch.cuda.current_stream(x.device), torch.cuda.Event()
-    if hosted:
-        y = _cached_mlp(w, cache, x, gate, idx, ws, host_up, host_down_T, lambda: read.record(stream))
-    else:
-        read.record(stream)
-        y = _cached_mlp(w, cache, x, gate, idx, ws, w.up_Wq, w.down_T_Wq)
+    try:
+        gate, idx, ws = _C.dip_gate_select(w.gate_Wq, w.gate_scale, x, dip_k, w.hidden_size, w.group_size,
+                                           cache.slot_of, count)
+        if hosted:
+            y = _cached_mlp(w, cache, x, gate, idx, ws, host_up, host_down_T, lambda: read.record(stream))
+        else:
+            read.record(stream)
+            y = _cached_mlp(w, cache, x, gate, idx, ws, w.up_Wq, w.down_T_Wq)
+    except BaseException:
+        # what was launched before the failure still writes the count and reads the host rows: neither may be given
+        # back before it has run
+        stream.synchronize()
+        raise
     # the count has arrived, and the host rows, which the caller may change or free once this returns, have been read
     read.synchronize()
     mc = int(count)

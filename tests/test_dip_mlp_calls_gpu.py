@@ -96,3 +96,29 @@ def test_host_rows_belong_to_the_caller_after_the_call(cuda):
     for p in pinned:  # 8 MB of misses take far longer over the link than this
         p.zero_()
     assert torch.equal(got[0], y) and torch.equal(got[1], idx)
+
+
+@pytest.mark.parametrize("side", ["up", "down"])
+def test_a_call_that_fails_leaves_nothing_running(cuda, side):
+    """A cache whose rows do not fit fails after the first launches of the call: by the time the error is raised they have
+    run, so the miss count's pinned word and the caller's host rows are free."""
+    import dataclasses
+
+    from soinfer.offload.hot_cache import HotCache
+    from soinfer.runtime import dip
+
+    w, x = make(cuda, 4096, 2048, 128, 9)
+    cache = HotCache.build(w.up_Wq, w.up_scale, w.down_T_Wq, w.down_T_scale, [7, 9])
+    name = {"up": "up_Wq", "down": "down_Wq"}[side]
+    bad = dataclasses.replace(cache, **{name: getattr(cache, name)[:, :-4].contiguous()})
+    pinned = [torch.empty(t.shape, dtype=torch.uint8, pin_memory=True).copy_(t) for t in (w.up_Wq, w.down_T_Wq)]
+    staging = torch.empty(pinned[0].numel(), dtype=torch.uint8, pin_memory=True)
+    for host in ((), (*pinned, staging)):
+        torch.cuda.synchronize()
+        torch.cuda._sleep(20_000_000)  # the launches of the call wait behind this
+        with pytest.raises(RuntimeError):
+            dip.cached_dip_mlp(w, bad, x, 4096, *host)
+        assert torch.cuda.current_stream().query()
+    y, idx = by_operators(w, x, 4096)
+    got = dip.cached_dip_mlp(w, cache, x, 4096, *pinned, staging)
+    assert torch.equal(got[0], y) and torch.equal(got[1], idx)
