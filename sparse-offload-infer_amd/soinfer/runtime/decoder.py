@@ -823,27 +823,36 @@ class DecodeEngine:
             bool(_C.attention_tokens_supported(c.q_heads, c.kv_heads, c.head_dim, c.max_seq))
 
     def _prompt_scratch(self, T: int) -> dict:
-        """Activations of T tokens, kept for the next prompt (T <= PROMPT_CHUNK; grown in powers of two)."""
+        """Activations of T tokens, kept for the next prompt (T <= PROMPT_CHUNK; grown in powers of two). The allocator
+        is told of every stream that uses them: growing, or the engine's end, gives the old ones back while a prompt on
+        another stream than theirs may still be running."""
+        stream = torch.cuda.current_stream(self.device)
         if self._prompt_buf is None or self._prompt_buf["T"] < T:
             c, cap = self.c, max(16, 1 << (T - 1).bit_length())
 
             def buf(n):
                 return torch.empty(cap * n, dtype=torch.float16, device=self.device)
 
-            self._prompt_buf = dict(T=cap, x=buf(c.hidden), h=buf(c.hidden), qkv=buf(c.qkv_rows),
-                                    q=buf(c.q_heads * c.head_dim), attn=buf(c.q_heads * c.head_dim),
-                                    gu=buf(2 * c.intermediate))
+            b = dict(T=cap, stream=stream, x=buf(c.hidden), h=buf(c.hidden), qkv=buf(c.qkv_rows),
+                     q=buf(c.q_heads * c.head_dim), attn=buf(c.q_heads * c.head_dim), gu=buf(2 * c.intermediate))
             if self.mode == "dense":
-                self._prompt_buf["m"] = buf(c.intermediate)
+                b["m"] = buf(c.intermediate)
             else:
-                self._prompt_buf["hs"] = buf(self.k)
-                self._prompt_buf["idx"] = torch.empty(cap * self.k, dtype=torch.int32, device=self.device)
+                b["hs"] = buf(self.k)
+                b["idx"] = torch.empty(cap * self.k, dtype=torch.int32, device=self.device)
             if self.mode == "cached_dip":  # images of one layer's up and down^T rows, and which rows are current
-                self._prompt_buf["images"] = [torch.empty(c.intermediate, self.st_up.shape[1], dtype=torch.uint8,
-                                                          device=self.device) for _ in range(2)]
-                self._prompt_buf["mark"] = torch.zeros(c.intermediate, dtype=torch.int32, device=self.device)
+                b["images"] = [torch.empty(c.intermediate, self.st_up.shape[1], dtype=torch.uint8, device=self.device)
+                               for _ in range(2)]
+                b["mark"] = torch.zeros(c.intermediate, dtype=torch.int32, device=self.device)
                 self._prompt_stamp = 0
-        return self._prompt_buf
+            self._prompt_buf = b
+        b = self._prompt_buf
+        if stream != b["stream"]:
+            for t in b.values():
+                for u in t if isinstance(t, list) else [t]:
+                    if isinstance(u, torch.Tensor):
+                        u.record_stream(stream)
+        return b
 
     def _prompt_mlp(self, l: int, L: LayerWeights, gu_il, b: dict, T: int, mfma: bool):
         """Layer l's MLP over T prompt tokens, added to their hidden states."""

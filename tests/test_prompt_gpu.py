@@ -256,3 +256,32 @@ def test_calibration_counts_of_a_token_without_numbers(dec, weights):
     got = dec.calibrate_channel_counts(w, k, prompt + [5])
     for a, b in zip(got, want):
         assert torch.equal(a, b) and int(b.sum()) == 21 * k
+
+
+@pytest.mark.parametrize("mode", ["dense", "dip", "cached_dip"])
+def test_scratch_given_back_while_another_stream_uses_it(cuda, dec, weights, mode):
+    """A prompt waits on a side stream while the scratch, which belongs to the default stream, is grown there and its old
+    memory is handed out again and overwritten: the prompt's state is that of an undisturbed one."""
+    c = weights.config
+    kw = {} if mode == "dense" else dict(dip_k=c.intermediate // 2)
+    if mode == "cached_dip":
+        kw["hot_channels"] = [list(range(0, c.intermediate, 3))] * c.layers
+    e = dec.DecodeEngine(weights, mode, max_new_tokens=1, **kw)
+    prompt = torch.tensor(tokens(16, c.vocab, 8), dtype=torch.int32, device=cuda)
+    e.reset()
+    e._prompt_layers(prompt)
+    want = e.x_final.clone()
+    sizes = [t.numel() * t.element_size() for v in e._prompt_buf.values() for t in (v if isinstance(v, list) else [v])
+             if isinstance(t, torch.Tensor)]
+    e.reset()
+    torch.cuda.synchronize()
+    side = torch.cuda.Stream()
+    with torch.cuda.stream(side):
+        torch.cuda._sleep(100_000_000)
+        e._prompt_layers(prompt)
+    e._prompt_scratch(200)
+    taken = [torch.full((n,), 255, dtype=torch.uint8, device=cuda) for n in sizes]
+    assert not side.query(), "the prompt is still waiting"
+    side.synchronize()
+    assert torch.equal(e.x_final, want)
+    del taken
