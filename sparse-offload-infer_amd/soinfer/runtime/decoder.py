@@ -368,6 +368,10 @@ class DecodeEngine:
             self._setup_offload()
         self._x_final = self.x
         self._prompt_buf = None  # scratch of _prompt_layers, made by the first prompt
+        # the token kernels read every row 16 bytes at a time; of the matrices that the steps take from any address, the
+        # o and down rows are the caller's (streamed ones lie in the slots, cached down^T rows in the images)
+        own = [L.o_Wq for L in w.layers] + [L.down_Wq if mode == "dense" else L.down_T_Wq for L in w.layers]
+        self._prompt_aligned = all(t.data_ptr() % 16 == 0 for t in own if t.device == dev)
         self._graph_layers = None
         self._graph_gen = None
         self._graph_gen_chunk = None  # GRAPH_CHUNK generation steps in one graph
@@ -819,7 +823,7 @@ class DecodeEngine:
             return False
         return n > 2 and self.fused and self.layer_hook is None and \
             c.hidden % 32 == 0 and c.intermediate % 32 == 0 and c.q_heads * c.head_dim % 32 == 0 and \
-            c.group_size % 32 == 0 and \
+            c.group_size % 32 == 0 and self._prompt_aligned and \
             bool(_C.attention_tokens_supported(c.q_heads, c.kv_heads, c.head_dim, c.max_seq))
 
     def _prompt_scratch(self, T: int) -> dict:

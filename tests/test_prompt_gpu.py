@@ -285,3 +285,25 @@ def test_scratch_given_back_while_another_stream_uses_it(cuda, dec, weights, mod
     side.synchronize()
     assert torch.equal(e.x_final, want)
     del taken
+
+
+@pytest.mark.parametrize("mode,name", [("dense", "o_Wq"), ("dense", "down_Wq"), ("dip", "o_Wq"), ("dip", "down_T_Wq")])
+def test_prompt_over_rows_off_16_bytes(cuda, dec, weights, mode, name):
+    """The decode step takes the down and down^T rows, and without the deferred attention combine the o rows, from any
+    address, so a prompt does too."""
+    import dataclasses
+
+    def off(t):
+        b = torch.empty(t.numel() + 16, dtype=t.dtype, device=t.device)
+        return b[4:4 + t.numel()].view(t.shape).copy_(t)
+
+    c = weights.config
+    kw = dict(dip_k=None if mode == "dense" else c.intermediate // 2, defer_attention_combine=name != "o_Wq")
+    moved = dataclasses.replace(weights, layers=[dataclasses.replace(L, **{name: off(getattr(L, name))})
+                                                 for L in weights.layers])
+    prompt = tokens(7, c.vocab, 4)
+    a = dec.DecodeEngine(moved, mode, max_new_tokens=3, **kw)
+    b = dec.DecodeEngine(weights, mode, max_new_tokens=3, **kw)
+    for use_graph in (False, True):
+        assert a.generate(prompt, 3, use_graph=use_graph) == b.generate(prompt, 3, use_graph=use_graph)
+        same_state(a, b, 10, f"{mode} {name}")
