@@ -212,13 +212,43 @@ def decoder_weights_from_arena(store, matrices, config: DecoderConfig, embed: to
     return DecoderWeights(config, embed, lm_head, final_norm, layers)
 
 
+def default_gated_form(H: int, I: int, k: int) -> Optional[str]:
+    """The MLP launches of a resident DIP engine without a named schedule: "ordered" (selection and down over the
+    transposed down_proj^T), "rows" (selection and gated sparse down over the selected rows), or None, the indexed ones.
+
+    The gated launches are two instead of four and read what the indexed ones leave out: up of the unselected channels
+    and, in the ordered form, their down values too (together `extra` bytes). An ordered workgroup takes 8 output columns
+    and all of its LDS tables, so H / 8 workgroups run in `rounds` of as many as fit the 256 CUs' LDS, and a second round
+    costs a launch's length. Above 16384 channels the row form selects in a launch of its own, and above 18432 an ordered
+    workgroup's threads hold too many channels each. Microseconds a layer and token, weights past the last-level cache,
+    indexed / ordered / rows:
+      2048 x 6144   k/I 0.5   30.4 / 23.0 / 26.8   one round, 6 MB     2560 x 9728   0.2   50.2 / 45.9 / 51.1   one, 20 MB
+      2560 x 9728   0.35      51.9 / 52.2 / 52.0   two, 16 MB          4096 x 6144   0.65  54.0 / 46.3 / 49.3   two, 9 MB
+      4096 x 12288  0.1       54.4 / 51.9 / 56.6   one, 45 MB          4096 x 12288  0.2   56.4 / 57.9 / 57.1   two, 40 MB
+      4096 x 12288  0.65      64.8 / - / 63.7      18 MB               5120 x 5120   0.8   68.8 / 66.5 / 62.3   three, 5 MB
+      5120 x 17408  0.2       79.1 / 106.4 / 88.6  three, 71 MB        1024 x 20480  0.05  39.2 / 40.7 / 41.8   one, 20 MB
+    """
+    extra = (I - k) * H
+    lds = _C.dip_select_down_ordered_lds_bytes(H, I, k)
+    if lds > 0 and I <= 18432:
+        per_cu = min(4, 160 * 1024 // (lds + 6 * 1024))
+        rounds = -(-(-(-H // 8)) // (256 * per_cu))
+        if (rounds == 1 and extra <= 50_000_000) or (rounds == 2 and extra <= 15_000_000):
+            return "ordered"
+    if I <= 8192 or (I <= 16384 and 2 * k >= I and extra <= 20_000_000):
+        return "rows"
+    return None
+
+
 class DecodeEngine:
     """Greedy decoder over DecoderWeights. mode: "dense", "dip" (top dip_k channels per layer, weights
     resident) or "cached_dip" (hot channels resident, the rest in pinned host memory; miss_path "direct" reads
     the misses in place inside the up / down kernels, "staged" gathers them into device staging first).
     dip_schedule (mode "dip"): "indexed" (4 MLP launches, the schedule cached_dip equals bit for bit), "gated" (2 MLP
     launches, the same tokens and hidden states as "indexed" bit for bit) or "dense_up" (2 MLP launches, y summed in
-    another order; dip_dense_up=True is the same). Default: the indexed results, by the gated launches where they fit.
+    another order; dip_dense_up=True is the same). Default: the indexed results, by the gated launches where these are
+    faster (default_gated_form). The gated launches keep a second copy of gate|up and, in the ordered form, of down_proj^T
+    (28 layers of the Qwen3-1.7B shape: 374 + 187 MB).
     offload=True keeps the dense weights of every layer (q|k|v, o, and gate|up + down for dense or gate for
     cached DIP) in a pinned host arena and copies each layer's block into one of two device slots: the
     reference's streamed configuration (WeightPipeline, generate.py:85-138). With overlap_copy=True (default)
@@ -248,13 +278,16 @@ class DecodeEngine:
         if mode not in ("dense", "dip", "cached_dip"):
             raise ValueError(f"unknown mode {mode!r}")
         # no schedule named: the indexed schedule's results from the gated schedule's two MLP launches, bit for bit the
-        # same where both norm the MLP input in one partition (a token of the 28-layer Qwen3-1.7B shape at k/I = 0.5
-        # takes 0.75 against 0.94 ms); single steps that a layer hook watches run the indexed launches
+        # same where both norm the MLP input in one partition, and where they are the faster ones (default_gated_form);
+        # single steps that a layer hook watches run the indexed launches
         c0 = w.config
-        self._gated_auto = dip_schedule is None and not dip_dense_up and mode == "dip" and fused and \
-            c0.intermediate % 4 == 0 and \
-            _C.norm_gemv_one_pass(c0.intermediate, c0.hidden, c0.group_size, False) == \
-            _C.norm_gemv_one_pass(2 * c0.intermediate, c0.hidden, c0.group_size, True)
+        auto = None
+        if dip_schedule is None and not dip_dense_up and mode == "dip" and fused and dip_k is not None and \
+                1 <= dip_k <= c0.intermediate and c0.intermediate % 4 == 0 and \
+                _C.norm_gemv_one_pass(c0.intermediate, c0.hidden, c0.group_size, False) == \
+                _C.norm_gemv_one_pass(2 * c0.intermediate, c0.hidden, c0.group_size, True):
+            auto = default_gated_form(c0.hidden, c0.intermediate, dip_k)
+        self._gated_auto = auto is not None
         if dip_schedule is None:
             dip_schedule = "dense_up" if dip_dense_up else "indexed"
         if dip_schedule not in ("indexed", "dense_up", "gated"):
@@ -293,7 +326,8 @@ class DecodeEngine:
         self.dip_schedule = dip_schedule
         self.dip_dense_up = dip_dense_up
         self.dip_gated = dip_schedule == "gated"
-        self.dip_gated_tr = (self.dip_gated or self._gated_auto) and dip_k is not None and 1 <= dip_k <= w.config.intermediate and \
+        self.dip_gated_tr = auto == "ordered" or self.dip_gated and dip_k is not None and \
+            1 <= dip_k <= w.config.intermediate and \
             _C.dip_select_down_ordered_lds_bytes(w.config.hidden, w.config.intermediate, dip_k) > 0
         c = w.config
         self.w, self.c, self.mode, self.fused = w, c, mode, fused
@@ -955,7 +989,7 @@ def calibrate_channel_counts(w: DecoderWeights, dip_k: int, calib_tokens) -> lis
     time through the DIP engine (eagerly) as the reference's calibrate_channel_frequencies does
     (generate.py:579-609). int64 [I] tensors on the engine's device; each sums to len(calib_tokens) * dip_k."""
     c = w.config
-    eng = DecodeEngine(w, "dip", dip_k=dip_k, max_new_tokens=1)
+    eng = DecodeEngine(w, "dip", dip_k=dip_k, max_new_tokens=1, dip_schedule="indexed")  # no copies of the weights
     eng.counts = [torch.zeros(c.intermediate, dtype=torch.int64, device=eng.device) for _ in range(c.layers)]
     eng.reset()
     eng.prefill(calib_tokens, use_graph=False)

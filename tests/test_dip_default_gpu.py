@@ -10,6 +10,8 @@ CONFIGS = {
     "ordered": (dict(hidden=256, q_heads=4, kv_heads=2, head_dim=64, intermediate=512), 200, True),
     "one_pass": (dict(hidden=2048, q_heads=4, kv_heads=2, head_dim=128, intermediate=1536), 700, True),
     "row_form": (dict(hidden=512, q_heads=4, kv_heads=2, head_dim=64, intermediate=9216), 6000, True),
+    "row_form_only": (dict(hidden=512, q_heads=4, kv_heads=2, head_dim=64, intermediate=9216), 8800, True),
+    "too_wide": (dict(hidden=1024, q_heads=4, kv_heads=2, head_dim=64, intermediate=20480), 2000, False),
     "other_norm": (dict(hidden=2048, q_heads=4, kv_heads=2, head_dim=128, intermediate=4100), 900, False),
     "odd_width": (dict(hidden=256, q_heads=4, kv_heads=2, head_dim=64, intermediate=518), 100, False),
 }
