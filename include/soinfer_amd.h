@@ -686,7 +686,8 @@ int soi_attention_tokens(const uint16_t* q, const uint16_t* k_cache, const uint1
 /* Dynamic Input Pruning over T tokens, every value bit for bit the decode step's:
  *   soi_dip_select_tokens: idx[t, k] = the rule-A selection over |gate[t * ld + i]|, i < n <=
  *     soi_dip_tokens_max_channels() (soi_topk_threshold_select_f16abs; -1 past the selected count). mark (optional,
- *     [n]): every selected channel's word = stamp.
+ *     [n]): every selected channel's word = stamp. last_idx [k], last_count [1] (optional, together): the last
+ *     token's indices and count, nothing past the count written.
  *   soi_dip_gate_tokens: h[t, j] = fp16(silu(gate) * up) of channel idx[t, j] (NaN for none).
  *   soi_dip_fetch_rows: rows whose mark is stamp into the device images image_up / image_down [num_channels,
  *     row_bytes], from the cache (row slot_of[c]) or the host rows (device mapping of pinned memory).
@@ -694,7 +695,7 @@ int soi_attention_tokens(const uint16_t* q, const uint16_t* k_cache, const uint1
  *     H and group_size multiples of 32, Wq_T 16-byte aligned. */
 int64_t soi_dip_tokens_max_channels(void);
 int soi_dip_select_tokens(const uint16_t* gate, int64_t ld, int64_t n, int64_t k, int64_t T, int32_t* idx,
-                          int32_t* mark, int32_t stamp, void* stream);
+                          int32_t* mark, int32_t stamp, int32_t* last_idx, int32_t* last_count, void* stream);
 int soi_dip_gate_tokens(const uint16_t* gate, const uint16_t* up, int64_t ld, int64_t n, const int32_t* idx,
                         uint16_t* h, int64_t k, int64_t T, void* stream);
 int soi_dip_fetch_rows(const uint8_t* cache_up, const uint8_t* host_up, uint8_t* image_up, int64_t up_row_bytes,

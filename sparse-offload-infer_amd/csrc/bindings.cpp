@@ -1685,14 +1685,16 @@ void prompt_mlp_dense_(int64_t T, torch::Tensor x, torch::Tensor norm, torch::Te
 // holds the gate rows; the up and down^T rows that any token selects are fetched from the hot cache (cache_up,
 // cache_down, slot_of) or the host arena (device addresses) into the images, which then serve as the matrices.
 // norm_pair: the norm's partition of the gate|up launch (two rows per channel) instead of the gate launch's.
-// h, gu [T, 2 I], idx [T, k], hs [T, k]: scratch; mark [I]: stamps of earlier calls, none equal to `stamp`.
+// h, gu [T, 2 I], idx [T, k], hs [T, k]: scratch; mark [I]: stamps of earlier calls, none equal to `stamp`. last_idx,
+// last_count: the last token's selection as a decode step leaves it.
 void prompt_mlp_dip_(int64_t T, int64_t k, torch::Tensor x, torch::Tensor norm, torch::Tensor h, torch::Tensor gate_Wq,
                      torch::Tensor gate_scale, torch::Tensor gu, torch::Tensor idx, torch::Tensor hs,
                      c10::optional<torch::Tensor> down_Wq, torch::Tensor down_scale, int64_t group_size, double eps,
                      bool norm_pair, c10::optional<torch::Tensor> up_scale, c10::optional<torch::Tensor> cache_up,
                      c10::optional<torch::Tensor> cache_down, c10::optional<torch::Tensor> slot_of, int64_t host_up,
                      int64_t host_down, c10::optional<torch::Tensor> image_up, c10::optional<torch::Tensor> image_down,
-                     c10::optional<torch::Tensor> mark, int64_t stamp) {
+                     c10::optional<torch::Tensor> mark, int64_t stamp, c10::optional<torch::Tensor> last_idx,
+                     c10::optional<torch::Tensor> last_count) {
     const char* n = "prompt_mlp_dip_";
     TORCH_CHECK(T >= 1, n, ": T must be positive");
     const bool cached = up_scale.has_value();
@@ -1708,6 +1710,13 @@ void prompt_mlp_dip_(int64_t T, int64_t k, torch::Tensor x, torch::Tensor norm, 
     need_numel(gu, T * 2 * I, n, "gu");
     need_numel(idx, T * k, n, "idx");
     need_numel(hs, T * k, n, "hs");
+    TORCH_CHECK(last_idx.has_value() == last_count.has_value(), n, ": last_idx and last_count go together");
+    if (last_idx) {
+        need(*last_idx, torch::kInt32, x, n, "last_idx");
+        need(*last_count, torch::kInt32, x, n, "last_count");
+        need_numel(*last_idx, k, n, "last_idx");
+        need_numel(*last_count, 1, n, "last_count");
+    }
     if (cached) {
         TORCH_CHECK(cache_up && cache_down && slot_of && image_up && image_down && mark && host_up && host_down, n,
                     ": the cached form needs every cache argument");
@@ -1741,7 +1750,8 @@ void prompt_mlp_dip_(int64_t T, int64_t k, torch::Tensor x, torch::Tensor norm, 
                  n);
     check_status(prompt_linear(gate_Wq, gate_scale, h16(h), gate, H, group_size, T, false, false, st), n);
     check_status(soi_dip_select_tokens(gate, ld, I, k, T, ip, cached ? mark->data_ptr<int32_t>() : nullptr,
-                                       static_cast<int32_t>(stamp), st),
+                                       static_cast<int32_t>(stamp), last_idx ? last_idx->data_ptr<int32_t>() : nullptr,
+                                       last_idx ? last_count->data_ptr<int32_t>() : nullptr, st),
                  n);
     const uint8_t* down = nullptr;
     if (cached) {
@@ -2024,7 +2034,8 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
           py::arg("group_size"), py::arg("eps"), py::arg("norm_pair"), py::arg("up_scale") = py::none(),
           py::arg("cache_up") = py::none(), py::arg("cache_down") = py::none(), py::arg("slot_of") = py::none(),
           py::arg("host_up") = 0, py::arg("host_down") = 0, py::arg("image_up") = py::none(),
-          py::arg("image_down") = py::none(), py::arg("mark") = py::none(), py::arg("stamp") = 0);
+          py::arg("image_down") = py::none(), py::arg("mark") = py::none(), py::arg("stamp") = 0,
+          py::arg("last_idx") = py::none(), py::arg("last_count") = py::none());
     m.def("quantize_group", &quantize_group, "symmetric group quantization: (codes, scales)");
     m.def("pack_int4", &pack_int4, "int8 codes to AWQ-order INT4 rows");
     m.def("transpose_int4", &transpose_int4, "the transpose of packed INT4 rows, packed");

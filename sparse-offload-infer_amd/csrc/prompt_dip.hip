@@ -21,10 +21,13 @@ constexpr int kSelMax = kSelThreads * 32;  // channels one workgroup holds in re
 
 // Workgroup t: the rule-A selection over |gate[t]| (topk_radix_kernel's partition), ascending, to idx[t, k]. mark: every
 // selected channel's word is set to `stamp`, so the union of the tokens' selections needs no clearing between calls.
+// last_idx, last_count: the last token's selection as the top-k kernel leaves it (nothing past the count is written).
 template <int E>
 __global__ __launch_bounds__(kSelThreads) void dip_select_tokens_kernel(const uint16_t* __restrict__ gate, int64_t ld,
                                                                         int n, int k, int32_t* __restrict__ idx,
-                                                                        int32_t* __restrict__ mark, int32_t stamp) {
+                                                                        int32_t* __restrict__ mark, int32_t stamp,
+                                                                        int32_t* __restrict__ last_idx,
+                                                                        int32_t* __restrict__ last_count) {
     __shared__ uint32_t s_hist[radix_hist_offset<F16AbsValues>(F16AbsValues::kPasses)];
     __shared__ float s_max[kSelWaves];
     __shared__ uint32_t s_tot[kSelWaves];
@@ -32,6 +35,7 @@ __global__ __launch_bounds__(kSelThreads) void dip_select_tokens_kernel(const ui
     const int base_i = wave * kWave * E + lane;
     const F16AbsValues v{gate + static_cast<int64_t>(blockIdx.x) * ld};
     int32_t* out = idx + static_cast<int64_t>(blockIdx.x) * k;
+    const bool last = last_idx != nullptr && blockIdx.x + 1 == gridDim.x;
     float val[E];
     uint32_t key[E];
     float local_max = 0.0f;
@@ -55,7 +59,9 @@ __global__ __launch_bounds__(kSelThreads) void dip_select_tokens_kernel(const ui
         const int c = base_i + j * kWave;
         stg(out + pos, c);
         if (mark) stg(mark + c, stamp);
+        if (last) stg(last_idx + pos, c);
     });
+    if (last && tid == 0) stg(last_count, static_cast<int32_t>(total < static_cast<uint32_t>(k) ? total : k));
     // fewer than k gates that are numbers: the rest of the list names no channel
     for (uint32_t i = total + static_cast<uint32_t>(tid); i < static_cast<uint32_t>(k); i += kSelThreads)
         stg(out + i, -1);
@@ -222,16 +228,18 @@ using namespace soi;
 extern "C" int64_t soi_dip_tokens_max_channels(void) { return kSelMax; }
 
 extern "C" int soi_dip_select_tokens(const uint16_t* gate, int64_t ld, int64_t n, int64_t k, int64_t T, int32_t* idx,
-                                     int32_t* mark, int32_t stamp, void* stream) {
+                                     int32_t* mark, int32_t stamp, int32_t* last_idx, int32_t* last_count,
+                                     void* stream) {
     const char* what = "soi_dip_select_tokens";
     SOI_REQUIRE(T >= 1 && T <= 65535, "%s: the token count must be in [1, 65535]", what);
     SOI_REQUIRE(n >= 1 && n <= kSelMax && ld >= n, "%s: n must be in [1, %d] and ld >= n", what, kSelMax);
     SOI_REQUIRE(k >= 1 && k <= n, "%s: k must be in [1, n]", what);
-    SOI_REQUIRE(gate && idx, "%s: null pointer", what);
+    SOI_REQUIRE(gate && idx && !last_idx == !last_count, "%s: null pointer, or one of last_idx and last_count", what);
     const int64_t e = ceil_div64(n, kSelThreads);
 #define SOI_S(EE)                                                                                                     \
     hipLaunchKernelGGL(dip_select_tokens_kernel<EE>, dim3(static_cast<unsigned>(T)), dim3(kSelThreads), 0,            \
-                       as_stream(stream), gate, ld, static_cast<int>(n), static_cast<int>(k), idx, mark, stamp)
+                       as_stream(stream), gate, ld, static_cast<int>(n), static_cast<int>(k), idx, mark, stamp,  \
+                       last_idx, last_count)
     if (e <= 1) SOI_S(1);
     else if (e <= 2) SOI_S(2);
     else if (e <= 4) SOI_S(4);

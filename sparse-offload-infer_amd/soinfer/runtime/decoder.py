@@ -610,13 +610,16 @@ class DecodeEngine:
     def _gated_down(self, l: int, L: LayerWeights, gate: torch.Tensor, hu: torch.Tensor,
                     res: Optional[torch.Tensor] = None, res_out: Optional[torch.Tensor] = None):
         """Selection + sparse down of the gated schedule. Over the transposed copy (hu = h of every channel) the
-        index list is written only for the eager consumers that read it, and with res_out the launch also writes
-        res + down there; over the selected rows (hu = up of every channel) h of the selected channels is formed
+        index list is written only for the eager consumers that read it and by the last layer of an engine without a named
+        schedule, and with res_out the launch also writes res + down there; over the selected rows (hu = up of every channel) h of the selected channels is formed
         on load, as the indexed up GEMV's SiLU epilogue rounds it."""
         c = self.c
         if self.dip_gated_tr:
             Wt, St = self.down_tt[l]
-            want = self.counts is not None or self.layer_hook is not None
+            # without a named schedule a step leaves the last layer's idx and cnt, as the indexed launches do (the list
+            # takes 1.9 us to write, so the layers whose list the next one replaces leave it out)
+            want = self.counts is not None or self.layer_hook is not None or \
+                (self._gated_auto and l == c.layers - 1)
             _C.dip_select_down_ordered_into(gate, hu, self.k, Wt, St, self.idx if want else None,
                                             self.cnt if want else None, self.down, c.group_size,
                                             res if res_out is not None else None, res_out)
@@ -902,7 +905,7 @@ class DecodeEngine:
         args = (T, self.k, b["x"], L.post_norm, b["h"])
         if self.mode == "dip":
             _C.prompt_mlp_dip_(*args, L.gu_Wq, L.gu_scale, b["gu"], b["idx"], b["hs"], L.down_T_Wq, L.down_T_scale, gs,
-                               eps, self.dip_gated)
+                               eps, self.dip_gated, last_idx=self.idx, last_count=self.cnt)
             if self.counts is not None:
                 add_selection_counts(self.counts[l], b["idx"][:T * self.k])
             return
@@ -911,7 +914,7 @@ class DecodeEngine:
         _C.prompt_mlp_dip_(*args, *L.gate(I), b["gu"], b["idx"], b["hs"], None, L.down_T_scale, gs, eps, False,
                            up_scale=L.up(I)[1], cache_up=cache.up_Wq, cache_down=cache.down_Wq, slot_of=cache.slot_of,
                            host_up=self.host_up_ptr[l], host_down=self.host_down_ptr[l], image_up=up, image_down=down,
-                           mark=b["mark"], stamp=self._prompt_stamp)
+                           mark=b["mark"], stamp=self._prompt_stamp, last_idx=self.idx, last_count=self.cnt)
 
     def _prompt_layers(self, tokens: torch.Tensor):
         """Every layer over the given tokens at positions pos, pos + 1, ... (device int32), then the final norm of

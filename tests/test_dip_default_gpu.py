@@ -43,3 +43,35 @@ def test_default_equals_indexed(cuda, name):
         e.layer_hook = None
     for x, y in zip(seen[id(a)], seen[id(b)]):
         assert all(torch.equal(p, q) for p, q in zip(x, y))
+
+
+@pytest.mark.parametrize("name", ["ordered", "one_pass", "row_form_only"])
+def test_selection_of_the_latest_step_is_readable(cuda, name):
+    """idx and cnt after prompts, single steps and graph replays are the indexed schedule's."""
+    from soinfer.runtime import decoder as D
+
+    kw, k, _ = CONFIGS[name]
+    w = D.random_decoder(D.DecoderConfig(layers=2, vocab=700, max_seq=400, **kw), seed=5, linear_std=0.05,
+                         norm_jitter=0.1)
+    a = D.DecodeEngine(w, "dip", dip_k=k, max_new_tokens=6)
+    b = D.DecodeEngine(w, "dip", dip_k=k, max_new_tokens=6, dip_schedule="indexed")
+    cached = D.DecodeEngine(w, "cached_dip", dip_k=k, max_new_tokens=6,
+                            hot_channels=[list(range(0, kw["intermediate"], 3))] * 2)
+    prompt = torch.randint(0, 700, (9,), generator=torch.Generator().manual_seed(3)).tolist()
+
+    def same(what):
+        assert torch.equal(a.idx, b.idx) and torch.equal(a.cnt, b.cnt), what
+        assert torch.equal(cached.idx, b.idx) and torch.equal(cached.cnt, b.cnt), what
+
+    for e in (a, b, cached):
+        e.reset()
+    b._prompt_together = lambda *_: False
+    for e in (a, b, cached):
+        e.prefill(prompt, use_graph=False)
+    same("prompt")
+    for e in (a, b, cached):
+        e.decode(1, use_graph=False)
+    same("one step")
+    for e in (a, b, cached):
+        e.generate(prompt, 6)
+    same("generate")

@@ -225,9 +225,10 @@ def test_selection_of_gates_that_are_not_numbers(cuda, n, k):
     gate[2, numbers] = kept
     idx = torch.full((4, k), 12345678, dtype=torch.int32, device=cuda)
     mark = torch.zeros(n, dtype=torch.int32, device=cuda)
-    ptr = [ctypes.c_void_p(t.data_ptr()) for t in (gate, idx, mark)]
+    last = [torch.full((s,), 77, dtype=torch.int32, device=cuda) for s in (k, 1)]
+    ptr = [ctypes.c_void_p(t.data_ptr()) for t in (gate, idx, mark, *last)]
     st = hip_lib().soi_dip_select_tokens(ptr[0], *(ctypes.c_int64(v) for v in (n, n, k, 4)), ptr[1], ptr[2],
-                                         ctypes.c_int32(9), ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+                                         ctypes.c_int32(9), *ptr[3:], ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
     assert st == 0
     from soinfer import ops
 
@@ -239,6 +240,11 @@ def test_selection_of_gates_that_are_not_numbers(cuda, n, k):
     for t in (0, 2, 3):
         named[idx[t][idx[t] >= 0].long()] = True
     assert torch.equal(mark == 9, named)
+    assert torch.equal(last[0], idx[3]) and int(last[1]) == k
+    st = hip_lib().soi_dip_select_tokens(ptr[0], *(ctypes.c_int64(v) for v in (n, n, k, 3)), ptr[1], None,
+                                         ctypes.c_int32(0), *ptr[3:], ctypes.c_void_p(torch.cuda.current_stream().cuda_stream))
+    assert st == 0 and int(last[1]) == m
+    assert torch.equal(last[0][:m].long(), numbers) and torch.equal(last[0][m:], idx[3, m:]), "nothing past the count"
 
 
 def test_calibration_counts_of_a_token_without_numbers(dec, weights):
