@@ -731,6 +731,8 @@ int soi_gemv_w4a16_pair(const uint8_t* Wq0, const float* scale0, int64_t N0, con
                         uint32_t* clear, int64_t clear_words, void* stream);
 /* Arrival-counter words at the start of a soi_sparse_accumulate workspace (the part that must start at zero). */
 int64_t soi_sparse_accumulate_counter_words(int64_t H);
+/* Row chunks of the sparse accumulate's partition of k rows of H columns. */
+int64_t soi_sparse_accumulate_row_chunks(int64_t H, int64_t k);
 
 #ifdef __cplusplus
 }

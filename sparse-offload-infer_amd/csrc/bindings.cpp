@@ -2027,6 +2027,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("norm_gemv_one_pass",
           [](int64_t N, int64_t K, int64_t gs, bool swiglu) { return soi_norm_gemv_one_pass(N, K, gs, swiglu ? 1 : 0) != 0; },
           "whether the RMSNorm-fused GEMV of [N, K] rows takes the one-pass norm partition");
+    m.def("sparse_accumulate_row_chunks", &soi_sparse_accumulate_row_chunks, "row chunks of the sparse down's partition");
     m.def("dip_tokens_max_channels", &soi_dip_tokens_max_channels, "most channels prompt_mlp_dip_ selects from");
     m.def("prompt_mlp_dip_", &prompt_mlp_dip_, "one layer's DIP MLP over T tokens, added to x", py::arg("T"),
           py::arg("k"), py::arg("x"), py::arg("norm"), py::arg("h"), py::arg("gate_Wq"), py::arg("gate_scale"),

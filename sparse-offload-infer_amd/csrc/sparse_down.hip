@@ -285,6 +285,10 @@ using namespace soi;
 
 extern "C" int64_t soi_sparse_accumulate_counter_words(int64_t H) { return H > 0 ? down_plan(H, 1).S : 0; }
 
+extern "C" int64_t soi_sparse_accumulate_row_chunks(int64_t H, int64_t k) {
+    return H > 0 && k > 0 ? down_plan(H, k).R : 0;
+}
+
 extern "C" size_t soi_sparse_accumulate_workspace_bytes(int64_t H, int64_t k) { return down_workspace_bytes(H, k); }
 
 extern "C" int soi_gemv_w4a16_sparse_accumulate(const uint8_t* Wq_sel, const float* scale_sel, const uint16_t* h_sel,

@@ -212,6 +212,33 @@ def decoder_weights_from_arena(store, matrices, config: DecoderConfig, embed: to
     return DecoderWeights(config, embed, lm_head, final_norm, layers)
 
 
+def prompt_tokens_from(c: DecoderConfig, mode: str, k: Optional[int], context: int, resident: Optional[int] = None,
+                       offload: bool = False) -> float:
+    """Fewest prompt tokens that go through the layers together at `context` earlier tokens (a DIP engine with k channels,
+    of which `resident` rows are cached; offload: the dense weights are streamed).
+
+    Microseconds a layer of T tokens, fitted to 934 measured pairs (10 shapes, 3 to 24 tokens, contexts 0 to 30000; the
+    choice is within 0.3% of the faster one on average): one at a time T (single + step), together once + 2 chunks + 7e-5
+    head_dim context. `single`: the launches of a step, its weights and, for DIP, its selection over I gates; `once`: the
+    launches and weights of all tokens. What grows faster together: a token's workgroup walks the down's row chunks and
+    the context's splits one after another, where a step spreads them over the chip. 4 layers of 2048 x 6144: dense, 3 tokens at context 0 / 4000 / 16000 together 229 / 399 /
+    826 us, one at a time 306 / 398 / 497; 256 x 6144 DIP, k/I 0.3 (58 chunks), 3 / 5 / 8 tokens 658 / 685 / 692 against
+    368 / 580 / 905. Two tokens are faster one at a time wherever measured."""
+    H, I, kv = c.hidden, c.intermediate, c.kv_heads
+    attn = H * (c.q_heads + kv) * c.head_dim  # INT4 bytes of a layer
+    cached = mode == "cached_dip"
+    weights = attn + (H * (I + 2 * (k or 0)) // 2 if cached else 3 * H * I // 2)
+    missed = H * k * (1.0 - (resident or 0) / I) if cached else 0.0  # bytes a token reads from the host
+    streamed = attn + (H * I // 2 if cached else 3 * H * I // 2) if offload else 0
+    host = (missed + streamed) / 57e3
+    single = 23 + weights / 4e6 + (0.9e-3 * I if mode != "dense" else 0) + (8 if cached else 0) + host
+    once = 52 + weights / 2.2e6 + (20 if cached else 0) + host
+    chunks = _C.sparse_accumulate_row_chunks(H, k) if mode != "dense" else 0
+    # a step's attention: its splits' passes, the states that the workgroups of a KV head combine, the K and V bytes
+    step = (1e-4 + 2e-3 / kv + 4 * kv * c.head_dim / 6e6) * context
+    return max(3.0, (once + 2 * chunks + 7e-5 * c.head_dim * context) / (single + step))
+
+
 def default_gated_form(H: int, I: int, k: int) -> Optional[str]:
     """The MLP launches of a resident DIP engine without a named schedule: "ordered" (selection and down over the
     transposed down_proj^T), "rows" (selection and gated sparse down over the selected rows), or None, the indexed ones.
@@ -401,6 +428,7 @@ class DecodeEngine:
         if offload:
             self._setup_offload()
         self._x_final = self.x
+        self._context = 0  # tokens behind the device position, as prefill and decode have counted them (it only decides speed)
         self._prompt_buf = None  # scratch of _prompt_layers, made by the first prompt
         # the token kernels read every row 16 bytes at a time; of the matrices that the steps take from any address, the
         # o and down rows are the caller's (streamed ones lie in the slots, cached down^T rows in the images)
@@ -846,19 +874,25 @@ class DecodeEngine:
     def reset(self):
         self.pos.zero_()
         self.log_len.zero_()
+        self._context = 0
         self._step_open = False
 
     # ---- prompts ----
     def _prompt_together(self, n: int) -> bool:
         """Whether n prompt tokens go through the layers together (_prompt_layers) instead of one at a time: fused
-        layers within the token kernels' limits, and nothing that watches single steps. Two tokens are faster one at
-        a time (1.14 against 1.29 ms, three 1.70 against 1.29)."""
+        layers within the token kernels' limits, nothing that watches single steps, and enough tokens to be faster
+        (prompt_tokens_from). The results are the same either way, but for dense prompts of PROMPT_MFMA tokens up, which
+        always go together."""
         c = self.c
         if self.mode != "dense" and (self.dip_dense_up or c.intermediate > _C.dip_tokens_max_channels()):
             return False  # the dense-up schedule's down sums in an order of its own
         if self.counts is not None and self.mode == "cached_dip":
             return False
-        return n > 2 and self.fused and self.layer_hook is None and \
+        resident = self.caches[0].cache_size if self.mode == "cached_dip" else None
+        if n < 3 or n < (PROMPT_MFMA if self.mode == "dense" else 1 << 30) and \
+                n < prompt_tokens_from(c, self.mode, getattr(self, "k", None), self._context, resident, self.offload):
+            return False
+        return self.fused and self.layer_hook is None and \
             c.hidden % 32 == 0 and c.intermediate % 32 == 0 and c.q_heads * c.head_dim % 32 == 0 and \
             c.group_size % 32 == 0 and self._prompt_aligned and \
             bool(_C.attention_tokens_supported(c.q_heads, c.kv_heads, c.head_dim, c.max_seq))
@@ -941,7 +975,9 @@ class DecodeEngine:
         prompt = torch.as_tensor(list(prompt_ids), dtype=torch.int32, device=self.device)
         if prompt.numel() + 1 > self.c.max_seq:
             raise ValueError("prompt longer than the KV cache")
-        if self._prompt_together(prompt.numel()):
+        together = self._prompt_together(prompt.numel())
+        self._context += prompt.numel()
+        if together:
             for part in prompt.split(PROMPT_CHUNK):
                 self._prompt_layers(part)
             self.token.copy_(prompt[-1:])
@@ -956,6 +992,7 @@ class DecodeEngine:
     def decode(self, n_new: int, use_graph: bool = True):
         if n_new > self.log.numel():
             raise ValueError("n_new exceeds max_new_tokens")
+        self._context += n_new
         if not use_graph:
             for _ in range(n_new):
                 self._gen_step()

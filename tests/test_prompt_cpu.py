@@ -34,3 +34,38 @@ def test_default_dip_launches(shape, form):
     from soinfer.runtime.decoder import default_gated_form
 
     assert default_gated_form(*shape) == form
+
+
+def config(H, I, nq, nkv, hd):
+    from soinfer.runtime.decoder import DecoderConfig
+
+    return DecoderConfig(hidden=H, layers=1, q_heads=nq, kv_heads=nkv, head_dim=hd, intermediate=I, vocab=10,
+                         group_size=128, max_seq=64)
+
+
+# shape, mode, k, context, tokens measured faster one at a time, tokens measured faster together
+MEASURED = [((2048, 6144, 16, 8, 128), "dense", None, 0, 2, 3), ((2048, 6144, 16, 8, 128), "dense", None, 8000, 3, 4),
+            ((2048, 6144, 16, 8, 128), "dense", None, 30000, 5, 8), ((1024, 3072, 8, 1, 64), "dense", None, 30000, 2, 3),
+            ((256, 6144, 4, 2, 64), "dip", 1843, 0, 5, 8), ((512, 1024, 4, 2, 64), "dip", 972, 0, 3, 5),
+            ((1024, 12288, 16, 8, 128), "dip", 3686, 0, 2, 3), ((1024, 12288, 16, 8, 128), "dip", 7372, 0, 3, 4),
+            ((2048, 6144, 16, 8, 128), "dip", 3072, 30000, 5, 8), ((512, 1024, 4, 2, 64), "cached_dip", 614, 0, 2, 4),
+            ((256, 6144, 4, 2, 64), "cached_dip", 3686, 0, 3, 5)]
+
+
+@pytest.mark.parametrize("shape,mode,k,context,apart,together", MEASURED)
+def test_prompt_route(shape, mode, k, context, apart, together):
+    from soinfer.runtime.decoder import prompt_tokens_from
+
+    n = prompt_tokens_from(config(*shape), mode, k, context, shape[1] // 3 if mode == "cached_dip" else None)
+    assert apart < n <= together
+
+
+def test_dense_prompts_on_the_matrix_cores_are_never_split_by_the_context():
+    """Nine dense tokens up take one route whatever the context (their bits differ from the single steps'), and for head
+    sizes up to 128 the estimate agrees."""
+    from soinfer.runtime import decoder as D
+
+    for shape in ((256, 512, 4, 2, 64), (2048, 6144, 16, 16, 128), (5120, 17408, 40, 8, 128)):
+        assert D.prompt_tokens_from(config(*shape), "dense", None, 10 ** 7) <= D.PROMPT_MFMA
+    # streamed weights cross the link once for all tokens together
+    assert D.prompt_tokens_from(config(2048, 6144, 16, 8, 128), "dense", None, 10 ** 5, offload=True) == 3.0

@@ -313,3 +313,31 @@ def test_prompt_over_rows_off_16_bytes(cuda, dec, weights, mode, name):
     for use_graph in (False, True):
         assert a.generate(prompt, 3, use_graph=use_graph) == b.generate(prompt, 3, use_graph=use_graph)
         same_state(a, b, 10, f"{mode} {name}")
+
+
+def test_short_prompts_behind_a_context(cuda, dec, weights):
+    """The engine counts the tokens behind it, and a short prompt's state is the single steps' on either route."""
+    c = weights.config
+    for mode, kw in (("dense", {}), ("dip", dict(dip_k=c.intermediate // 2))):
+        a = dec.DecodeEngine(weights, mode, max_new_tokens=4, **kw)
+        b = dec.DecodeEngine(weights, mode, max_new_tokens=4, **kw)
+        a.generate(tokens(5, c.vocab, 1), 3)
+        assert a._context == int(a.pos) == 8
+        for e in (a, b):
+            e.reset()
+        total = 0
+        for n, apart in ((3, False), (4, True), (2, False), (5, False), (3, True)):
+            part = tokens(n, c.vocab, total)
+            assert a._prompt_together(n) == (n > 2)
+            if apart:
+                a._prompt_together = lambda *_: False
+            a.prefill(part, use_graph=a._graph_layers is not None)
+            a.__dict__.pop("_prompt_together", None)
+            one_at_a_time(b, part)
+            total += n
+            same_state(a, b, total, f"{mode}, {total} tokens")
+            assert a._context == int(a.pos) == total
+        a.decode(2)
+        assert a._context == int(a.pos) == total + 2
+        a._context = 1 << 30
+        assert mode == "dip" or a._prompt_together(9)
