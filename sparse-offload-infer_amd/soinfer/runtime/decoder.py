@@ -878,20 +878,23 @@ class DecodeEngine:
         self._step_open = False
 
     # ---- prompts ----
-    def _prompt_together(self, n: int) -> bool:
+    def _prompt_together(self, n: int, use_graph: bool = True) -> bool:
         """Whether n prompt tokens go through the layers together (_prompt_layers) instead of one at a time: fused
-        layers within the token kernels' limits, nothing that watches single steps, and enough tokens to be faster
-        (prompt_tokens_from). The results are the same either way, but for dense prompts of PROMPT_MFMA tokens up, which
+        layers within the token kernels' limits, nothing that watches single steps, and enough tokens to be faster than
+        replays of the captured step (prompt_tokens_from; than eager steps three are). The results are the same either way, but for dense prompts of PROMPT_MFMA tokens up, which
         always go together."""
         c = self.c
         if self.mode != "dense" and (self.dip_dense_up or c.intermediate > _C.dip_tokens_max_channels()):
             return False  # the dense-up schedule's down sums in an order of its own
         if self.counts is not None and self.mode == "cached_dip":
             return False
-        resident = self.caches[0].cache_size if self.mode == "cached_dip" else None
-        if n < 3 or n < (PROMPT_MFMA if self.mode == "dense" else 1 << 30) and \
-                n < prompt_tokens_from(c, self.mode, getattr(self, "k", None), self._context, resident, self.offload):
+        if n < 3:
             return False
+        if use_graph and self._graph_layers is not None and not (self.mode == "dense" and n >= PROMPT_MFMA):
+            resident = self.caches[0].cache_size if self.mode == "cached_dip" else None
+            if n < prompt_tokens_from(c, self.mode, None if self.mode == "dense" else self.k, self._context, resident,
+                                      self.offload):
+                return False
         return self.fused and self.layer_hook is None and \
             c.hidden % 32 == 0 and c.intermediate % 32 == 0 and c.q_heads * c.head_dim % 32 == 0 and \
             c.group_size % 32 == 0 and self._prompt_aligned and \
@@ -975,7 +978,7 @@ class DecodeEngine:
         prompt = torch.as_tensor(list(prompt_ids), dtype=torch.int32, device=self.device)
         if prompt.numel() + 1 > self.c.max_seq:
             raise ValueError("prompt longer than the KV cache")
-        together = self._prompt_together(prompt.numel())
+        together = self._prompt_together(prompt.numel(), use_graph)
         self._context += prompt.numel()
         if together:
             for part in prompt.split(PROMPT_CHUNK):

@@ -328,7 +328,7 @@ def test_short_prompts_behind_a_context(cuda, dec, weights):
         total = 0
         for n, apart in ((3, False), (4, True), (2, False), (5, False), (3, True)):
             part = tokens(n, c.vocab, total)
-            assert a._prompt_together(n) == (n > 2)
+            assert a._prompt_together(n, a._graph_layers is not None) == (n > 2)
             if apart:
                 a._prompt_together = lambda *_: False
             a.prefill(part, use_graph=a._graph_layers is not None)
@@ -341,3 +341,7 @@ def test_short_prompts_behind_a_context(cuda, dec, weights):
         assert a._context == int(a.pos) == total + 2
         a._context = 1 << 30
         assert mode == "dip" or a._prompt_together(9)
+        assert a._prompt_together(3, use_graph=False), "eager steps are slower"
+    b.reset()
+    b.prefill(tokens(3, c.vocab, 7))  # no graph captured
+    assert int(b.pos) == 3
