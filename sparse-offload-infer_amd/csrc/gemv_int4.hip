@@ -389,12 +389,18 @@ static int launch_int4(const Rows& rows, int64_t N, const uint16_t* x, const EP&
     if (N == 0) return SOI_OK;
     const int vec = aligned ? kAligned : K >= 32 ? kAnyAlign : kScalar;
     Int4Plan pl = plan_int4(N, K, vec);
-    // rows of more than 3 passes, over more than 2048 rows: 4 rows per wave (2560 x 9728 6.34 against 6.35 us with 2,
-    // 4096 x 12288 8.0 against 8.3, 5120 x 17408 14.5 against 14.9, 8192 x 8192 9.6 against 10.7, cold copies); rows of
-    // 2 or 3 passes stay at 2 (4096 x 4096 3.9 against 4.2 us with 4, 5120 x 5120 5.7 against 6.3, 2048 x 6144 3.8
-    // against 4.0)
-    const int64_t passes = ceil_div64(ceil_div64(ceil_div64(K, 8), 4), kWave);
-    if (pl.PU > 1 && N > 2 * 1024 && (passes > 3 || vec != kAligned)) pl.R = 4;
+    // rows of several passes, over more than 2048 rows: 2 or 4 rows per wave (us, cold copies, 2 rows / 4 rows). More than
+    // 3 passes: 4 (4096 x 12288 8.3 / 8.0, 5120 x 17408 14.9 / 14.5, 8192 x 8192 10.7 / 9.6). 2 passes, or 3 whole ones:
+    // 2 below 8192 rows, where the finer tiles even out the last round of waves (5120 x 3072 4.71 / 5.06, 5120 x 4096
+    // 4.70 / 5.03, 5120 x 6144 5.81 / 6.08), 4 from there, where the extra waves are a round of their own (12288 x 2560
+    // 7.56 / 6.77, 12288 x 6144 9.62 / 9.03, 17408 x 2560 9.37 / 8.86). 3 passes with a part: 4 up to 4096 rows and from
+    // 24576 (4096 x 5120 5.13 / 5.00, 24576 x 5120 4% apart), 2 between (5120 x 5120 5.98 / 6.50, 17408 x 5120 12.2 / 12.8)
+    const int64_t chunks = ceil_div64(ceil_div64(K, 8), 4), passes = ceil_div64(chunks, kWave);
+    if (pl.PU > 1 && N > 2 * 1024) {
+        const bool part = passes == 3 && chunks % kWave != 0;
+        const bool two = vec == kAligned && passes <= 3 && (part ? N > 4096 && N < 24576 : N < 8192);
+        if (!two) pl.R = 4;
+    }
     const bool cs = (gs % 32) == 0;
     const bool full = aligned && cs && (N % pl.R == 0) && ((K / 32) % (64 * pl.PU) == 0);
     const dim3 grid(static_cast<unsigned>(ceil_div64(N, pl.R)));

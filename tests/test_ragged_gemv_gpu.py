@@ -79,3 +79,18 @@ def test_int8(ops, N, K, gs):
     assert all(torch.equal(y, want) for y in ops.Int8Batch([q, q.clone()], [s, s], [x, x.clone()], gs).run())
     one = s[:, :1].contiguous()  # one scale per row
     assert torch.equal(ops.gemv_w8a16(q, one, x, K), ops.gemv_w8a16(qp, one, xp, P))
+
+
+@pytest.mark.parametrize("K", [2560, 4096, 5120, 6144, 8192])
+@pytest.mark.parametrize("N", [2049, 4096, 4100, 8191, 8192, 8198, 24575, 24577])
+def test_int4_rows_per_wave(ops, N, K):
+    """Every line of the rows-per-wave rule (2 and 4 rows, their remainders): a row's result does not depend on its tile,
+    so it is the one-row tile's of the same rows in matrices of under 2048."""
+    from soinfer.quant import pack
+
+    q, s, x = codes(N, K, 128, 4, N + K)
+    W = pack.pack_int4(q)[0]
+    got = ops.gemv_w4a16_group_lop3(W, s, x, K, 128)
+    for r in range(0, N, 1024):
+        part = slice(r, min(N, r + 1024))
+        assert torch.equal(got[part], ops.gemv_w4a16_group_lop3(W[part], s[part], x, K, 128))
