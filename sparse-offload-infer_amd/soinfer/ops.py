@@ -273,13 +273,13 @@ def transposed_down_T(Wq_T: torch.Tensor, scale_T: torch.Tensor, H: int) -> tupl
     """The same quantized down_proj^T values laid out for dip_select_dense_down: Wq_T [n, ceil(H/8)*4] packed
     rows (channel c's H nibbles) -> Wt [H, n/2] (output column col's n nibbles, packed like every INT4 row,
     n % 8 == 0), scale_T [n, G] -> St [G, n]. No rounding: Wt unpacks to the transpose of Wq_T's values."""
-    from soinfer.quant import pack
+    from soinfer.quant import _device, pack
 
     n = Wq_T.shape[0]
     if n % 8:
         raise ValueError("transposed_down_T: the channel count must be a multiple of 8")
-    if Wq_T.is_cuda and Wq_T.dtype == torch.uint8 and Wq_T.is_contiguous() and Wq_T.data_ptr() % 4 == 0 and n and \
-            Wq_T.dim() == 2 and Wq_T.shape[1] == -(-H // 8) * 4:
+    if _device.takes_kernel(Wq_T) and Wq_T.dtype == torch.uint8 and Wq_T.is_contiguous() and \
+            Wq_T.data_ptr() % 4 == 0 and Wq_T.dim() == 2 and Wq_T.shape[1] == -(-H // 8) * 4 and n < 1 << 22:
         return _C.transpose_int4(Wq_T, H), scale_T.t().contiguous()
     q = pack.unpack_int4(Wq_T, H)  # int8 [n, H]
     Wt, _ = pack.pack_int4(q.t().contiguous())

@@ -88,3 +88,32 @@ def test_transposed_rows(cuda, n, H):
     got, gs = ops.transposed_down_T(W.to(cuda), s.to(cuda), H)
     same(got, pack.pack_int4(q.t().contiguous())[0])
     same(gs, s.t().contiguous())
+
+
+def test_negative_views_and_modes(cuda):
+    """A negative view (its negation still to be done) and calls under a dispatch mode take the expressions."""
+    from torch.utils._python_dispatch import TorchDispatchMode
+
+    from soinfer import ops
+    from soinfer.quant import formats, pack
+
+    cfg = formats.QuantConfig(4, "group", 64)
+    w = torch.randn(4, 128, device=cuda, generator=torch.Generator(device=cuda).manual_seed(5))
+    want, got = formats.quantize(-w, cfg), formats.quantize(torch._neg_view(w), cfg)
+    same(got.qweight, want.qweight)
+    same(got.scale, want.scale)
+    q = torch.randint(-8, 8, (64, 128), generator=torch.Generator().manual_seed(6), dtype=torch.int8).to(cuda)
+    same(pack.pack_int4(torch._neg_view(q))[0], pack.pack_int4(-q)[0])
+
+    class Seen(TorchDispatchMode):
+        ops = 0
+
+        def __torch_dispatch__(self, func, types, args=(), kwargs=None):
+            Seen.ops += 1
+            return func(*args, **(kwargs or {}))
+
+    W, s = pack.pack_int4(q)[0], torch.rand(64, 1, device=cuda)
+    want = ops.transposed_down_T(W, s, 128)
+    with Seen():
+        got = ops.transposed_down_T(W, s, 128)
+    assert Seen.ops > 5 and all(torch.equal(a, b) for a, b in zip(got, want))
