@@ -115,7 +115,7 @@ def test_cached_dip_bit_identical_to_dip(dec, tiny, fused, miss_path):
     cfg = tiny.config
     k = cfg.intermediate // 2
     prompt = prompt_ids(6, cfg.vocab, seed=5)
-    plain = dec.DecodeEngine(tiny, "dip", dip_k=k, max_new_tokens=6, fused=fused)
+    plain = dec.DecodeEngine(tiny, "dip", dip_k=k, max_new_tokens=6, fused=fused, dip_schedule="indexed")
     want = plain.generate(prompt, 6, use_graph=True)
     calib = prompt_ids(16, cfg.vocab, seed=1000)
     hot20 = dec.calibrate_hot_channels(tiny, k, calib, cache_fraction=0.2)
@@ -145,7 +145,7 @@ def test_dip_dense_up_schedule(dec, tiny, fused):
     cfg = tiny.config
     k = cfg.intermediate // 2
     prompt = prompt_ids(6, cfg.vocab, seed=9)
-    plain = dec.DecodeEngine(tiny, "dip", dip_k=k, max_new_tokens=6, fused=fused)
+    plain = dec.DecodeEngine(tiny, "dip", dip_k=k, max_new_tokens=6, fused=fused, dip_schedule="indexed")
     want = plain.generate(prompt, 6, use_graph=True)
     eng = dec.DecodeEngine(tiny, "dip", dip_k=k, max_new_tokens=6, fused=fused, dip_dense_up=True)
     got = eng.generate(prompt, 6, use_graph=False)
@@ -170,7 +170,7 @@ def test_dip_gated_schedule_bit_identical_to_indexed(dec, tiny, fused, ordered):
     cfg = tiny.config
     k = cfg.intermediate // 2
     prompt = prompt_ids(6, cfg.vocab, seed=19)
-    plain = dec.DecodeEngine(tiny, "dip", dip_k=k, max_new_tokens=6, fused=fused)
+    plain = dec.DecodeEngine(tiny, "dip", dip_k=k, max_new_tokens=6, fused=fused, dip_schedule="indexed")
     want = plain.generate(prompt, 6, use_graph=True)
     eng = dec.DecodeEngine(tiny, "dip", dip_k=k, max_new_tokens=6, fused=fused, dip_schedule="gated")
     assert eng.dip_gated_tr  # this shape fits the ordered down
@@ -193,7 +193,7 @@ def test_offloaded_dense_weights_bit_identical(dec, fused):
     prompt = prompt_ids(6, cfg.vocab, seed=21)
     dense = dec.DecodeEngine(tiny, "dense", max_new_tokens=6, fused=fused)
     want_dense = dense.generate(prompt, 6, use_graph=True)
-    dip = dec.DecodeEngine(tiny, "dip", dip_k=k, max_new_tokens=6, fused=fused)
+    dip = dec.DecodeEngine(tiny, "dip", dip_k=k, max_new_tokens=6, fused=fused, dip_schedule="indexed")
     want_dip = dip.generate(prompt, 6, use_graph=True)
     hot = [list(range(0, cfg.intermediate, 4)) for _ in range(cfg.layers)]
     cases = (("dense", dense, want_dense, dict()),

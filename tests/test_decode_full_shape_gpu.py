@@ -43,7 +43,7 @@ def setup(cuda):
 
 def _engines(D, w, hot):
     return {
-        "dip": D.DecodeEngine(w, "dip", dip_k=DIP_K, max_new_tokens=N_NEW),
+        "dip": D.DecodeEngine(w, "dip", dip_k=DIP_K, max_new_tokens=N_NEW, dip_schedule="indexed"),
         "dip_dense_up": D.DecodeEngine(w, "dip", dip_k=DIP_K, max_new_tokens=N_NEW, dip_dense_up=True),
         "dip_gated": D.DecodeEngine(w, "dip", dip_k=DIP_K, max_new_tokens=N_NEW, dip_schedule="gated"),
         "cached_direct": D.DecodeEngine(w, "cached_dip", dip_k=DIP_K, hot_channels=hot, max_new_tokens=N_NEW),
@@ -169,11 +169,11 @@ def _prompt5(V):
 
 def test_config5_full_length_cached_dip_equals_dip(setup):
     """64 + 128 tokens through 28 layers: cache-aware DIP (20% calibrated hot cache, misses from pinned host
-    memory, direct and staged) and the gated DIP schedule generate DIP's tokens and end with its final hidden
-    state, bit for bit."""
+    memory, direct and staged), the gated DIP schedule and an engine without a named one generate indexed DIP's tokens and
+    end with its final hidden state, bit for bit."""
     D, w, _, hot = setup
     prompt = _prompt5(w.config.vocab)
-    dip = D.DecodeEngine(w, "dip", dip_k=DIP_K, max_new_tokens=N_NEW5)
+    dip = D.DecodeEngine(w, "dip", dip_k=DIP_K, max_new_tokens=N_NEW5, dip_schedule="indexed")
     want = dip.generate(prompt, N_NEW5)
     x_ref = dip.x_final.clone()
     assert len(want) == N_PROMPT5 + N_NEW5 and int(dip.pos.item()) == N_PROMPT5 + N_NEW5
@@ -184,10 +184,12 @@ def test_config5_full_length_cached_dip_equals_dip(setup):
         assert got == want, f"cached DIP ({path}): tokens differ from DIP"
         assert torch.equal(eng.x_final, x_ref), f"cached DIP ({path}): final hidden state differs from DIP"
         del eng
-    # the two-launch gated schedule: the same tokens and final hidden state as well
-    eng = D.DecodeEngine(w, "dip", dip_k=DIP_K, max_new_tokens=N_NEW5, dip_schedule="gated")
-    assert eng.generate(prompt, N_NEW5) == want, "gated DIP: tokens differ from DIP"
-    assert torch.equal(eng.x_final, x_ref), "gated DIP: final hidden state differs from DIP"
+    # the two-launch gated schedule and an engine without a named one: the same tokens and final hidden state as well
+    for schedule in ("gated", None):
+        eng = D.DecodeEngine(w, "dip", dip_k=DIP_K, max_new_tokens=N_NEW5, dip_schedule=schedule)
+        assert eng.generate(prompt, N_NEW5) == want, f"{schedule} DIP: tokens differ from DIP"
+        assert torch.equal(eng.x_final, x_ref), f"{schedule} DIP: final hidden state differs from DIP"
+        del eng
 
 
 def test_config5_last_step_per_layer_matches_oracle(setup):
@@ -201,7 +203,8 @@ def test_config5_last_step_per_layer_matches_oracle(setup):
 
     c = w.config
     I, H, gs, NQ, NKV, hd = c.intermediate, c.hidden, c.group_size, c.q_heads, c.kv_heads, c.head_dim
-    eng = D.DecodeEngine(w, "dip", dip_k=DIP_K, max_new_tokens=N_NEW5, defer_attention_combine=False)
+    eng = D.DecodeEngine(w, "dip", dip_k=DIP_K, max_new_tokens=N_NEW5, defer_attention_combine=False,
+                         dip_schedule="indexed")
     eng.capture()
     eng.reset()
     eng.prefill(_prompt5(c.vocab))

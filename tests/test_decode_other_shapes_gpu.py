@@ -14,8 +14,8 @@ tested here):
   on the kernel's own h within the per-element bound, and the MLP output within 1e-3 (normalized) of the
   oracle's DIP MLP on the same input (free-running DIP logits are not compared: one |gate| at the selection
   boundary rounded to the other binary16 neighbour swaps a channel and moves the logits past any tight bound);
-* over a 300-token context (split attention), the gated DIP schedule and cache-aware DIP (a calibrated 20% hot
-  cache, misses read from pinned host memory) give DIP's tokens and final hidden state bit for bit, eager and
+* over a 300-token context (split attention), the gated DIP schedule, an engine without a named schedule and
+  cache-aware DIP (a calibrated 20% hot cache, misses read from pinned host memory) give indexed DIP's tokens and final hidden state bit for bit, eager and
   graph replays.
 """
 import numpy as np
@@ -89,14 +89,15 @@ def test_gated_and_cached_dip_bit_identical_to_dip(dec, model):
     cfg = w.config
     k = cfg.intermediate // 2
     prompt = prompt_ids(300, cfg.vocab, seed=23)
-    plain = dec.DecodeEngine(w, "dip", dip_k=k, max_new_tokens=4)
+    plain = dec.DecodeEngine(w, "dip", dip_k=k, max_new_tokens=4, dip_schedule="indexed")
     want = plain.generate(prompt, 4, use_graph=True)
     assert plain.defer_combine == (cfg.q_heads * cfg.head_dim <= 2048), name
     gated = dec.DecodeEngine(w, "dip", dip_k=k, max_new_tokens=4, dip_schedule="gated")
     assert gated.dip_gated_tr, f"{name}: the ordered down should fit this shape"
     hot = dec.calibrate_hot_channels(w, k, prompt_ids(16, cfg.vocab, seed=1001), cache_fraction=0.2)
     cached = dec.DecodeEngine(w, "cached_dip", dip_k=k, hot_channels=hot, max_new_tokens=4)
-    for eng, tag in ((gated, "gated"), (cached, "cached_dip")):
+    default = dec.DecodeEngine(w, "dip", dip_k=k, max_new_tokens=4)  # no schedule named
+    for eng, tag in ((gated, "gated"), (cached, "cached_dip"), (default, "default")):
         for use_graph in (False, True):
             assert eng.generate(prompt, 4, use_graph=use_graph) == want, f"{name} {tag} graph={use_graph}"
             assert torch.equal(eng.x_final, plain.x_final), f"{name} {tag} graph={use_graph}: hidden state"

@@ -89,12 +89,13 @@ def test_gated_and_cached_dip_bit_identical_to_dip(dec, model):
     c, k, w = model
     cfg = w.config
     prompt = prompt_ids(540, cfg.vocab, seed=37)
-    plain = dec.DecodeEngine(w, "dip", dip_k=k, max_new_tokens=4)
+    plain = dec.DecodeEngine(w, "dip", dip_k=k, max_new_tokens=4, dip_schedule="indexed")
     want = plain.generate(prompt, 4, use_graph=True)
     r = np.random.default_rng(cfg.intermediate + k)
     hot = [sorted(r.choice(cfg.intermediate, size=int(r.integers(0, cfg.intermediate + 1)), replace=False).tolist())
            for _ in range(cfg.layers)]
     engines = [("gated", dec.DecodeEngine(w, "dip", dip_k=k, max_new_tokens=4, dip_schedule="gated")),
+               ("default", dec.DecodeEngine(w, "dip", dip_k=k, max_new_tokens=4)),
                ("cached_dip", dec.DecodeEngine(w, "cached_dip", dip_k=k, hot_channels=hot, max_new_tokens=4))]
     for tag, eng in engines:
         for use_graph in (False, True):

@@ -217,7 +217,7 @@ def test_engine_runs_a_loaded_checkpoint_from_host_memory(off, tmp_path, fused):
     hot = [list(range(0, cfg.intermediate, 3)) for _ in range(cfg.layers)]
     dense = D.DecodeEngine(w_dev, "dense", max_new_tokens=6, fused=fused)
     want_dense = dense.generate(prompt, 6)
-    dip = D.DecodeEngine(w_dev, "dip", dip_k=k, max_new_tokens=6, fused=fused)
+    dip = D.DecodeEngine(w_dev, "dip", dip_k=k, max_new_tokens=6, fused=fused, dip_schedule="indexed")
     want_dip = dip.generate(prompt, 6)
     for mode, kw, want, ref in (("dense", {}, want_dense, dense),
                                 ("cached_dip", dict(dip_k=k, hot_channels=[[] for _ in range(cfg.layers)]), want_dip,

@@ -25,7 +25,8 @@ FORMS = [((2048, 6144, 3072), "ordered"), ((512, 1024, 51), "ordered"), ((2560, 
          ((4096, 12288, 1228), "ordered"), ((4096, 12288, 2457), None), ((4096, 12288, 6144), None),
          ((4096, 12288, 9830), "rows"), ((5120, 5120, 1024), "ordered"), ((5120, 5120, 1792), "rows"),
          ((5120, 5120, 4096), "rows"), ((3072, 8192, 2000), "ordered"), ((2048, 11008, 8806), "rows"),
-         ((2048, 16384, 13107), "rows"), ((2048, 16384, 8192), "rows"), ((4096, 12288, 7987), "rows"), ((2560, 9728, 3404), None), ((5120, 17408, 3481), None),
+         ((2048, 16384, 13107), "rows"), ((2048, 16384, 8192), "rows"), ((4096, 12288, 7987), "rows"),
+         ((2560, 9728, 3404), None), ((5120, 17408, 3481), None),
          ((5120, 17408, 13926), None), ((1024, 20480, 1024), None)]
 
 

@@ -93,7 +93,8 @@ def test_streamed_prompt_equals_resident(dec, weights):
 def dip_engines(dec, w, k):
     hot = [list(range(0, w.config.intermediate, 3)) for _ in range(w.config.layers)]
     none = [[] for _ in range(w.config.layers)]
-    return {"indexed": dict(mode="dip"), "gated": dict(mode="dip", dip_schedule="gated"),
+    return {"indexed": dict(mode="dip", dip_schedule="indexed"), "default": dict(mode="dip"),
+            "gated": dict(mode="dip", dip_schedule="gated"),
             "cached": dict(mode="cached_dip", hot_channels=hot),
             "all missing": dict(mode="cached_dip", hot_channels=none, miss_path="staged"),
             "streamed": dict(mode="cached_dip", hot_channels=hot, offload=True)}
@@ -142,6 +143,31 @@ def test_matrix_core_prompt_near_single_steps(dec, weights, n):
         e.reset()
     a.prefill(prompt)
     one_at_a_time(b, prompt)
+    near_state(a, b, n)
+
+
+@pytest.mark.parametrize("what", ["dense", "default", "indexed", "cached", "streamed"])
+def test_prompt_in_parts(dec, weights, monkeypatch, what):
+    """A prompt longer than one part: parts of 16, 16 and 1 tokens, the later ones behind a context (dense: the first two
+    on the matrix cores, the last in the step's order)."""
+    monkeypatch.setattr(dec, "PROMPT_CHUNK", 16)
+    c = weights.config
+    kw = dict(mode="dense") if what == "dense" else dict(dip_k=c.intermediate // 2,
+                                                         **dip_engines(dec, weights, 1)[what])
+    a, b = (dec.DecodeEngine(weights, max_new_tokens=2, **kw) for _ in range(2))
+    prompt = tokens(33, c.vocab, 11)
+    for e in (a, b):
+        e.reset()
+    a.prefill(prompt)
+    one_at_a_time(b, prompt)
+    b.token.fill_(prompt[-1])
+    if what != "dense":
+        same_state(a, b, 33, what)
+        return
+    near_state(a, b, 33)
+
+
+def near_state(a, b, n):
     pairs = [(a.x_final, b.x_final), (a.hn, b.hn)]
     for l in range(2):
         pairs += [(a.k_cache[l][:, :n], b.k_cache[l][:, :n]), (a.v_cache[l][:, :n], b.v_cache[l][:, :n])]
@@ -164,16 +190,33 @@ def fragments(x):
                                     (2048, 6144, 128)])
 @pytest.mark.parametrize("T", [1, 16, 17, 33, 64, 65, 200])
 def test_matrix_core_linear(cuda, N, K, gs, T):
-    """Tiles of 16, 32 and 64 rows (N below, at and past each), one to four token tiles and their remainders, 4 and 8
-    waves over 1 to 48 steps, scale groups of 1 to 3 steps: against binary64. The sum of K products in binary32 is
-    within K 2^-24 of the sum of their absolute values; the result is then rounded to binary16."""
+    """Tiles of 16 and 32 rows (N below, at and past each), one to four token tiles and their remainders, 4 and 8 waves
+    over 1 to 48 steps, scale groups of 1 to 3 steps."""
+    check_matrix_core_linear(cuda, N, K, gs, T)
+
+
+@pytest.mark.parametrize("N,K,T", [(12288, 256, 200), (12308, 384, 193), (33024, 256, 16), (33024, 128, 32)])
+def test_matrix_core_linear_of_64_row_tiles(cuda, N, K, T):
+    """The tiles of launches of 2048 16-row x token tiles up, over one, two and four token tiles, N with and without a
+    remainder."""
+    check_matrix_core_linear(cuda, N, K, 128, T)
+
+
+@pytest.mark.parametrize("scale", [1e-5, 3e-7])
+def test_matrix_core_linear_of_subnormal_activations(cuda, scale):
+    check_matrix_core_linear(cuda, 256, 1024, 128, 33, scale)
+
+
+def check_matrix_core_linear(cuda, N, K, gs, T, x_scale=1.0):
+    """Every epilogue against binary64. The sum of K products in binary32 is within K 2^-24 of the sum of their absolute
+    values; the result is then rounded to binary16."""
     from soinfer.quant import formats, pack
 
     lib = ctypes.CDLL(str(Path(pack.__file__).resolve().parent.parent / "libsoinfer_hip.so"))
     g = torch.Generator(device=cuda).manual_seed(N + K + T)
     qt = formats.quantize(torch.randn(N, K, generator=g, device=cuda) * 0.02, formats.QuantConfig(4, "group", gs))
     W = pack.pack_int4(qt.qweight)[0].contiguous()
-    x = torch.randn(T, K, generator=g, device=cuda).half()
+    x = (torch.randn(T, K, generator=g, device=cuda) * x_scale).half()
     w64 = (qt.qweight.double().view(N, K // gs, gs) * qt.scale.double()[..., None]).view(N, K)
     ref, mag = x.double() @ w64.T, x.double().abs() @ w64.abs().T
     bound = K * 2.0 ** -24 * mag + 2.0 ** -11 * ref.abs() + 2.0 ** -24
@@ -345,3 +388,28 @@ def test_short_prompts_behind_a_context(cuda, dec, weights):
     b.reset()
     b.prefill(tokens(3, c.vocab, 7))  # no graph captured
     assert int(b.pos) == 3
+
+
+@pytest.mark.parametrize("mode", ["dense", "dip", "cached_dip"])
+@pytest.mark.parametrize("bad", [float("nan"), float("inf")])
+def test_a_token_that_is_not_a_number_leaves_the_others_alone(cuda, dec, weights, mode, bad):
+    """Its hidden state is not a number; the K and V of the tokens before it are those of the prompt without it."""
+    import dataclasses
+
+    c = weights.config
+    embed = weights.embed.clone()
+    embed[5, ::3] = bad
+    w = dataclasses.replace(weights, embed=embed)
+    kw = {} if mode == "dense" else dict(dip_k=c.intermediate // 2)
+    if mode == "cached_dip":
+        kw["hot_channels"] = [list(range(0, c.intermediate, 3))] * c.layers
+    a, b = (dec.DecodeEngine(w, mode, max_new_tokens=1, **kw) for _ in range(2))
+    prompt = [t if t != 5 else 6 for t in tokens(20, c.vocab, 5)]
+    for e, p in ((a, prompt + [5]), (b, prompt)):
+        e.reset()
+        e.prefill(p, use_graph=False)
+    assert not bool(torch.isfinite(a.x_final).any())
+    for l in range(c.layers):
+        assert torch.equal(a.k_cache[l][:, :20], b.k_cache[l][:, :20])
+        assert torch.equal(a.v_cache[l][:, :20], b.v_cache[l][:, :20])
+        assert bool(torch.isfinite(b.k_cache[l][:, :20]).all())

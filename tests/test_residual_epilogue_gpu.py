@@ -139,6 +139,7 @@ def tiny(dec):
 
 
 @pytest.mark.parametrize("mode,k,extra", [("dense", None, {}), ("dip", 256, {}), ("dip", 256, {"dip_dense_up": True}),
+                                          ("dip", 256, {"dip_schedule": "indexed"}),
                                           ("cached_dip", 256, {"hot_channels": "third"}),
                                           ("dense", None, {"offload": True})])
 def test_engine_residual_epilogue_bit_identical(dec, tiny, mode, k, extra):
