@@ -1838,8 +1838,8 @@ void check_dip_x(const torch::Tensor& x, int64_t K, const char* n) {
 }  // namespace
 
 // (y [H], idx [k]) of the DIP MLP over resident weights in two launches: gate and up of every channel, then the
-// selection in each workgroup of the gated sparse down. At 2048 x 6144, k = 3072: 15.7 us a call, bound by the two
-// launches' latency; as 14 launches from Python (|gate| conversions, gathers, SiLU, a zeroed workspace) 59-69 us.
+// selection in each workgroup of the gated sparse down. At 2048 x 6144, k = 3072: 15.7 us a call, all of it the two
+// dependent kernels (5.4 and 11.5 us in a kernel trace from cold weights); as 14 launches from Python (|gate| conversions, gathers, SiLU, a zeroed workspace) 59-69 us.
 std::tuple<torch::Tensor, torch::Tensor> dip_mlp(torch::Tensor gate_Wq, torch::Tensor gate_scale, torch::Tensor up_Wq,
                                                  torch::Tensor up_scale, torch::Tensor down_T_Wq,
                                                  torch::Tensor down_T_scale, torch::Tensor x, int64_t k, int64_t K,

@@ -7,12 +7,15 @@
 // Values: these kernels evaluate, for every (token, row) and (token, head), the expressions of the decode step in
 // the decode step's order (the lane partition and reduction tree of gemv_int4_tile, the norm's partition, the
 // split plan and combine of the attention), so hidden states, caches and selections are bit for bit those of
-// the same tokens fed one at a time. Reference: the prompt loop of generate_streaming / generate_dip
+// the same tokens fed one at a time. The linears of dense prompts of 9 tokens up are the exception: they run in
+// prompt_mfma.hip, whose sums take another order (here are their norms, attention and, for group sizes or widths that
+// kernel does not take, their linears too). Reference: the prompt loop of generate_streaming / generate_dip
 // (python/soinfer/runtime/generate.py:429-520), one token per step.
 //
-// Measured (28-layer Qwen3-1.7B shape, dense): a 256-token prompt and its first token take 13.2 ms against 146.2 ms
-// with one layers-graph replay per token; 48 tokens and 4 new ones with 8 layers streamed from host memory 20.3
-// against 197 ms (the weights cross PCIe once for the prompt instead of once per token).
+// Measured (Qwen3-1.7B shape, dense): 8 tokens through 4 layers 289 us against 732 with one layers-graph replay per
+// token. With the linears on the matrix cores, 28 layers, a 256-token prompt and its first token 3.8 ms against 146 (13.2
+// with these linears); 48 tokens and 4 new ones with 8 layers streamed from host memory 19.7 against 197 (the weights
+// cross PCIe once for the prompt instead of once per token).
 #include "soi_device.h"
 #include "soi_host.h"
 #include "soi_attn.h"

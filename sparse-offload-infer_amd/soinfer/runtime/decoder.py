@@ -49,12 +49,12 @@ from ..quant import formats, pack
 
 # Generation steps per replay of the chunk graph (decode replays it for each full chunk of the requested steps)
 GRAPH_CHUNK = 4
-# Prompt tokens that go through the layers together (bounds the activations' scratch: about 50 KB per token of the
-# Qwen3-1.7B shape)
+# Prompt tokens that go through the layers together (bounds the activations' scratch: 60 KB per token of the
+# Qwen3-1.7B shape, 66 KB with DIP at k/I = 0.5)
 PROMPT_CHUNK = 1024
 # Dense prompts of this many tokens up run their linears on the matrix cores; shorter ones (one 8-token tile) keep the
-# decode step's order and bits (28-layer Qwen3-1.7B shape: 8 tokens 1.7 ms, 9 tokens 1.2 against 1.9 ms in the step's
-# order, 256 tokens 3.1 against 12.4)
+# decode step's order and so its bits, which costs time (28-layer Qwen3-1.7B shape: 8 tokens 1.7 ms, 9 tokens 1.2 against
+# 1.9 ms in the step's order, 256 tokens 3.1 against 12.4)
 PROMPT_MFMA = 9
 
 
@@ -1028,9 +1028,10 @@ def add_selection_counts(counts: torch.Tensor, sel: torch.Tensor) -> None:
 
 
 def calibrate_channel_counts(w: DecoderWeights, dip_k: int, calib_tokens) -> list:
-    """Per layer, counts[c] = how many of the calib_tokens steps selected channel c, feeding the tokens one at a
-    time through the DIP engine (eagerly) as the reference's calibrate_channel_frequencies does
-    (generate.py:579-609). int64 [I] tensors on the engine's device; each sums to len(calib_tokens) * dip_k."""
+    """Per layer, counts[c] = how many of the calib_tokens selected channel c, with the selections of the DIP engine's
+    single steps (its prompts give the same ones bit for bit), as the reference's calibrate_channel_frequencies counts
+    them one token at a time (generate.py:579-609). int64 [I] tensors on the engine's device; each sums to
+    len(calib_tokens) * dip_k (a token whose gates are not numbers counts nothing)."""
     c = w.config
     eng = DecodeEngine(w, "dip", dip_k=dip_k, max_new_tokens=1, dip_schedule="indexed")  # no copies of the weights
     eng.counts = [torch.zeros(c.intermediate, dtype=torch.int64, device=eng.device) for _ in range(c.layers)]

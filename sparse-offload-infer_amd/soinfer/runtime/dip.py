@@ -64,8 +64,10 @@ def silu_gate(gate: torch.Tensor, idx: torch.Tensor, u: torch.Tensor) -> torch.T
 
 def dip_mlp(w: DipMLPWeights, x: torch.Tensor, dip_k: int, channel_counts: Optional[torch.Tensor] = None):
     """Resident-weight DIP MLP. Returns (y [H] fp16, idx [dip_k] int32). Two launches: gate and up of every channel,
-    then the selection inside the sparse down (up of an unselected channel is not used: reading it costs less than
-    the launch that would leave it out)."""
+    then the selection inside the sparse down. up of an unselected channel is read and not used; leaving it out takes two
+    launches more (top-k, and up over its selection: as cached_dip_mlp_direct), which cost more up to 4096 x 12288 (2048
+    x 6144, k/I 0.05 / 0.3: 16.5 / 16.4 us against 23.7 / 22.6; 4096 x 12288: 25.9 / 29.5 against 25.4 / 30.2) and less
+    where few of very many channels are selected (5120 x 17408: 38.3 / 43.4 against 34.1 / 43.2)."""
     y, idx = _C.dip_mlp(w.gate_Wq, w.gate_scale, w.up_Wq, w.up_scale, w.down_T_Wq, w.down_T_scale, x, dip_k,
                         w.hidden_size, w.group_size)
     if channel_counts is not None:
