@@ -274,7 +274,8 @@ class DecodeEngine:
     dip_schedule (mode "dip"): "indexed" (4 MLP launches, the schedule cached_dip equals bit for bit), "gated" (2 MLP
     launches, the same tokens and hidden states as "indexed" bit for bit) or "dense_up" (2 MLP launches, y summed in
     another order; dip_dense_up=True is the same). Default: the indexed results, by the gated launches where these are
-    faster (default_gated_form). The gated launches keep a second copy of gate|up and, in the ordered form, of down_proj^T
+    faster (default_gated_form; where a token has fewer than k gates that are numbers these add what is selected, the
+    indexed ones NaN). The gated launches keep a second copy of gate|up and, in the ordered form, of down_proj^T
     (28 layers of the Qwen3-1.7B shape: 374 + 187 MB).
     offload=True keeps the dense weights of every layer (q|k|v, o, and gate|up + down for dense or gate for
     cached DIP) in a pinned host arena and copies each layer's block into one of two device slots: the
