@@ -1837,13 +1837,14 @@ void check_dip_x(const torch::Tensor& x, int64_t K, const char* n) {
 
 }  // namespace
 
-// (y [H], idx [k]) of the DIP MLP over resident weights in two launches: gate and up of every channel, then the
+// (y [H], idx [k], their count [1]) of the DIP MLP over resident weights in two launches: gate and up of every channel, then the
 // selection in each workgroup of the gated sparse down. At 2048 x 6144, k = 3072: 15.7 us a call, all of it the two
 // dependent kernels (5.4 and 11.5 us in a kernel trace from cold weights); as 14 launches from Python (|gate| conversions, gathers, SiLU, a zeroed workspace) 59-69 us.
-std::tuple<torch::Tensor, torch::Tensor> dip_mlp(torch::Tensor gate_Wq, torch::Tensor gate_scale, torch::Tensor up_Wq,
-                                                 torch::Tensor up_scale, torch::Tensor down_T_Wq,
-                                                 torch::Tensor down_T_scale, torch::Tensor x, int64_t k, int64_t K,
-                                                 int64_t group_size) {
+std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> dip_mlp(torch::Tensor gate_Wq, torch::Tensor gate_scale,
+                                                                torch::Tensor up_Wq, torch::Tensor up_scale,
+                                                                torch::Tensor down_T_Wq, torch::Tensor down_T_scale,
+                                                                torch::Tensor x, int64_t k, int64_t K,
+                                                                int64_t group_size) {
     const char* n = "dip_mlp";
     check_dip_x(x, K, n);
     TORCH_CHECK(group_size >= 1 && group_size % 8 == 0, n, ": group_size must be a positive multiple of 8");
@@ -1869,7 +1870,7 @@ std::tuple<torch::Tensor, torch::Tensor> dip_mlp(torch::Tensor gate_Wq, torch::T
                                            down_T_scale.data_ptr<float>(), I, ip, ip + k, h16m(y), K, group_size, G,
                                            ws.buf.data_ptr<uint8_t>(), ws.buf.numel(), st),
                  n);
-    return {y, idx.narrow(0, 0, k)};
+    return {y, idx.narrow(0, 0, k), idx.narrow(0, k, 1)};
 }
 
 // First half of the cache-aware DIP MLP: (gate [I], idx [k], workspace of the down, counters cleared). With slot_of,
@@ -2040,7 +2041,7 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("quantize_group", &quantize_group, "symmetric group quantization: (codes, scales)");
     m.def("pack_int4", &pack_int4, "int8 codes to AWQ-order INT4 rows");
     m.def("transpose_int4", &transpose_int4, "the transpose of packed INT4 rows, packed");
-    m.def("dip_mlp", &dip_mlp, "one DIP MLP over resident weights: (y, idx)");
+    m.def("dip_mlp", &dip_mlp, "one DIP MLP over resident weights: (y, idx, count)");
     m.def("dip_gate_select", &dip_gate_select, "gate, selection and a cleared down workspace (and the miss count)",
           py::arg("gate_Wq"), py::arg("gate_scale"), py::arg("x"), py::arg("k"), py::arg("K"), py::arg("group_size"),
           py::arg("slot_of") = py::none(), py::arg("miss_count") = py::none());

@@ -122,3 +122,26 @@ def test_a_call_that_fails_leaves_nothing_running(cuda, side):
     y, idx = by_operators(w, x, 4096)
     got = dip.cached_dip_mlp(w, cache, x, 4096, *pinned, staging)
     assert torch.equal(got[0], y) and torch.equal(got[1], idx)
+
+
+@pytest.mark.parametrize("I,k", [(512, 200), (9000, 4000)])
+def test_channel_counts_of_gates_that_are_not_numbers(cuda, I, k):
+    """Fewer than k gates that are numbers: those channels count once, the rest of the list nothing (the fused selection
+    and the separate one above its widths)."""
+    from soinfer.runtime import dip
+
+    w, x = make(cuda, I, 256, 128, I)
+    counts = torch.zeros(I, dtype=torch.int64, device=cuda)
+    _, idx = dip.dip_mlp(w, x, k, counts)
+    assert torch.equal(counts.nonzero().flatten(), idx.long()) and int(counts.max()) == 1
+    few = torch.arange(3, I, 7, device=cuda)[:k // 3]
+    scale = torch.full_like(w.gate_scale, float("nan"))
+    scale[few] = w.gate_scale[few]
+    w.gate_scale = scale
+    counts.zero_()
+    _, idx = dip.dip_mlp(w, x, k, counts)
+    assert torch.equal(counts.nonzero().flatten(), few) and int(counts.sum()) == few.numel()
+    assert torch.equal(idx[:few.numel()].long(), few)
+    counts.zero_()
+    dip.dip_mlp(w, torch.full_like(x, float("nan")), k, counts)
+    assert int(counts.sum()) == 0
