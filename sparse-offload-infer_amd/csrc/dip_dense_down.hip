@@ -349,7 +349,10 @@ __global__ __launch_bounds__(kDdThreads) void dip_dense_down_kernel(DdArgs a) {
 //   3. the chunk masks [|gate| >= tau] and each wave's packed row go to LDS
 //      (one barrier); each thread finds the positions of its selected
 //      channels from the chunk prefix counts and writes (coef, location of
-//      the channel's nibble in a row) per position p < k (one barrier);
+//      the channel's nibble in a row) per position p < k, and in workgroup 0,
+//      when the index list is asked for, the channel to it (one barrier);
+//      written after y by every workgroup's window of positions the list took
+//      1.9 us;
 //   4. thread t runs chain (r, g) = (t / 32, t % 32) (then t + 512, ...) for
 //      all 8 rows of the workgroup, two positions per step: one read of two
 //      table entries feeds 16 row-byte reads (a signed bitfield extract gives
@@ -520,6 +523,7 @@ __global__ __launch_bounds__(kDdThreads) void dip_down_ordered_kernel(OdArgs a) 
     // channels this wave's lane 8 * wave + (lane >> 3) holds at index m; the group's channels sit at bits
     // 4 (lane & 7) .. + 3 of the chunk's mask
     {
+        const bool list = b == 0 && a.out_idx != nullptr;
         const int src = 8 * wave + (lane >> 3);
         const uint32_t sh = 4u * static_cast<uint32_t>(lane & 7);
 #pragma unroll
@@ -539,6 +543,7 @@ __global__ __launch_bounds__(kDdThreads) void dip_down_ordered_kernel(OdArgs a) 
                     const uint32_t loc = (byte0 + 2u * static_cast<uint32_t>(p & 1)) |
                                          ((4u * static_cast<uint32_t>(p >> 1)) << 16);
                     s_pos[pos] = u32x2{__builtin_bit_cast(uint32_t, xc[m][p]), loc};
+                    if (list) stg(a.out_idx + pos, static_cast<int32_t>(4 * t + static_cast<uint32_t>(p)));
                 }
                 pos += on ? 1u : 0u;
             }
@@ -605,28 +610,7 @@ __global__ __launch_bounds__(kDdThreads) void dip_down_ordered_kernel(OdArgs a) 
         if (a.res_out) stg(a.res_out + row, static_cast<uint16_t>(add_f16x2(rv, yb)));
     }
 
-    // 5. the index list when asked for (after y), by wave 0: workgroup b writes positions [b*win, (b+1)*win)
     if (b == 0 && tid == 0 && a.out_count) stg(a.out_count, static_cast<int32_t>(kk));
-    if (!a.out_idx || wave != 0) return;  // wave-uniform
-    const uint32_t win = (kk + nb - 1) / nb;
-    const uint32_t lo = b * win;
-    const uint32_t hi = lo + win < kk ? lo + win : kk;
-#pragma unroll
-    for (int i = 0; i < NC; ++i) {
-        const int c = lane + i * kWave;
-        const int keep = before[i] >= k ? 0
-                         : (before[i] + static_cast<uint32_t>(__builtin_popcount(bits[i])) <= k
-                                ? 32
-                                : nth_set_bit(bits[i], k - before[i]) + 1);
-        uint32_t x = keep >= 32 ? bits[i] : (bits[i] & ((1u << keep) - 1u));
-        uint32_t pos = before[i];
-        if (c >= chunks || pos >= hi || pos + static_cast<uint32_t>(__builtin_popcount(x)) <= lo) continue;
-        while (x != 0u) {
-            if (pos >= lo && pos < hi) stg(a.out_idx + pos, static_cast<int32_t>(32 * c + __builtin_ctz(x)));
-            ++pos;
-            x &= x - 1u;
-        }
-    }
 }
 
 }  // namespace soi

@@ -645,8 +645,7 @@ class DecodeEngine:
         c = self.c
         if self.dip_gated_tr:
             Wt, St = self.down_tt[l]
-            # without a named schedule a step leaves the last layer's idx and cnt, as the indexed launches do (the list
-            # takes 1.9 us to write, so the layers whose list the next one replaces leave it out)
+            # without a named schedule a step leaves the last layer's idx and cnt, as the indexed launches do
             want = self.counts is not None or self.layer_hook is not None or \
                 (self._gated_auto and l == c.layers - 1)
             _C.dip_select_down_ordered_into(gate, hu, self.k, Wt, St, self.idx if want else None,
