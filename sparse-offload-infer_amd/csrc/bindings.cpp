@@ -1837,14 +1837,14 @@ void check_dip_x(const torch::Tensor& x, int64_t K, const char* n) {
 
 }  // namespace
 
-// (y [H], idx [k], their count [1]) of the DIP MLP over resident weights in two launches: gate and up of every channel, then the
-// selection in each workgroup of the gated sparse down. At 2048 x 6144, k = 3072: 15.7 us a call, all of it the two
-// dependent kernels (5.4 and 11.5 us in a kernel trace from cold weights); as 14 launches from Python (|gate| conversions, gathers, SiLU, a zeroed workspace) 59-69 us.
-std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> dip_mlp(torch::Tensor gate_Wq, torch::Tensor gate_scale,
-                                                                torch::Tensor up_Wq, torch::Tensor up_scale,
-                                                                torch::Tensor down_T_Wq, torch::Tensor down_T_scale,
-                                                                torch::Tensor x, int64_t k, int64_t K,
-                                                                int64_t group_size) {
+// (y [H], idx [k]) of the DIP MLP over resident weights in two launches: gate and up of every channel, then the
+// selection in each workgroup of the gated sparse down; count [1], when given: the selected channels. At 2048 x 6144,
+// k = 3072: 15.7 us a call, all of it the two dependent kernels (5.4 and 11.5 us in a kernel trace from cold weights);
+// as 14 launches from Python (|gate| conversions, gathers, SiLU, a zeroed workspace) 59-69 us.
+std::tuple<torch::Tensor, torch::Tensor> dip_mlp(torch::Tensor gate_Wq, torch::Tensor gate_scale, torch::Tensor up_Wq,
+                                                 torch::Tensor up_scale, torch::Tensor down_T_Wq,
+                                                 torch::Tensor down_T_scale, torch::Tensor x, int64_t k, int64_t K,
+                                                 int64_t group_size, c10::optional<torch::Tensor> count) {
     const char* n = "dip_mlp";
     check_dip_x(x, K, n);
     TORCH_CHECK(group_size >= 1 && group_size % 8 == 0, n, ": group_size must be a positive multiple of 8");
@@ -1854,6 +1854,10 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> dip_mlp(torch::Tensor ga
     const int64_t I = gate_Wq.size(0);
     TORCH_CHECK(up_Wq.size(0) == I && down_T_Wq.size(0) == I, n, ": gate, up and down^T must have the same rows");
     TORCH_CHECK(k >= 1 && k <= I, n, ": k must be in [1, n]");
+    if (count) {
+        need(*count, torch::kInt32, x, n, "count");
+        need_numel(*count, 1, n, "count");
+    }
     const at::DeviceGuard guard(x.device());
     auto gu = torch::empty({2 * I}, x.options());
     auto y = torch::empty({K}, x.options());
@@ -1867,10 +1871,11 @@ std::tuple<torch::Tensor, torch::Tensor, torch::Tensor> dip_mlp(torch::Tensor ga
                  n);
     int32_t* ip = idx.data_ptr<int32_t>();
     check_status(soi_dip_select_gated_down(h16(gu), h16(gu) + I, I, k, down_T_Wq.data_ptr<uint8_t>(),
-                                           down_T_scale.data_ptr<float>(), I, ip, ip + k, h16m(y), K, group_size, G,
+                                           down_T_scale.data_ptr<float>(), I, ip,
+                                           count ? count->data_ptr<int32_t>() : ip + k, h16m(y), K, group_size, G,
                                            ws.buf.data_ptr<uint8_t>(), ws.buf.numel(), st),
                  n);
-    return {y, idx.narrow(0, 0, k), idx.narrow(0, k, 1)};
+    return {y, idx.narrow(0, 0, k)};
 }
 
 // First half of the cache-aware DIP MLP: (gate [I], idx [k], workspace of the down, counters cleared). With slot_of,
@@ -2041,7 +2046,9 @@ PYBIND11_MODULE(TORCH_EXTENSION_NAME, m) {
     m.def("quantize_group", &quantize_group, "symmetric group quantization: (codes, scales)");
     m.def("pack_int4", &pack_int4, "int8 codes to AWQ-order INT4 rows");
     m.def("transpose_int4", &transpose_int4, "the transpose of packed INT4 rows, packed");
-    m.def("dip_mlp", &dip_mlp, "one DIP MLP over resident weights: (y, idx, count)");
+    m.def("dip_mlp", &dip_mlp, "one DIP MLP over resident weights: (y, idx)", py::arg("gate_Wq"), py::arg("gate_scale"),
+          py::arg("up_Wq"), py::arg("up_scale"), py::arg("down_T_Wq"), py::arg("down_T_scale"), py::arg("x"), py::arg("k"),
+          py::arg("K"), py::arg("group_size"), py::arg("count") = py::none());
     m.def("dip_gate_select", &dip_gate_select, "gate, selection and a cleared down workspace (and the miss count)",
           py::arg("gate_Wq"), py::arg("gate_scale"), py::arg("x"), py::arg("k"), py::arg("K"), py::arg("group_size"),
           py::arg("slot_of") = py::none(), py::arg("miss_count") = py::none());

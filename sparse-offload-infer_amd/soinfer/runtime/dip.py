@@ -68,8 +68,9 @@ def dip_mlp(w: DipMLPWeights, x: torch.Tensor, dip_k: int, channel_counts: Optio
     launches more (top-k, and up over its selection: as cached_dip_mlp_direct), which cost more up to 4096 x 12288 (2048
     x 6144, k/I 0.05 / 0.3: 16.5 / 16.4 us against 23.7 / 22.6; 4096 x 12288: 25.9 / 29.5 against 25.4 / 30.2) and less
     where few of very many channels are selected (5120 x 17408: 38.3 / 43.4 against 34.1 / 43.2)."""
-    y, idx, count = _C.dip_mlp(w.gate_Wq, w.gate_scale, w.up_Wq, w.up_scale, w.down_T_Wq, w.down_T_scale, x, dip_k,
-                               w.hidden_size, w.group_size)
+    count = None if channel_counts is None else torch.empty(1, dtype=torch.int32, device=x.device)
+    y, idx = _C.dip_mlp(w.gate_Wq, w.gate_scale, w.up_Wq, w.up_scale, w.down_T_Wq, w.down_T_scale, x, dip_k,
+                        w.hidden_size, w.group_size, count)
     if channel_counts is not None:
         # fewer than k gates that are numbers: the list past the count is not written
         kept = torch.arange(idx.shape[0], dtype=torch.int32, device=idx.device) < count
