@@ -349,10 +349,10 @@ __global__ __launch_bounds__(kDdThreads) void dip_dense_down_kernel(DdArgs a) {
 //   3. the chunk masks [|gate| >= tau] and each wave's packed row go to LDS
 //      (one barrier); each thread finds the positions of its selected
 //      channels from the chunk prefix counts and writes (coef, location of
-//      the channel's nibble in a row) per position p < k, and in workgroup 0,
-//      when the index list is asked for, the channel to it (one barrier);
-//      written after y by every workgroup's window of positions the list took
-//      1.9 us;
+//      the channel's nibble in a row) per position p < k (one barrier).
+//      Workgroup 0 writes the index list, when asked for, from that table (a
+//      window of positions per workgroup after y took up to 2 us: 2048 x 6144,
+//      k = 3072 7.2 -> 9.0 us; from the table 7.2);
 //   4. thread t runs chain (r, g) = (t / 32, t % 32) (then t + 512, ...) for
 //      all 8 rows of the workgroup, two positions per step: one read of two
 //      table entries feeds 16 row-byte reads (a signed bitfield extract gives
@@ -523,7 +523,6 @@ __global__ __launch_bounds__(kDdThreads) void dip_down_ordered_kernel(OdArgs a) 
     // channels this wave's lane 8 * wave + (lane >> 3) holds at index m; the group's channels sit at bits
     // 4 (lane & 7) .. + 3 of the chunk's mask
     {
-        const bool list = b == 0 && a.out_idx != nullptr;
         const int src = 8 * wave + (lane >> 3);
         const uint32_t sh = 4u * static_cast<uint32_t>(lane & 7);
 #pragma unroll
@@ -543,13 +542,22 @@ __global__ __launch_bounds__(kDdThreads) void dip_down_ordered_kernel(OdArgs a) 
                     const uint32_t loc = (byte0 + 2u * static_cast<uint32_t>(p & 1)) |
                                          ((4u * static_cast<uint32_t>(p >> 1)) << 16);
                     s_pos[pos] = u32x2{__builtin_bit_cast(uint32_t, xc[m][p]), loc};
-                    if (list) stg(a.out_idx + pos, static_cast<int32_t>(4 * t + static_cast<uint32_t>(p)));
                 }
                 pos += on ? 1u : 0u;
             }
         }
     }
     __syncthreads();
+
+    // the index list when asked for, by workgroup 0, its stores in flight during the chains: entry p's byte and shift give
+    // its channel 4t + e back (byte 4 (t >> 1) + (t & 1) + 2 (e & 1), shift 4 (e >> 1))
+    if (b == 0 && a.out_idx) {
+        for (int p = tid; p < static_cast<int>(kk); p += kDdThreads) {
+            const uint32_t loc = s_pos[p].y, byte = loc & 0xffffu;
+            const uint32_t t = 2u * (byte >> 2) + (byte & 1u);
+            stg(a.out_idx + p, static_cast<int32_t>(4u * t + ((byte >> 1) & 1u) + 2u * (loc >> 18)));
+        }
+    }
 
     // 4. the chains: thread t takes chain (r, gsub) = (t / 32, t % 32), then t + 512, ..., for all 8 rows of the
     // workgroup at once (sparse-down wave gsub >> 3 and row lane gsub & 7 read positions r * rpc + gsub + 32i)
