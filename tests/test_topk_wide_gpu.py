@@ -21,3 +21,22 @@ def test_wide_selection(cuda, n, frac):
     g[5] = np.float32(1e30)
     got = ops.topk_threshold_select(torch.from_numpy(g).to(cuda), k)
     assert np.array_equal(got.cpu().numpy(), O.topk_rule_a(g, k))
+
+
+@pytest.mark.parametrize("n", [16384, 16385, 17408, 24576, 24577, 32768, 32769])
+@pytest.mark.parametrize("frac", [0.0, 0.3, 1.0])
+def test_wide_selection_of_binary16_gates(cuda, n, frac):
+    """The |gate| form of the same kernels (what a 17408-wide engine selects with): signs, ties, infinities, and NaN (never
+    selected: with every channel asked for, fewer than k are)."""
+    from soinfer import _C
+
+    k = max(1, int(n * frac))
+    gate = torch.randn(n, generator=torch.Generator().manual_seed(n + k)).half()
+    gate[::7], gate[1::11], gate[5], gate[9] = gate[3].clone(), 0.0, float("inf"), float("-inf")
+    gate[13::101] = float("nan")
+    want = O.topk_rule_a(gate.float().abs().numpy(), k)
+    idx = torch.full((k,), -7, dtype=torch.int32, device=cuda)
+    cnt = torch.zeros(1, dtype=torch.int32, device=cuda)
+    _C.topk_threshold_select_f16abs_into(gate.to(cuda), k, idx, cnt)
+    assert int(cnt) == want.size
+    assert np.array_equal(idx.cpu().numpy()[:want.size], want) and bool((idx[want.size:] == -7).all())
