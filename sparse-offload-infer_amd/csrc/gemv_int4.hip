@@ -393,12 +393,13 @@ static int launch_int4(const Rows& rows, int64_t N, const uint16_t* x, const EP&
     // 3 passes: 4 (4096 x 12288 8.3 / 8.0, 5120 x 17408 14.9 / 14.5, 8192 x 8192 10.7 / 9.6). 2 passes, or 3 whole ones:
     // 2 below 8192 rows, where the finer tiles even out the last round of waves (5120 x 3072 4.71 / 5.06, 5120 x 4096
     // 4.70 / 5.03, 5120 x 6144 5.81 / 6.08), 4 from there, where the extra waves are a round of their own (12288 x 2560
-    // 7.56 / 6.77, 12288 x 6144 9.62 / 9.03, 17408 x 2560 9.37 / 8.86). 3 passes with a part: 4 up to 4096 rows and from
-    // 24576 (4096 x 5120 5.13 / 5.00, 24576 x 5120 4% apart), 2 between (5120 x 5120 5.98 / 6.50, 17408 x 5120 12.2 / 12.8)
+    // 7.56 / 6.77, 12288 x 6144 9.62 / 9.03, 17408 x 2560 9.37 / 8.86). 3 passes with a part: 4 where the 1024 SIMDs need no
+    // more than half the rounds of waves that 2 rows need (4096 x 5120 5.13 / 5.00, 12288 x 5120 9.66 / 9.27, 16384 x 5120
+    // 11.5 / 11.1), else 2 (5120 x 5120 5.98 / 6.50, 10240 x 5120 4% apart, 17408 x 5120 12.2 / 12.8)
     const int64_t chunks = ceil_div64(ceil_div64(K, 8), 4), passes = ceil_div64(chunks, kWave);
     if (pl.PU > 1 && N > 2 * 1024) {
         const bool part = passes == 3 && chunks % kWave != 0;
-        const bool two = vec == kAligned && passes <= 3 && (part ? N > 4096 && N < 24576 : N < 8192);
+        const bool two = vec == kAligned && passes <= 3 && (part ? 2 * ceil_div64(N, 4096) > ceil_div64(N, 2048) : N < 8192);
         if (!two) pl.R = 4;
     }
     const bool cs = (gs % 32) == 0;

@@ -82,7 +82,7 @@ def test_int8(ops, N, K, gs):
 
 
 @pytest.mark.parametrize("K", [2560, 4096, 5120, 6144, 8192])
-@pytest.mark.parametrize("N", [2049, 4096, 4100, 8191, 8192, 8198, 24575, 24577])
+@pytest.mark.parametrize("N", [2049, 4096, 4100, 6145, 8191, 8192, 8198, 12287, 24577])
 def test_int4_rows_per_wave(ops, N, K):
     """Every line of the rows-per-wave rule (2 and 4 rows, their remainders): a row's result does not depend on its tile,
     so it is the one-row tile's of the same rows in matrices of under 2048."""
